@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/gaga_amd.h"
+#include "xcs_resident.h"
 #include "xcs_sched.h"
 #include "xcs_smvgen.h"
 #include "xcs_subset.h"
@@ -529,6 +530,7 @@ struct xcs_plan {
   XProblem h{};         // host copy (device pointers)
   XProblem *d = nullptr;
   int team = 1, block = 256, mode = 0;
+  bool resident = false;  // solve_resident_kernel instead of solve_coop_kernel
   long spin_limit = BAR_SPIN_LIMIT;  // team-barrier wait bound (sleeps)
   double *red = nullptr;
   unsigned *bar = nullptr;
@@ -603,6 +605,56 @@ static int timing_fields(XProblem &P, int alg, int k, const xcs_options *o) {
   return XCS_OK;
 }
 
+static const void *resident_kernel(int alg, int block) {
+  const bool s = block <= 512;
+  switch (alg) {
+    case ALG_NIHT:
+      return s ? (const void *)solve_resident_kernel<ALG_NIHT, 512>
+               : (const void *)solve_resident_kernel<ALG_NIHT, 1024>;
+    case ALG_HTP:
+      return s ? (const void *)solve_resident_kernel<ALG_HTP, 512>
+               : (const void *)solve_resident_kernel<ALG_HTP, 1024>;
+    case ALG_CGIHT:
+      return s ? (const void *)solve_resident_kernel<ALG_CGIHT, 512>
+               : (const void *)solve_resident_kernel<ALG_CGIHT, 1024>;
+  }
+  return nullptr;
+}
+
+// Whether the plan runs in the resident form (xcs_resident.h), and its geometry.
+static int plan_resident(xcs_plan *pl, int alg, const xcs_options *o) {
+  const XProblem &P = pl->h;
+  const int block = o->block_size > 0 ? o->block_size : 512;
+  int cus = 0, per = 0, dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const void *kernel = resident_kernel(alg, block);
+  if (!kernel) return XCS_OK;
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, block, 0));
+  int team = o->team_size;
+  if (team <= 0) {
+    // Streaming A wants many workgroups, the three exchanges per iteration few:
+    // the optimum grows with the square root of A's bytes.  Measured on MI355X,
+    // ms per solve with 512 threads (256 and 1024 are slower at every size):
+    // NIHT 256 x 1024 (1 MiB) 0.253 / 0.247 / 0.247 / 0.291 at 16 / 32 / 64 / 128
+    // workgroups (general form: 0.9); CGIHT 1024 x 4096 (16 MiB) 0.439 / 0.341 /
+    // 0.328 / 0.364 at 32 / 64 / 128 / 256; CGIHT 2048 x 8192 (64 MiB) 0.728 /
+    // 0.569 / 0.551 at 64 / 128 / 256 (general form: 1.70).  HTP spends its time
+    // in CG steps, whose products touch the support's columns only: half the team
+    // (1001 x 5003: 0.343 / 0.357 / 0.426 at 64 / 128 / 256; general form 1.65).
+    const double mib = 4.0 * P.lda * (double)P.n / (1 << 20);
+    const double want = (alg == ALG_HTP ? 16.0 : 32.0) * std::sqrt(mib);
+    team = 16;
+    while (team < 256 && team * 1.42 < want) team *= 2;
+  }
+  if (team > per * cus || team > BAR_MAX_TEAM) return XCS_OK;
+  if (!res_fits(alg, P.ens, P.n, P.lda, P.num_bins, P.timing, team)) return XCS_OK;
+  pl->resident = true;
+  pl->team = team;
+  pl->block = block;
+  return XCS_OK;
+}
+
 // Allocate workspace for (alg, ens, m, n) and fill the sizes in plan->h.
 static int plan_alloc(xcs_plan *pl, int alg, int ens, int k, int m, int n, int p, int nz,
                       const xcs_options *o) {
@@ -655,6 +707,7 @@ static int plan_alloc(xcs_plan *pl, int alg, int ens, int k, int m, int n, int p
     }
   }
   pl->team = std::min({team, maxb, BAR_MAX_TEAM});
+  XCS_TRY(plan_resident(pl, alg, o));
   // CSMPSP is switched off on the device: two of its runs (a 4-workgroup team
   // and later a single workgroup) faulted the GPU and the cause is not yet
   // found; it stays off until it is.
@@ -865,6 +918,20 @@ static int plan_generate(xcs_plan *pl, int alg, int ens, int k, int m, int n, in
   return XCS_OK;
 }
 
+static int launch_solve(xcs_plan *pl, int budget) {
+  if (pl->resident) {
+    void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->bar, (void *)&pl->spin_limit};
+    HIP_TRY(hipLaunchCooperativeKernel(resident_kernel(pl->h.alg, pl->block), dim3(pl->team),
+                                       dim3(pl->block), args, 0, pl->stream));
+    return XCS_OK;
+  }
+  void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->red, (void *)&pl->bar,
+                  (void *)&pl->spin_limit};
+  HIP_TRY(hipLaunchCooperativeKernel((const void *)solve_coop_kernel, dim3(pl->team),
+                                     dim3(pl->block), args, 0, pl->stream));
+  return XCS_OK;
+}
+
 static int plan_run(xcs_plan *pl, float *ms) {
   XProblem &P = pl->h;
   // reset: x = 0 and a fresh state (inputs stay resident)
@@ -881,10 +948,7 @@ static int plan_run(xcs_plan *pl, float *ms) {
     // (an aborted team marks the instance done, so launching stops there too)
     int budget = 1;
     for (int launch = 0; launch < P.maxiter + 4; launch++) {
-      void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->red, (void *)&pl->bar,
-                      (void *)&pl->spin_limit};
-      HIP_TRY(hipLaunchCooperativeKernel((const void *)solve_coop_kernel, dim3(pl->team),
-                                         dim3(pl->block), args, 0, pl->stream));
+      XCS_TRY(launch_solve(pl, budget));
       int done = 0;
       HIP_TRY(d2h(&done, &P.st->done, sizeof(int), pl->stream));
       HIP_TRY(hipStreamSynchronize(pl->stream));
@@ -892,10 +956,7 @@ static int plan_run(xcs_plan *pl, float *ms) {
     }
   } else {
     int budget = P.maxiter + 4;
-    void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->red, (void *)&pl->bar,
-                    (void *)&pl->spin_limit};
-    HIP_TRY(hipLaunchCooperativeKernel((const void *)solve_coop_kernel, dim3(pl->team),
-                                       dim3(pl->block), args, 0, pl->stream));
+    XCS_TRY(launch_solve(pl, budget));
   }
   HIP_TRY(hipEventRecord(e1, pl->stream));
   HIP_TRY(hipEventSynchronize(e1));
