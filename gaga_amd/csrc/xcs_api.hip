@@ -15,7 +15,7 @@
 #include <vector>
 
 #include "../../include/gaga_amd.h"
-#include "xcs_resident.h"
+#include "xcs_split.h"
 #include "xcs_sched.h"
 #include "xcs_smvgen.h"
 #include "xcs_subset.h"
@@ -530,7 +530,7 @@ struct xcs_plan {
   XProblem h{};         // host copy (device pointers)
   XProblem *d = nullptr;
   int team = 1, block = 256, mode = 0;
-  bool resident = false;  // solve_resident_kernel instead of solve_coop_kernel
+  const void *kernel = nullptr;  // solve_resident_kernel or solve_split_kernel instead of solve_coop_kernel
   long spin_limit = BAR_SPIN_LIMIT;  // team-barrier wait bound (sleeps)
   double *red = nullptr;
   unsigned *bar = nullptr;
@@ -649,7 +649,57 @@ static int plan_resident(xcs_plan *pl, int alg, const xcs_options *o) {
   }
   if (team > per * cus || team > BAR_MAX_TEAM) return XCS_OK;
   if (!res_fits(alg, P.ens, P.n, P.lda, P.num_bins, P.timing, team)) return XCS_OK;
-  pl->resident = true;
+  pl->kernel = kernel;
+  pl->team = team;
+  pl->block = block;
+  return XCS_OK;
+}
+
+static const void *split_kernel(int ens, int alg) {
+  switch (alg) {
+    case ALG_NIHT:
+      return ens == ENS_DCT ? (const void *)solve_split_kernel<ENS_DCT, ALG_NIHT>
+                            : (const void *)solve_split_kernel<ENS_SMV, ALG_NIHT>;
+    case ALG_HTP:
+      return ens == ENS_DCT ? (const void *)solve_split_kernel<ENS_DCT, ALG_HTP>
+                            : (const void *)solve_split_kernel<ENS_SMV, ALG_HTP>;
+    case ALG_CGIHT:
+      return ens == ENS_DCT ? (const void *)solve_split_kernel<ENS_DCT, ALG_CGIHT>
+                            : (const void *)solve_split_kernel<ENS_SMV, ALG_CGIHT>;
+  }
+  return nullptr;
+}
+
+// Whether the plan runs in the split form (xcs_split.h), and its geometry.
+static int plan_split(xcs_plan *pl, int alg, const xcs_options *o) {
+  const XProblem &P = pl->h;
+  if (P.ens != ENS_SMV && P.ens != ENS_DCT) return XCS_OK;
+  const void *kernel = split_kernel(P.ens, alg);
+  const int block = o->block_size > 0 ? o->block_size : SP_THREADS;
+  if (!kernel || block > SP_THREADS) return XCS_OK;
+  int cus = 0, per = 0, dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, block, 0));
+  int team = o->team_size;
+  if (team <= 0) {
+    // As for the dense form the optimum grows with the square root of the size:
+    // half of sqrt(n), in powers of two.  Measured on MI355X, ms per solve:
+    // NIHT smv 1000 x 4001 0.294 / 0.259 / 0.279 at 8 / 16 / 32 workgroups; NIHT smv
+    // 4999 x 20001 0.546 / 0.495 / 0.543 at 32 / 64 / 128 (general form 1.64); CGIHT
+    // smv 2^15 x 2^18 4.48 / 3.03 / 2.58 at 64 / 128 / 256 (6.6); NIHT dct n = 2^17
+    // 0.785 / 0.619 / 0.552 at 32 / 64 / 128; CGIHT dct n = 2^14 0.366 / 0.302 / 0.307
+    // at 8 / 16 / 32; NIHT dct n = 2^20 1.66 at 256 (5.7; fewer do not fit its LDS).
+    team = 2;
+    while (team < 256 && 4.0 * team <= std::sqrt((double)P.n)) team *= 2;
+    if (P.ens == ENS_DCT) {  // the factorisation allows up to half its rows
+      const int n1 = P.log2n > 1 ? 1 << ((P.log2n - 1) / 2) : 1;
+      team = std::min(team, n1 / 2);
+    }
+  }
+  if (team > per * cus || team > BAR_MAX_TEAM) return XCS_OK;
+  if (!split_fits(alg, P.ens, P.m, P.n, P.log2n, P.num_bins, P.timing, team, block)) return XCS_OK;
+  pl->kernel = kernel;
   pl->team = team;
   pl->block = block;
   return XCS_OK;
@@ -708,6 +758,7 @@ static int plan_alloc(xcs_plan *pl, int alg, int ens, int k, int m, int n, int p
   }
   pl->team = std::min({team, maxb, BAR_MAX_TEAM});
   XCS_TRY(plan_resident(pl, alg, o));
+  if (!pl->kernel) XCS_TRY(plan_split(pl, alg, o));
   // CSMPSP is switched off on the device: two of its runs (a 4-workgroup team
   // and later a single workgroup) faulted the GPU and the cause is not yet
   // found; it stays off until it is.
@@ -919,10 +970,9 @@ static int plan_generate(xcs_plan *pl, int alg, int ens, int k, int m, int n, in
 }
 
 static int launch_solve(xcs_plan *pl, int budget) {
-  if (pl->resident) {
+  if (pl->kernel) {
     void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->bar, (void *)&pl->spin_limit};
-    HIP_TRY(hipLaunchCooperativeKernel(resident_kernel(pl->h.alg, pl->block), dim3(pl->team),
-                                       dim3(pl->block), args, 0, pl->stream));
+    HIP_TRY(hipLaunchCooperativeKernel(pl->kernel, dim3(pl->team), dim3(pl->block), args, 0, pl->stream));
     return XCS_OK;
   }
   void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->red, (void *)&pl->bar,

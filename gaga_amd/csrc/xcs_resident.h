@@ -86,6 +86,16 @@ __device__ __forceinline__ double wsum_d(double v) {
   v += dpp_d<DPP_BCAST31, 0xc>(v);
   return lane_d(v, 63);
 }
+// Maximum of non-negative values (0 is the identity).
+__device__ __forceinline__ double wmax_d(double v) {
+  v = fmax(v, dpp_d<DPP_SHR1, 0xf>(v));
+  v = fmax(v, dpp_d<DPP_SHR2, 0xf>(v));
+  v = fmax(v, dpp_d<DPP_SHR4, 0xf>(v));
+  v = fmax(v, dpp_d<DPP_SHR8, 0xf>(v));
+  v = fmax(v, dpp_d<DPP_BCAST15, 0xa>(v));
+  v = fmax(v, dpp_d<DPP_BCAST31, 0xc>(v));
+  return lane_d(v, 63);
+}
 __device__ __forceinline__ float wsum_f(float v) {
   v += dpp_f<DPP_SHR1, 0xf>(v);
   v += dpp_f<DPP_SHR2, 0xf>(v);
@@ -95,7 +105,6 @@ __device__ __forceinline__ float wsum_f(float v) {
   v += dpp_f<DPP_BCAST31, 0xc>(v);
   return lane_f(v, 63);
 }
-// Maximum of non-negative values (0 is the identity).
 __device__ __forceinline__ float wmax_f(float v) {
   v = fmaxf(v, dpp_f<DPP_SHR1, 0xf>(v));
   v = fmaxf(v, dpp_f<DPP_SHR2, 0xf>(v));
@@ -191,7 +200,8 @@ struct RtSlots {
   int bad;
 };
 
-// Barrier over the team that sums K doubles (one partial per thread): one hop.
+// Barrier over the team that sums K doubles (one partial per thread; double k is
+// maximised instead where bit k of MAXES is set, non-negative values): one hop.
 // Every wave first waits for its own device-scope stores (vmcnt), so what the
 // workgroup published before the call has arrived when its words do.  Each
 // workgroup posts its partials as 64-bit words of tag and half a double (one
@@ -203,7 +213,7 @@ struct RtSlots {
 // at 64 / 128 / 256 workgroups, against 2.8 / 3.8 / 5.7 for the two-hop flag
 // barrier with its fences (4.5-6 us in a solve).  Waits are bounded as in
 // team_barrier.
-template <int K>
+template <int K, int MAXES = 0>
 __device__ __forceinline__ void rt_allreduce(RTeam &t, RtSlots &X, const double (&v)[K ? K : 1],
                                              double (&out)[K ? K : 1]) {
   constexpr int KK = K ? K : 1, W = K ? 2 * K : 1;
@@ -215,7 +225,7 @@ __device__ __forceinline__ void rt_allreduce(RTeam &t, RtSlots &X, const double 
   if (K) {
 #pragma unroll
     for (int k = 0; k < K; k++) {
-      const double s = wsum_d(v[k]);
+      const double s = (MAXES >> k & 1) ? wmax_d(v[k]) : wsum_d(v[k]);
       if (lane == 0) X.part[k][wave] = s;
     }
   }
@@ -230,7 +240,8 @@ __device__ __forceinline__ void rt_allreduce(RTeam &t, RtSlots &X, const double 
     if (K) {
 #pragma unroll
       for (int k = 0; k < K; k++) {
-        const double s = wsum_d(lane < nw ? X.part[k][lane] : 0.0);
+        const double part = lane < nw ? X.part[k][lane] : 0.0;
+        const double s = (MAXES >> k & 1) ? wmax_d(part) : wsum_d(part);
         const unsigned long long b = (unsigned long long)__double_as_longlong(s);
         if ((lane >> 1) == k) mine = T | ((lane & 1) ? (b >> 32) : (b & 0xFFFFFFFFull));
       }
@@ -266,15 +277,17 @@ __device__ __forceinline__ void rt_allreduce(RTeam &t, RtSlots &X, const double 
       }
       if (K && !bad && r < t.size) {
 #pragma unroll
-        for (int k = 0; k < K; k++)
-          acc[k] += __longlong_as_double(
+        for (int k = 0; k < K; k++) {
+          const double b = __longlong_as_double(
               (long long)((w[(2 * k + 1) % W] << 32) | (w[(2 * k) % W] & 0xFFFFFFFFull)));
+          acc[k] = (MAXES >> k & 1) ? fmax(acc[k], b) : acc[k] + b;
+        }
       }
     }
     if (K) {
 #pragma unroll
       for (int k = 0; k < K; k++) {
-        const double s = wsum_d(acc[k]);
+        const double s = (MAXES >> k & 1) ? wmax_d(acc[k]) : wsum_d(acc[k]);
         if (lane == 0) X.out[k] = s;
       }
     }
