@@ -100,106 +100,179 @@ __device__ void mlp_features(const float *g, int n, int m, int k, float *X) {
   __syncthreads();
 }
 
+// Rows of the batch one workgroup of the row-blocked kernels takes, and the
+// partial column sums it leaves (summed over the row blocks in a fixed order by
+// mlp_final_kernel): dW1 and db1, dW3 and db2, db3.
+constexpr int MLP_R = 32;
+constexpr int MLP_PW1 = 0, MLP_PB1 = MLP_H * MLP_F, MLP_PW3 = MLP_PB1 + MLP_H,
+              MLP_PB2 = MLP_PW3 + MLP_H, MLP_PB3 = MLP_PB2 + MLP_H, MLP_PN = MLP_PB3 + 64;
+
 // ------------------------------------------------------------- forward -----
-// h1[c][u] = bf16(relu(sum_f X[c][f] W1[u][f] + b1[u])), one thread per (c, u).
-__global__ void mlp_l1_kernel(const float *X, int B, const float *p, uint16_t *h1b) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long)B * MLP_H) return;
-  const int c = (int)(e / MLP_H), u = (int)(e % MLP_H);
-  const float *x = X + (long)c * MLP_F, *w = p + MLP_OW1 + (long)u * MLP_F;
-  float z = p[MLP_OB1 + u];
+// h1[c][u] = bf16(relu(sum_f X[c][f] W1[u][f] + b1[u])).  One workgroup per
+// MLP_R rows, two neighbouring units per thread with their weights in registers
+// (one thread per entry re-read 16 values for each).
+__global__ void __launch_bounds__(256) mlp_l1_kernel(const float *X, int B, const float *p,
+                                                     uint16_t *h1b) {
+  __shared__ float xs[MLP_R][MLP_F];
+  const int c0 = blockIdx.x * MLP_R, rows = min(MLP_R, B - c0), u = 2 * threadIdx.x;
+  for (int e = threadIdx.x; e < rows * MLP_F; e += 256) (&xs[0][0])[e] = X[(long)c0 * MLP_F + e];
+  float w[2][MLP_F], b[2];
 #pragma unroll
-  for (int f = 0; f < MLP_F; f++) z = fmaf(x[f], w[f], z);
-  h1b[e] = f2bf16_rne(fmaxf(z, 0.f));
+  for (int q = 0; q < 2; q++) {
+    b[q] = p[MLP_OB1 + u + q];
+#pragma unroll
+    for (int f = 0; f < MLP_F; f++) w[q][f] = p[MLP_OW1 + (long)(u + q) * MLP_F + f];
+  }
+  __syncthreads();
+  uint32_t *out = (uint32_t *)(h1b + (long)c0 * MLP_H) + threadIdx.x;
+  for (int r = 0; r < rows; r++) {
+    float z0 = b[0], z1 = b[1];
+#pragma unroll
+    for (int f = 0; f < MLP_F; f++) {
+      z0 = fmaf(xs[r][f], w[0][f], z0);
+      z1 = fmaf(xs[r][f], w[1][f], z1);
+    }
+    out[r * (MLP_H / 2)] =
+        (uint32_t)f2bf16_rne(fmaxf(z0, 0.f)) | ((uint32_t)f2bf16_rne(fmaxf(z1, 0.f)) << 16);
+  }
 }
 
-// Logit of each coordinate (one wave per coordinate) from z2 = W2 h1 (GEMM):
-// a2 = relu(z2 + b2), logit = W3 . a2 + b3.  With labels (training): the
-// weighted BCE loss, dlogit = w (sigmoid - y) / B, dz2 = dlogit W3 [a2 > 0]
-// (FP32 and BF16 copies) and a2 kept for the weight gradients.
-__global__ void __launch_bounds__(256) mlp_l3_kernel(const float *z2, int B, const float *p,
-                                                     const float *labels, float pos_w,
-                                                     float *logit, float *loss, float *a2,
-                                                     float *dlogit, float *dz2,
-                                                     uint16_t *dz2b) {
+// Logit of one coordinate by one wave from its z2 row (z2 = W2 h1, GEMM):
+// a2 = relu(z2 + b2), logit = W3 . a2 + b3.
+__device__ __forceinline__ float mlp_logit(const float *z, const float *p) {
   const int lane = threadIdx.x & 63;
+  float acc = 0.f;
+#pragma unroll
+  for (int q = 0; q < MLP_H / 64; q++) {
+    const int u = lane + 64 * q;
+    acc = fmaf(fmaxf(z[u] + p[MLP_OB2 + u], 0.f), p[MLP_OW3 + u], acc);
+  }
+  return wave_sum(acc) + p[MLP_OB3];
+}
+__global__ void __launch_bounds__(256) mlp_l3_kernel(const float *z2, int B, const float *p,
+                                                     float *logit) {
   const long c = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   if (c >= B) return;
-  const float *z = z2 + c * MLP_H;
-  float acc = 0.f;
-  float av[MLP_H / 64];
-#pragma unroll
-  for (int q = 0; q < MLP_H / 64; q++) {
-    const int u = lane + 64 * q;
-    av[q] = fmaxf(z[u] + p[MLP_OB2 + u], 0.f);
-    acc = fmaf(av[q], p[MLP_OW3 + u], acc);
+  const float lg = mlp_logit(z2 + c * MLP_H, p);
+  if ((threadIdx.x & 63) == 0) logit[c] = lg;
+}
+
+// The output layer of a training pass on MLP_R coordinates per workgroup: each
+// wave's logits, weighted BCE losses and dlogit = w (sigmoid - y) / B, then two
+// neighbouring columns per thread over the rows (still in cache): dz2 = dlogit
+// W3 [a2 > 0] (FP32 and BF16) and the row block's sums of dW3, db2 and db3.  The
+// sums used to be passes of their own over a2 and dz2 with 64 workgroups each
+// (51 us apiece at B = 8192); here they ride on the pass that forms dz2.
+__global__ void __launch_bounds__(256) mlp_out_kernel(const float *z2, int B, const float *p,
+                                                      const float *labels, float pos_w,
+                                                      float *logit, float *loss, float *dz2,
+                                                      uint16_t *dz2b, float *part) {
+  __shared__ float dl[MLP_R];
+  const int c0 = blockIdx.x * MLP_R, rows = min(MLP_R, B - c0);
+  const int lane = threadIdx.x & 63;
+  for (int r = threadIdx.x >> 6; r < rows; r += 4) {
+    const long c = c0 + r;
+    const float lg = mlp_logit(z2 + c * MLP_H, p);
+    if (lane == 0) {
+      const float y = labels[c];
+      const float w = y > 0.5f ? pos_w : 1.0f;
+      const float sig = 1.0f / (1.0f + expf(-lg));
+      logit[c] = lg;
+      loss[c] = w * (fmaxf(lg, 0.f) - lg * y + log1pf(expf(-fabsf(lg))));
+      dl[r] = w * (sig - y) / (float)B;
+    }
   }
-  acc = wave_sum(acc);
-  const float lg = acc + p[MLP_OB3];
-  if (lane == 0) logit[c] = lg;
-  if (!labels) return;
-  const float y = labels[c];
-  const float w = y > 0.5f ? pos_w : 1.0f;
-  const float sig = 1.0f / (1.0f + expf(-lg));
-  const float dl = w * (sig - y) / (float)B;
-  if (lane == 0) {
-    loss[c] = w * (fmaxf(lg, 0.f) - lg * y + log1pf(expf(-fabsf(lg))));
-    dlogit[c] = dl;
+  __syncthreads();
+  const int u = 2 * threadIdx.x;
+  const float2 b2 = make_float2(p[MLP_OB2 + u], p[MLP_OB2 + u + 1]);
+  const float2 w3 = make_float2(p[MLP_OW3 + u], p[MLP_OW3 + u + 1]);
+  float gw0 = 0.f, gw1 = 0.f, gb0 = 0.f, gb1 = 0.f, gl = 0.f;
+#pragma unroll 4
+  for (int r = 0; r < rows; r++) {
+    const long o = (long)(c0 + r) * MLP_H + u;
+    const float2 z = *(const float2 *)(z2 + o);
+    const float d = dl[r];
+    const float a0 = fmaxf(z.x + b2.x, 0.f), a1 = fmaxf(z.y + b2.y, 0.f);
+    const float d0 = a0 > 0.f ? d * w3.x : 0.f, d1 = a1 > 0.f ? d * w3.y : 0.f;
+    *(float2 *)(dz2 + o) = make_float2(d0, d1);
+    *(uint32_t *)(dz2b + o) = (uint32_t)f2bf16_rne(d0) | ((uint32_t)f2bf16_rne(d1) << 16);
+    gw0 = fmaf(a0, d, gw0);
+    gw1 = fmaf(a1, d, gw1);
+    gb0 += d0;
+    gb1 += d1;
+    gl += d;
   }
-#pragma unroll
-  for (int q = 0; q < MLP_H / 64; q++) {
-    const int u = lane + 64 * q;
-    a2[c * MLP_H + u] = av[q];
-    const float d = av[q] > 0.f ? dl * p[MLP_OW3 + u] : 0.f;
-    dz2[c * MLP_H + u] = d;
-    dz2b[c * MLP_H + u] = f2bf16_rne(d);
-  }
+  float *o = part + (long)blockIdx.x * MLP_PN;
+  *(float2 *)(o + MLP_PW3 + u) = make_float2(gw0, gw1);
+  *(float2 *)(o + MLP_PB2 + u) = make_float2(gb0, gb1);
+  if (threadIdx.x == 0) o[MLP_PB3] = gl;
 }
 
 // ------------------------------------------------------------ backward -----
-// Column sums over the batch in fixed order: out[u] = sum_c a[c*ld + u] * (w ? w[c] : 1),
-// for u < cols.  Stage 1: partials per (chunk of rows); stage 2 sums chunks in order.
-constexpr int MLP_RCHUNK = 256;
-__global__ void mlp_colsum_partial(const float *a, int B, int cols, long ld, const float *w,
-                                   float *part) {
-  const int u = blockIdx.x * blockDim.x + threadIdx.x, ch = blockIdx.y;
-  if (u >= cols) return;
-  const int c0 = ch * MLP_RCHUNK, c1 = min(B, c0 + MLP_RCHUNK);
-  float s = 0.f;
-  for (int c = c0; c < c1; c++) s = fmaf(a[(long)c * ld + u], w ? w[c] : 1.0f, s);
-  part[(long)ch * cols + u] = s;
-}
-__global__ void mlp_colsum_final(const float *part, int nch, int cols, float *out) {
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= cols) return;
-  float s = 0.f;
-  for (int ch = 0; ch < nch; ch++) s += part[(long)ch * cols + u];
-  out[u] = s;
-}
-
-// dz1 = dh1 [h1 > 0]; in place on dh1.
-__global__ void mlp_relu_back_kernel(float *dh1, const uint16_t *h1b, long cnt) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < cnt && !(bf16_to_f(h1b[e]) > 0.f)) dh1[e] = 0.f;
-}
-
-// dW1[u][f] = sum_c dz1[c][u] X[c][f] (one thread per (u, f), fixed order).
-__global__ void mlp_dw1_partial(const float *dz1, const float *X, int B, float *part) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x, ch = blockIdx.y;
-  if (e >= MLP_H * MLP_F) return;
-  const int u = e / MLP_F, f = e % MLP_F;
-  const int c0 = ch * MLP_RCHUNK, c1 = min(B, c0 + MLP_RCHUNK);
-  float s = 0.f;
-  for (int c = c0; c < c1; c++) s = fmaf(dz1[(long)c * MLP_H + u], X[(long)c * MLP_F + f], s);
-  part[(long)ch * MLP_H * MLP_F + e] = s;
+// dz1 = dh1 [h1 > 0] and the row block's sums of db1 and dW1[u][f] = sum_c
+// dz1[c][u] X[c][f], two units per thread, in one pass over dh1 (three passes of
+// 9, 51 and 64 us before, one of them reading dz1 once per feature).
+__global__ void __launch_bounds__(256) mlp_in_kernel(const float *dh1, const uint16_t *h1b,
+                                                     const float *X, int B, float *part) {
+  __shared__ float xs[MLP_R][MLP_F];
+  const int c0 = blockIdx.x * MLP_R, rows = min(MLP_R, B - c0), u = 2 * threadIdx.x;
+  for (int e = threadIdx.x; e < rows * MLP_F; e += 256) (&xs[0][0])[e] = X[(long)c0 * MLP_F + e];
+  __syncthreads();
+  float g[2][MLP_F] = {}, gb[2] = {};
+#pragma unroll 4
+  for (int r = 0; r < rows; r++) {
+    const long o = (long)(c0 + r) * MLP_H + u;
+    const float2 d = *(const float2 *)(dh1 + o);
+    const uint32_t h = *(const uint32_t *)(h1b + o);
+    const float d0 = bf16_to_f((uint16_t)h) > 0.f ? d.x : 0.f;
+    const float d1 = bf16_to_f((uint16_t)(h >> 16)) > 0.f ? d.y : 0.f;
+    gb[0] += d0;
+    gb[1] += d1;
+#pragma unroll
+    for (int f = 0; f < MLP_F; f++) {
+      g[0][f] = fmaf(d0, xs[r][f], g[0][f]);
+      g[1][f] = fmaf(d1, xs[r][f], g[1][f]);
+    }
+  }
+  float *o = part + (long)blockIdx.x * MLP_PN;
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+#pragma unroll
+    for (int f = 0; f < MLP_F; f++) o[MLP_PW1 + (u + q) * MLP_F + f] = g[q][f];
+    o[MLP_PB1 + u + q] = gb[q];
+  }
 }
 
-// FP32 tiled GEMM, C[i][j] = sum_k A(i, k) B(j, k) with strided operands
-// (B may be BF16), 64 x 64 tile per 256-thread block, 4 x 4 per thread, K in
-// steps of 16 through LDS; blockIdx.z = K split (slice z of C at z * c_split).
-template <bool BB16>
+// The row blocks' partial sums, 64 columns per workgroup: each of 16 thread rows
+// sums a contiguous run of blocks, then the runs in order.
+__global__ void __launch_bounds__(1024) mlp_final_kernel(const float *part, int nch, float *g) {
+  __shared__ float s[16][64];
+  const int e = blockIdx.x * 64 + (threadIdx.x & 63), run = threadIdx.x >> 6;
+  const int per = (nch + 15) / 16, a = min(nch, run * per), b = min(nch, a + per);
+  float t = 0.f;
+  if (e <= MLP_PB3) {
+#pragma unroll 8
+    for (int ch = a; ch < b; ch++) t += part[(long)ch * MLP_PN + e];
+  }
+  s[run][threadIdx.x & 63] = t;
+  __syncthreads();
+  if (run == 0 && e <= MLP_PB3) {
+    float v = 0.f;
+    for (int q = 0; q < 16; q++) v += s[q][threadIdx.x];
+    const long at = e < MLP_PB1   ? MLP_OW1 + e
+                    : e < MLP_PW3 ? MLP_OB1 + (e - MLP_PB1)
+                    : e < MLP_PB2 ? MLP_OW3 + (e - MLP_PW3)
+                    : e < MLP_PB3 ? MLP_OB2 + (e - MLP_PB2)
+                                  : MLP_OB3;
+    g[at] = v;
+  }
+}
+
+// FP32 tiled GEMM, C[i][j] = sum_k A(i, k) B(j, k) with strided operands,
+// 64 x 64 tile per 256-thread block, 4 x 4 per thread, K in steps of 16
+// through LDS; blockIdx.z = K split (slice z of C at z * c_split).
 __global__ void __launch_bounds__(256) f32_gemm_kernel(int M, int N, int K, const float *A,
-                                                       long sai, long sak, const void *Bv,
+                                                       long sai, long sak, const float *Bm,
                                                        long sbj, long sbk, float *C, long sci,
                                                        long scj, int ksplit, long c_split) {
   __shared__ float As[16][64 + 4], Bs[16][64 + 4];
@@ -218,12 +291,7 @@ __global__ void __launch_bounds__(256) f32_gemm_kernel(int M, int N, int K, cons
     for (int e = threadIdx.x; e < 16 * 64; e += 256) {
       const int kk = b_kc ? (e & 15) : (e >> 6), r = b_kc ? (e >> 4) : (e & 63);
       const int k = k0 + kk, j = j0 + r;
-      float bv = 0.f;
-      if (k < kb && j < N) {
-        const long off = (long)j * sbj + (long)k * sbk;
-        bv = BB16 ? bf16_to_f(((const uint16_t *)Bv)[off]) : ((const float *)Bv)[off];
-      }
-      Bs[kk][r] = bv;
+      Bs[kk][r] = (k < kb && j < N) ? Bm[(long)j * sbj + (long)k * sbk] : 0.f;
     }
     __syncthreads();
 #pragma unroll
@@ -251,11 +319,101 @@ __global__ void __launch_bounds__(256) f32_gemm_kernel(int M, int N, int K, cons
     }
 }
 
+// dW2[o][i] = sum_c dz2[c][o] h1[c][i] in FP32 on the matrix cores
+// (v_mfma_f32_32x32x2_f32: FP32 products and sums): both operands have the batch
+// as their outer index, which is the layout the instruction takes (lane l: entry
+// l % 32 of batch row l / 32), so the tiles go from memory to LDS as they lie.
+// 128 x 128 tile, 4 waves of 64 x 64, 16 batch rows per stage (the next stage's
+// loads in flight during the products), blockIdx.z = slice of the batch (kc
+// rows, a multiple of 16; rows past B count as zero).  The bound is the FP32
+// matrix rate (157 TFLOP/s: 27 us at B = 8192); the VALU form took 130 us.
+typedef float f32x16m_t __attribute__((ext_vector_type(16)));
+__global__ void __launch_bounds__(256) mlp_dw2_kernel(const float *dz2, const uint16_t *h1b, int B,
+                                                      int kc, float *C) {
+  constexpr int KS = 16;
+  __shared__ __attribute__((aligned(16))) float As[2][KS][128], Bs[2][KS][128];
+  const int o0 = blockIdx.x * 128, i0 = blockIdx.y * 128;
+  const int ka = blockIdx.z * kc, kb = min(B, ka + kc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64, r32 = lane & 31, h = lane >> 5;
+  // a thread's part of a stage: 8 consecutive columns of one batch row
+  const int lk = threadIdx.x >> 4, lc = (threadIdx.x & 15) * 8;
+  float4 ra[2];
+  uint4 rb;
+  auto load = [&](int k0) {
+    const int c = k0 + lk;
+    ra[0] = ra[1] = make_float4(0.f, 0.f, 0.f, 0.f);
+    rb = make_uint4(0u, 0u, 0u, 0u);
+    if (c < kb) {
+      const float4 *a = (const float4 *)(dz2 + (long)c * MLP_H + o0 + lc);
+      ra[0] = a[0];
+      ra[1] = a[1];
+      rb = *(const uint4 *)(h1b + (long)c * MLP_H + i0 + lc);
+    }
+  };
+  auto store = [&](int buf) {
+    *(float4 *)&As[buf][lk][lc] = ra[0];
+    *(float4 *)&As[buf][lk][lc + 4] = ra[1];
+    const uint32_t w[4] = {rb.x, rb.y, rb.z, rb.w};
+    float f[8];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      f[2 * q] = bf16_to_f((uint16_t)w[q]);
+      f[2 * q + 1] = bf16_to_f((uint16_t)(w[q] >> 16));
+    }
+    *(float4 *)&Bs[buf][lk][lc] = make_float4(f[0], f[1], f[2], f[3]);
+    *(float4 *)&Bs[buf][lk][lc + 4] = make_float4(f[4], f[5], f[6], f[7]);
+  };
+  f32x16m_t acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
+  if (ka < kb) {  // uniform
+    load(ka);
+    store(0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = ka; k0 < kb; k0 += KS, buf ^= 1) {
+      if (k0 + KS < kb) load(k0 + KS);
+#pragma unroll
+      for (int k = 0; k < KS; k += 2) {
+        float fa[2], fb[2];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+          fa[q] = As[buf][k + h][wm + 32 * q + r32];
+          fb[q] = Bs[buf][k + h][wn + 32 * q + r32];
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int b = 0; b < 2; b++)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a], fb[b], acc[a][b], 0, 0, 0);
+      }
+      if (k0 + KS < kb) store(buf ^ 1);
+      __syncthreads();
+    }
+  }
+  float *Cz = C + (long)blockIdx.z * MLP_H * MLP_H;
+#pragma unroll
+  for (int a = 0; a < 2; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const int o = o0 + wm + 32 * a + 8 * (v / 4) + 4 * h + v % 4;
+        Cz[(long)o * MLP_H + i0 + wn + 32 * b + r32] = acc[a][b][v];
+      }
+}
+
 // Sum of K-split slices in order: out[e] = sum_z part[z * stride + e].
 __global__ void mlp_split_sum(const float *part, int nz, long stride, long cnt, float *out) {
   for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < cnt;
        e += (long)gridDim.x * blockDim.x) {
     float s = 0.f;
+#pragma unroll 8
     for (int z = 0; z < nz; z++) s += part[z * stride + e];
     out[e] = s;
   }
@@ -399,8 +557,8 @@ struct xcs_mlp {
   long step = 0;
   // batch buffers (capacity cap coordinates)
   long cap = 0;
-  float *X = nullptr, *lab = nullptr, *z2 = nullptr, *a2 = nullptr, *dz2 = nullptr, *dh1 = nullptr;
-  float *logit = nullptr, *loss = nullptr, *dlogit = nullptr, *part = nullptr, *gpart = nullptr;
+  float *X = nullptr, *lab = nullptr, *z2 = nullptr, *dz2 = nullptr, *dh1 = nullptr;
+  float *logit = nullptr, *loss = nullptr, *part = nullptr, *gpart = nullptr;
   uint16_t *h1b = nullptr, *dz2b = nullptr;
   std::vector<void *> batch_allocs;
   // training set
@@ -442,27 +600,28 @@ static int mlp_reserve(xcs_mlp *net, long B) {
   XCS_TRY(net->alloc_in(L, &net->lab, (size_t)B));
   XCS_TRY(net->alloc_in(L, &net->h1b, (size_t)B * H));
   XCS_TRY(net->alloc_in(L, &net->z2, (size_t)B * H));
-  XCS_TRY(net->alloc_in(L, &net->a2, (size_t)B * H));
   XCS_TRY(net->alloc_in(L, &net->dz2, (size_t)B * H));
   XCS_TRY(net->alloc_in(L, &net->dz2b, (size_t)B * H));
   XCS_TRY(net->alloc_in(L, &net->dh1, (size_t)B * H));
   XCS_TRY(net->alloc_in(L, &net->logit, (size_t)B));
   XCS_TRY(net->alloc_in(L, &net->loss, (size_t)B));
-  XCS_TRY(net->alloc_in(L, &net->dlogit, (size_t)B));
-  const long nch = (B + MLP_RCHUNK - 1) / MLP_RCHUNK;
-  XCS_TRY(net->alloc_in(L, &net->part, (size_t)nch * H * MLP_F + (size_t)nch * H + 64));
+  const long nch = (B + MLP_R - 1) / MLP_R;
+  XCS_TRY(net->alloc_in(L, &net->part, (size_t)nch * MLP_PN));
   XCS_TRY(net->alloc_in(L, &net->gpart, (size_t)MLP_KSPLIT * H * H));
   net->cap = B;
   return XCS_OK;
 }
 
 // Forward over B coordinates in net->X; logits in net->logit.  With labels
-// in net->lab: backward into net->g (and per-coordinate losses).
+// in net->lab: backward into net->g (and per-coordinate losses).  Eight launches
+// for a training pass (nineteen before); measured on MI355X at B = 8192: l1 8.5,
+// the GEMMs 14 each, out 22, dW2 50 (its FP32 matrix-rate floor is 27), in 10, the
+// sums 9 us; an Adam step of 8192 504 -> 126 us, of 100 171 -> 77 us.
 static int mlp_pass(xcs_mlp *net, int B, bool train, float pos_w) {
   const long H = MLP_H;
   hipStream_t st = net->stream;
-  hipLaunchKernelGGL(mlp_l1_kernel, dim3((unsigned)((B * H + 255) / 256)), dim3(256), 0, st, net->X,
-                     B, net->p, net->h1b);
+  const int nch = (B + MLP_R - 1) / MLP_R;
+  hipLaunchKernelGGL(mlp_l1_kernel, dim3(nch), dim3(256), 0, st, net->X, B, net->p, net->h1b);
   GemmArgs ga{};
   ga.A = (const uint8_t *)net->w2b;
   ga.lda_bytes = 2 * H;
@@ -476,32 +635,22 @@ static int mlp_pass(xcs_mlp *net, int B, bool train, float pos_w) {
   ga.ksplit = 1;
   hipLaunchKernelGGL((gemm_tn_kernel<FMT_BF16, 2, 2>), dim3(H / GT_M, (B + GT_N - 1) / GT_N, 1),
                      dim3(GT_THREADS), 0, st, ga);
-  hipLaunchKernelGGL(mlp_l3_kernel, dim3((unsigned)((B * 64L + 255) / 256)), dim3(256), 0, st,
-                     net->z2, B, net->p, train ? net->lab : nullptr, pos_w, net->logit, net->loss,
-                     net->a2, net->dlogit, net->dz2, net->dz2b);
+  if (!train) {
+    hipLaunchKernelGGL(mlp_l3_kernel, dim3((unsigned)((B * 64L + 255) / 256)), dim3(256), 0, st,
+                       net->z2, B, net->p, net->logit);
+    HIP_TRY(hipGetLastError());
+    return XCS_OK;
+  }
+  hipLaunchKernelGGL(mlp_out_kernel, dim3(nch), dim3(256), 0, st, net->z2, B, net->p, net->lab,
+                     pos_w, net->logit, net->loss, net->dz2, net->dz2b, net->part);
   HIP_TRY(hipGetLastError());
-  if (!train) return XCS_OK;
-  const int nch = (B + MLP_RCHUNK - 1) / MLP_RCHUNK;
-  float *gp = net->g;
-  // dW3 = sum_c dlogit_c a2[c], db3 = sum_c dlogit_c, db2 = sum_c dz2[c]
-  hipLaunchKernelGGL(mlp_colsum_partial, dim3(H / 256, nch), dim3(256), 0, st, net->a2, B, (int)H,
-                     H, net->dlogit, net->part);
-  hipLaunchKernelGGL(mlp_colsum_final, dim3(H / 256), dim3(256), 0, st, net->part, nch, (int)H,
-                     gp + MLP_OW3);
-  hipLaunchKernelGGL(mlp_colsum_partial, dim3(1, nch), dim3(64), 0, st, net->dlogit, B, 1, 1L,
-                     (const float *)nullptr, net->part);
-  hipLaunchKernelGGL(mlp_colsum_final, dim3(1), dim3(64), 0, st, net->part, nch, 1, gp + MLP_OB3);
-  hipLaunchKernelGGL(mlp_colsum_partial, dim3(H / 256, nch), dim3(256), 0, st, net->dz2, B, (int)H,
-                     H, (const float *)nullptr, net->part);
-  hipLaunchKernelGGL(mlp_colsum_final, dim3(H / 256), dim3(256), 0, st, net->part, nch, (int)H,
-                     gp + MLP_OB2);
-  // dW2[o][i] = sum_c dz2[c][o] h1[c][i] (FP32, K split over the batch)
-  hipLaunchKernelGGL(f32_gemm_kernel<true>, dim3(H / 64, H / 64, MLP_KSPLIT), dim3(256), 0, st,
-                     (int)H, (int)H, B, net->dz2, 1L, H, (const void *)net->h1b, 1L, H, net->gpart,
-                     H, 1L, MLP_KSPLIT, H * H);
+  // dW2[o][i] = sum_c dz2[c][o] h1[c][i], the batch split over the grid
+  const int kc = ((B + MLP_KSPLIT - 1) / MLP_KSPLIT + 15) / 16 * 16;
+  hipLaunchKernelGGL(mlp_dw2_kernel, dim3(H / 128, H / 128, MLP_KSPLIT), dim3(256), 0, st,
+                     net->dz2, net->h1b, B, kc, net->gpart);
   hipLaunchKernelGGL(mlp_split_sum, dim3(1024), dim3(256), 0, st, net->gpart, MLP_KSPLIT, H * H,
-                     H * H, gp + MLP_OW2);
-  // dh1 = dz2 W2 (MFMA: A = W2^T, B = dz2 in BF16), then dz1 = dh1 [h1 > 0]
+                     H * H, net->g + MLP_OW2);
+  // dh1 = dz2 W2 (MFMA: A = W2^T, B = dz2 in BF16)
   GemmArgs gb{};
   gb.A = (const uint8_t *)net->w2tb;
   gb.lda_bytes = 2 * H;
@@ -515,17 +664,11 @@ static int mlp_pass(xcs_mlp *net, int B, bool train, float pos_w) {
   gb.ksplit = 1;
   hipLaunchKernelGGL((gemm_tn_kernel<FMT_BF16, 2, 2>), dim3(H / GT_M, (B + GT_N - 1) / GT_N, 1),
                      dim3(GT_THREADS), 0, st, gb);
-  hipLaunchKernelGGL(mlp_relu_back_kernel, dim3((unsigned)((B * H + 255) / 256)), dim3(256), 0, st,
-                     net->dh1, net->h1b, (long)B * H);
-  // dW1, db1
-  hipLaunchKernelGGL(mlp_dw1_partial, dim3((MLP_H * MLP_F + 255) / 256, nch), dim3(256), 0, st,
-                     net->dh1, net->X, B, net->part);
-  hipLaunchKernelGGL(mlp_colsum_final, dim3((MLP_H * MLP_F + 255) / 256), dim3(256), 0, st,
-                     net->part, nch, MLP_H * MLP_F, gp + MLP_OW1);
-  hipLaunchKernelGGL(mlp_colsum_partial, dim3(H / 256, nch), dim3(256), 0, st, net->dh1, B, (int)H,
-                     H, (const float *)nullptr, net->part);
-  hipLaunchKernelGGL(mlp_colsum_final, dim3(H / 256), dim3(256), 0, st, net->part, nch, (int)H,
-                     gp + MLP_OB1);
+  // dz1, dW1, db1, then every sum over the row blocks
+  hipLaunchKernelGGL(mlp_in_kernel, dim3(nch), dim3(256), 0, st, net->dh1, net->h1b, net->X, B,
+                     net->part);
+  hipLaunchKernelGGL(mlp_final_kernel, dim3((MLP_PB3 + 64) / 64), dim3(1024), 0, st, net->part, nch,
+                     net->g);
   HIP_TRY(hipGetLastError());
   return XCS_OK;
 }
@@ -715,9 +858,9 @@ int xcs_mrhs_samples(xcs_mrhs *h, int per, unsigned int seed, float *X_out, floa
   if (!r) r = grab((void **)&Lo, 4 * (size_t)S * per);
   if (!r) {
     // G[s*n + j] = sum_i A[j*m + i] y_s[i]
-    hipLaunchKernelGGL(f32_gemm_kernel<false>, dim3((unsigned)((n + 63) / 64), (unsigned)((S + 63) / 64), 1),
+    hipLaunchKernelGGL(f32_gemm_kernel, dim3((unsigned)((n + 63) / 64), (unsigned)((S + 63) / 64), 1),
                        dim3(256), 0, h->stream, (int)n, (int)S, (int)m, (const float *)h->A32, m, 1L,
-                       (const void *)h->D.y, m, 1L, G, 1L, n, 1, 0L);
+                       h->D.y, m, 1L, G, 1L, n, 1, 0L);
     hipLaunchKernelGGL(mlp_features_kernel, dim3((unsigned)S), dim3(1024), 0, h->stream, G, (int)n,
                        (int)m, h->k, Xf);
     hipLaunchKernelGGL(mlp_samples_kernel, dim3((unsigned)S), dim3(1024), 0, h->stream, G, Xf,
