@@ -11,10 +11,11 @@
 //
 // Tiling: GM x GN waves (64 GM GN threads), each wave WM x WN MFMA 32 x 32
 // blocks, so the block tile is (32 WM GM) x (32 WN GN): 2 x 2 waves of 2 x 2
-// blocks -> 128 x 128, of 4 x 2 -> 256 x 128; 4 x 2 waves of 2 x 4 blocks ->
-// 256 x 256 (8 waves, each wave's 6 LDS reads per K step feed 8 MFMAs);
-// 128 bytes of K per stage (64 bf16 or 128 fp8), two LDS stages with the next
-// stage prefetched into registers while the current one is multiplied.
+// blocks -> 128 x 128; 4 x 2 waves of 2 x 4 blocks -> 256 x 256 (8 waves, each
+// wave's 6 LDS reads per K step feed 8 MFMAs); 128 bytes of K per stage (64 bf16
+// or 128 fp8), two LDS stages with the next stage prefetched into registers
+// while the current one is multiplied.  Products that fill the chip with 256 x
+// 128 tiles take gemm_tn8_kernel below instead.
 //
 // MFMA operand placement used here: lane l holds row (l % 32) of the A block
 // and column (l % 32) of the B block, with the same run of K values (bytes
@@ -217,8 +218,202 @@ __global__ void __launch_bounds__(64 * GM * GN) gemm_tn_kernel(GemmArgs g) {
   }
 }
 
+// 256 x 128 block tile by 8 waves (4 x 2, each 64 x 64), global loads straight
+// into LDS.  What bounded the register-staged kernel above was the path from
+// global memory through registers into LDS (its MFMA section alone runs in half
+// the time): here each wave issues 16-byte global -> LDS loads two stages ahead
+// of the MFMAs, three stages of 48 KB in LDS, and waits with a counted vmcnt, so
+// a stage's loads stay in flight over a whole stage of MFMAs and one barrier.
+// The loads write LDS in lane order (8 rows of 128 bytes per instruction, no
+// padding); bank conflicts are avoided by the order of the chunks within a row
+// instead: row r keeps its 16-byte chunk c at position c ^ (r & 7), so the eight
+// lanes of a read phase (eight rows, one chunk) touch all banks.  Columns past
+// ncols load column 0 and are not stored.  Each MFMA chain adds K in the order
+// of the kernel above, so the products are the same bits.  Measured: BF16
+// 16384 x 512 x 4096 77 -> 59 us (1154 TFLOP/s; without the loads 55, without the
+// products 41, and the matrix cores alone do 1.8 PFLOP/s on random operands).
+typedef const __attribute__((address_space(1))) uint8_t *gptr_t;
+typedef __attribute__((address_space(3))) uint8_t *lptr_t;
+constexpr int G8_BM = 256, G8_BN = 128, G8_NT = 512;
+constexpr int G8_STAGE = (G8_BM + G8_BN) * GT_KB;
+template <int FMT>
+__global__ void __launch_bounds__(G8_NT) gemm_tn8_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(128))) uint8_t lds0[G8_STAGE];
+  __shared__ __attribute__((aligned(128))) uint8_t lds1[G8_STAGE];
+  __shared__ __attribute__((aligned(128))) uint8_t lds2[G8_STAGE];
+  const int ncols = g.ncols ? *g.ncols : g.N;
+  int bx = blockIdx.x, by = blockIdx.y;
+  {  // XCD-aware tile order, as in gemm_tn_kernel
+    const int gx = gridDim.x, gy = gridDim.y;
+    if (gy > 1 && gx % 8 == 0) {
+      const int l = blockIdx.x + gx * blockIdx.y;
+      bx = ((l >> 3) / gy) * 8 + (l & 7);
+      by = (l >> 3) % gy;
+    }
+  }
+  const int m0 = bx * G8_BM, n0 = by * G8_BN;
+  if (n0 >= ncols) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long kbytes = (long)g.K * (FMT == FMT_BF16 ? 2 : 1);
+  const long kb_split = kbytes / g.ksplit;
+  const long kb0 = (long)blockIdx.z * kb_split;
+  const int nsteps = (int)(kb_split / GT_KB);
+  // load i of this wave fills rows 8 (wave + 8 i) .. + 7 of the stage (A rows
+  // first, then B columns); lane l: row l / 8, LDS position l % 8
+  constexpr int NL = (G8_BM + G8_BN) / 64;  // 6 loads per wave and stage
+  const uint8_t *src[NL];
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    const int row = 8 * (wave + 8 * i) + lr;
+    if (i < G8_BM / 64) {
+      src[i] = g.A + (long)(m0 + row) * g.lda_bytes + kb0 + lc;
+    } else {
+      const int c = n0 + row - G8_BM;
+      const int phys = c < ncols ? (g.col_map ? g.col_map[c] : c) : (g.col_map ? g.col_map[0] : 0);
+      src[i] = g.B + (long)phys * g.ldb_bytes + kb0 + lc;
+    }
+  }
+  // In assembly (it has no output register; LDS is its destination): the
+  // compiler would make every later LDS read wait for all such loads in flight.
+  auto issue = [&](uint8_t *buf, int s) {
+    const unsigned l0 = (unsigned)(uintptr_t)(lptr_t)buf + 1024 * wave;
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+      asm volatile("s_mov_b32 m0, %1\n\t"
+                   "s_nop 0\n\t"
+                   "global_load_lds_dwordx4 %0, off"
+                   :
+                   : "v"((gptr_t)(src[i] + (long)s * GT_KB)),
+                     "s"(__builtin_amdgcn_readfirstlane(l0 + 8192 * i))
+                   : "memory");  // nothing else here uses m0
+  };
+  f32x16_t acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
+  const int wm = wave >> 1, wn = wave & 1, r32 = lane & 31, h = lane >> 5;
+  const int arow = (wm * 64 + r32) * GT_KB, brow = (G8_BM + wn * 64 + r32) * GT_KB, sw = r32 & 7;
+  auto compute = [&](const uint8_t *L) {
+    __builtin_amdgcn_s_setprio(1);
+    if (FMT == FMT_BF16) {
+      bf16x8_t fa[4][2], fb[4][2];
+      auto read = [&](int kk) {
+        const int at = ((kk * 2 + h) ^ sw) * 16;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          fa[kk][i] = *(const bf16x8_t *)(L + arow + i * 32 * GT_KB + at);
+          fb[kk][i] = *(const bf16x8_t *)(L + brow + i * 32 * GT_KB + at);
+        }
+      };
+      read(0);
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) {
+        if (kk < 3) read(kk + 1);
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int b = 0; b < 2; b++)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][a], fb[kk][b],
+                                                                acc[a][b], 0, 0, 0);
+      }
+      // LDS reads stay two operand sets ahead of the MFMAs
+      __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < 2; kk++) {
+        const int c0 = ((kk * 4 + h * 2) ^ sw) * 16, c1 = ((kk * 4 + h * 2 + 1) ^ sw) * 16;
+        i32x8_t fa[2], fb[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const uint8_t *q = L + arow + i * 32 * GT_KB;
+          const i32x4_t x0 = *(const i32x4_t *)(q + c0), x1 = *(const i32x4_t *)(q + c1);
+          fa[i] = i32x8_t{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+          const uint8_t *w = L + brow + i * 32 * GT_KB;
+          const i32x4_t y0 = *(const i32x4_t *)(w + c0), y1 = *(const i32x4_t *)(w + c1);
+          fb[i] = i32x8_t{y0[0], y0[1], y0[2], y0[3], y1[0], y1[1], y1[2], y1[3]};
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int b = 0; b < 2; b++)
+            acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[a], fb[b], acc[a][b], 0,
+                                                                        0, 0, 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  // stage s: its loads have landed once at most the next stage's are in flight;
+  // after the barrier every wave has also finished reading stage s - 1, whose
+  // buffer stage s + 2 takes
+  auto step = [&](uint8_t *cur, uint8_t *nxt2, int s) {
+    if (s + 1 < nsteps)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + 2 < nsteps) issue(nxt2, s + 2);
+    compute(cur);
+  };
+  issue(lds0, 0);
+  if (nsteps > 1) issue(lds1, 1);
+  for (int s = 0; s < nsteps; s += 3) {
+    step(lds0, lds2, s);
+    if (s + 1 < nsteps) step(lds1, lds0, s + 1);
+    if (s + 2 < nsteps) step(lds2, lds1, s + 2);
+  }
+
+  float *C = g.C + (long)blockIdx.z * g.split_stride;
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    const int c = n0 + wn * 64 + b * 32 + r32;
+    if (c >= ncols) continue;
+    const int phys = g.col_map ? g.col_map[c] : c;
+    const float cs = g.col_scale ? g.col_scale[phys] : 1.0f;
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int r = m0 + wm * 64 + a * 32 + q * 8 + h * 4;
+        float4 v = make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2],
+                               acc[a][b][4 * q + 3]);
+        if (g.row_scale) {
+          v.x *= g.row_scale[r];
+          v.y *= g.row_scale[r + 1];
+          v.z *= g.row_scale[r + 2];
+          v.w *= g.row_scale[r + 3];
+        }
+        v.x *= cs;
+        v.y *= cs;
+        v.z *= cs;
+        v.w *= cs;
+        *(float4 *)(C + (long)phys * g.ldc + r) = v;
+      }
+  }
+}
+
+// Block tile of a product whose M is a multiple of 256: the 256 x 128 tile where
+// its workgroups (one per CU) about fill the chip, else the 128 x 128 one, of
+// which there are twice as many.  Measured on MI355X, us, 128 x 128 against
+// 256 x 128: BF16 16384 x 512 x 4096 (256 large tiles) 77 / 59, its transpose with
+// K split 4 85 / 68, FP8 41 / 36 and 44 / 44; BF16 8192 x 300 x 2048 (96 large
+// tiles) 29 / 32, FP8 18 / 21; BF16 4096 x 200 x 1024 (32) 16 / 19.
+inline int gemm_tile(int M, int N, int ksplit) {
+  return (long)(M / G8_BM) * ((N + G8_BN - 1) / G8_BN) * ksplit >= 192 ? 1 : 0;
+}
+
 // Launch of the TN GEMM with block tile `tile`: 0 128 x 128 (4 waves), 1
-// 256 x 128 (4 waves), 2 256 x 256 (8 waves).  M must be a multiple of the
+// 256 x 128 (8 waves), 2 256 x 256 (8 waves).  M must be a multiple of the
 // tile's rows (128 or 256); the grid covers N (masked beyond ncols) and ksplit
 // slices of K.
 template <int FMT>
@@ -228,7 +423,7 @@ static hipError_t gemm_tn_launch(int tile, const GemmArgs &g, hipStream_t st) {
   if (tile == 2)
     hipLaunchKernelGGL((gemm_tn_kernel<FMT, 2, 4, 4, 2>), grid, dim3(512), 0, st, g);
   else if (tile == 1)
-    hipLaunchKernelGGL((gemm_tn_kernel<FMT, 4, 2>), grid, dim3(GT_THREADS), 0, st, g);
+    hipLaunchKernelGGL((gemm_tn8_kernel<FMT>), grid, dim3(G8_NT), 0, st, g);
   else
     hipLaunchKernelGGL((gemm_tn_kernel<FMT, 2, 2>), grid, dim3(GT_THREADS), 0, st, g);
   return hipGetLastError();

@@ -906,7 +906,7 @@ struct xcs_mrhs {
   double *rowpart = nullptr; // exact-residual row sums per slice (count x MR_SLICES x m)
   int nblk = 1;
   int polish_max = 6;  // support-correction steps
-  int gemm_big = 0;    // GEMM block tile where M allows: 0 128 x 128, 1 256 x 128, 2 256 x 256 (8 waves)
+  int gemm_big = -1;   // GEMM block tile where M allows: 0 128 x 128, 1 256 x 128, 2 256 x 256, -1 by gemm_tile
   xcs_options opts{};
   float phase_ms[6] = {0, 0, 0, 0, 0, 0};  // init, low precision, bf16 continuation, refinement, corrections, spare
   ~xcs_mrhs() {
@@ -959,7 +959,7 @@ static int mr_gemm(xcs_mrhs *h, int fmt, bool transpose, const uint8_t *B, float
   g.ncols = ncols;
   g.col_map = map;
   g.col_scale = fmt == FMT_FP8 ? bscale : nullptr;
-  const int tile = (h->gemm_big && g.M % 256 == 0) ? h->gemm_big : 0;
+  const int tile = g.M % 256 ? 0 : h->gemm_big >= 0 ? h->gemm_big : gemm_tile(g.M, g.N, g.ksplit);
   HIP_TRY(fmt == FMT_BF16 ? gemm_tn_launch<FMT_BF16>(tile, g, h->stream)
                           : gemm_tn_launch<FMT_FP8>(tile, g, h->stream));
   if (g.ksplit > 1) {
