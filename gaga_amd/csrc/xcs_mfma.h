@@ -3,7 +3,8 @@
 // C = A_op * B_op with both operands K-contiguous ("TN"):
 //   A_op: M x K, row r at A + r * lda_bytes
 //   B_op: K x N, column c at B + col(c) * ldb_bytes
-//   C:    C[col(c) * ldc + r] (fp32), optionally one slice per K split
+//   C:    C[col(c) * ldc + r] or, by position, C[c * ldc + r] (fp32), optionally
+//         one slice per K split
 // col(c) = col_map ? col_map[c] : c for c < *ncols, so a product can run over
 // the active signals only.  Formats: BF16 (v_mfma_f32_32x32x16_bf16) and OCP
 // FP8 e4m3 (v_mfma_f32_32x32x64_f8f6f4, format code 0 for both operands);
@@ -53,6 +54,7 @@ struct GemmArgs {
   int ksplit;
   const int *ncols;      // device, nullable (then N)
   const int *col_map;    // device, nullable (identity)
+  int c_by_pos;          // C's columns by position c instead of col(c)
   const float *row_scale;  // per output row, nullable
   const float *col_scale;  // per physical column, nullable
 };
@@ -213,7 +215,7 @@ __global__ void __launch_bounds__(64 * GM * GN) gemm_tn_kernel(GemmArgs g) {
         v.y *= cs;
         v.z *= cs;
         v.w *= cs;
-        *(float4 *)(C + (long)phys * g.ldc + r) = v;
+        *(float4 *)(C + (long)(g.c_by_pos ? c : phys) * g.ldc + r) = v;
       }
   }
 }
@@ -397,7 +399,7 @@ __global__ void __launch_bounds__(G8_NT) gemm_tn8_kernel(GemmArgs g) {
         v.y *= cs;
         v.z *= cs;
         v.w *= cs;
-        *(float4 *)(C + (long)phys * g.ldc + r) = v;
+        *(float4 *)(C + (long)(g.c_by_pos ? c : phys) * g.ldc + r) = v;
       }
   }
 }

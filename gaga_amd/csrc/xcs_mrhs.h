@@ -34,554 +34,755 @@ namespace xcs {
 
 constexpr int MR_THREADS = 256;  // row-parallel kernels (one row or 4 rows per thread)
 constexpr int MR_VT = 1024;      // per-signal vector kernels (one workgroup per signal)
-constexpr int MR_KSPLIT = 4;  // K splits of the A * V products (K = n)
+constexpr int MR_KMAX = 16;      // K slices of a product (at most)
+constexpr int MR_HIST = 2048;    // histogram bins held in LDS
+constexpr int MR_XLDS = 16384;   // largest n whose x the selection holds in LDS (two workgroups per CU)
 
+// Products are stored by position: column c of a product belongs to the c-th
+// listed signal, and its K slices lie st_* floats apart; the kernel that uses a
+// product adds its slices as it reads it.
 struct MrhsDesc {
-  int m, n, k, count, num_bins, cstride, restart, maxiter, fmt;
+  int m, n, k, count, num_bins, cstride, restart, maxiter, fmt, words;
   float tol;
   const float *y;
-  float *x, *grad, *thres, *gprev, *gprev_thres, *resid, *resid_update, *aux, *tol_lp;
-  int *bins, *bins2, *counters, *stage, *mode;
+  float *x, *gprev, *resid, *aux, *tol_lp;
+  unsigned long long *mask, *mask2, *mask3;  // support bits (words per signal), scratch
+  int *counters, *stage, *mode, *wpos;
   XState *st;
-  uint8_t *xb, *rb, *vb1, *vb2;
-  float *sx, *sr, *sv1, *sv2;
-  float *ax, *g, *w1, *w2;
+  uint8_t *xb, *rb, *vb;  // operands; vb: the step's direction, then (count on) its gradient
+  float *sx, *sr, *sv;
+  float *ax, *g, *w;
+  int ks_ax, ks_g, ks_w;
+  long st_ax, st_g, st_w;
   const float *colscale;
-  int *active, *nactive, *ulist, *nu;
+  int *active, *nactive, *wlist;  // nactive[0]: active signals, [1]: columns of the step product
   double *ref;  // per signal: gamma, |r|^2, |y|^2, spare
   int *supp, *supp_cnt;
+  float *cp, *cd;  // refinement: CG direction and correction, by list position
   const float *A32;
 };
 
-__device__ __forceinline__ long mr_ldb(const MrhsDesc &D, int K) {
-  return (long)K * (D.fmt == FMT_BF16 ? 2 : 1);
+__device__ __forceinline__ float4 mr_ld4(const float *p, long o) {
+  return *reinterpret_cast<const float4 *>(p + o);
+}
+// Four (one) consecutive values of a product column, its K slices added in order.
+__device__ __forceinline__ float4 mr_sum4(const float *p, long stride, int ks, long o) {
+  float4 s = mr_ld4(p, o);
+  for (int z = 1; z < ks; z++) {
+    const float4 v = mr_ld4(p + z * stride, o);
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  return s;
+}
+__device__ __forceinline__ float mr_sum1(const float *p, long stride, int ks, long o) {
+  float s = p[o];
+  for (int z = 1; z < ks; z++) s += p[z * stride + o];
+  return s;
+}
+__device__ __forceinline__ float mr_get(const float4 &v, int e) {
+  return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
+}
+__device__ __forceinline__ uint2 mr_bf4(float4 v) {
+  return make_uint2((uint32_t)f2bf16_rne(v.x) | ((uint32_t)f2bf16_rne(v.y) << 16),
+                    (uint32_t)f2bf16_rne(v.z) | ((uint32_t)f2bf16_rne(v.w) << 16));
+}
+__device__ __forceinline__ float mr_max4(float4 v, float m) {
+  return fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w));
+}
+__device__ __forceinline__ float4 mr_mul4(float4 a, float4 b) {
+  return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w);
+}
+__device__ __forceinline__ float4 mr_keep4(float4 v, unsigned bits) {
+  return make_float4((bits & 1) ? v.x : 0.f, (bits & 2) ? v.y : 0.f, (bits & 4) ? v.z : 0.f,
+                     (bits & 8) ? v.w : 0.f);
+}
+__device__ __forceinline__ unsigned mr_bits4(const unsigned long long *mask, int q) {
+  return (unsigned)(mask[q >> 4] >> ((4 * q) & 63)) & 15u;
+}
+__device__ __forceinline__ float mr_fp8_scale(float mx) { return mx > 0.f ? mx / FP8_MAX : 1.0f; }
+__device__ __forceinline__ uint32_t mr_fp84(float4 v, float sc) {
+  return f2fp8x4(__fdiv_rn(v.x, sc), __fdiv_rn(v.y, sc), __fdiv_rn(v.z, sc), __fdiv_rn(v.w, sc));
 }
 
-// Per-signal descriptor for the engine's device functions (thread 0 fills it).
-__device__ void mr_view(XProblem &P, const MrhsDesc &D, int s, float tol) {
-  __builtin_memset(&P, 0, sizeof(P));
-  P.alg = ALG_CGIHT;
-  P.ens = ENS_GEN;
-  P.m = D.m;
-  P.n = D.n;
-  P.k = D.k;
-  P.lda = D.m;
-  P.num_bins = D.num_bins;
-  P.maxiter = D.maxiter;
-  P.restart = D.restart;
-  P.tol = tol;
-  const long n = D.n, m = D.m;
-  xset(P.y, D.y + s * m);
-  xset(P.x, D.x + s * n);
-  xset(P.thres, D.thres + s * n);
-  xset(P.grad, D.grad + s * n);
-  xset(P.gprev, D.gprev + s * n);
-  xset(P.gprev_thres, D.gprev_thres + s * n);
-  xset(P.bins, D.bins + s * n);
-  xset(P.bins2, D.bins2 + s * n);
-  xset(P.resid, D.resid + s * m);
-  xset(P.resid_update, D.resid_update + s * m);
-  xset(P.counters, D.counters + (long)s * D.cstride);
-  xset(P.st, D.st + s);
-}
-
-// v (times pre[i] when given) as column `col` of a B operand in the current
-// format; FP8 also writes the column scale.  v must be visible to the block.
-__device__ void mr_quant(Team &t, const MrhsDesc &D, const float *v, const float *pre, int len,
-                         uint8_t *base, float *scales, int col) {
+// The vector of float4s f(q), q < len / 4, as column `col` of a B operand in the
+// current format; FP8 also writes the column scale (f is evaluated twice).
+template <class F>
+__device__ __forceinline__ void mr_quant(const MrhsDesc &D, WgSlots &W, int &bank, F &&f, int len,
+                                         uint8_t *base, float *scales, long col) {
   if (D.fmt == FMT_BF16) {
-    uint16_t *o = (uint16_t *)(base + (long)col * len * 2);
-    for (int i = threadIdx.x; i < len; i += blockDim.x) {
-      const float a = pre ? v[i] * pre[i] : v[i];
-      o[i] = f2bf16_rne(a);
-    }
+    uint2 *o = reinterpret_cast<uint2 *>(base + col * len * 2);
+    for (int q = threadIdx.x; q < len / 4; q += blockDim.x) o[q] = mr_bf4(f(q));
     return;
   }
-  float mx = 0.f;
-  for (int i = threadIdx.x; i < len; i += blockDim.x) mx = fmaxf(mx, fabsf(pre ? v[i] * pre[i] : v[i]));
-  double r[1] = {mx};
-  const int op[1] = {1};
-  team_reduce<double, 1>(t, r, op);
-  const float sc = r[0] > 0.0 ? (float)r[0] / FP8_MAX : 1.0f;
-  uint32_t *o = (uint32_t *)(base + (long)col * len);
-  for (int q = threadIdx.x; q < len / 4; q += blockDim.x) {
-    float a[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int i = 4 * q + e;
-      a[e] = __fdiv_rn(pre ? v[i] * pre[i] : v[i], sc);
-    }
-    o[q] = f2fp8x4(a[0], a[1], a[2], a[3]);
-  }
+  float mx[1] = {0.f};
+  double none[1];
+  for (int q = threadIdx.x; q < len / 4; q += blockDim.x) mx[0] = mr_max4(f(q), mx[0]);
+  wg_reduce<0, 1>(W, bank, none, mx);
+  const float sc = mr_fp8_scale(mx[0]);
+  uint32_t *o = reinterpret_cast<uint32_t *>(base + col * len);
+  for (int q = threadIdx.x; q < len / 4; q += blockDim.x) o[q] = mr_fp84(f(q), sc);
   if (threadIdx.x == 0) scales[col] = sc;
 }
 
-__device__ __forceinline__ const float *mr_pre(const MrhsDesc &D) {
-  return D.fmt == FMT_FP8 ? D.colscale : nullptr;
+// FP8 A V operands carry A's column scales.
+__device__ __forceinline__ float4 mr_pre4(const MrhsDesc &D, float4 v, int q) {
+  return D.fmt == FMT_FP8 ? mr_mul4(v, mr_ld4(D.colscale, 4 * q)) : v;
 }
-
-#define MR_PROLOGUE(tolv)                            \
-  __shared__ Lds L;                                  \
-  __shared__ XProblem sP;                            \
-  const int s = blockIdx.x;                          \
-  if (threadIdx.x == 0) mr_view(sP, D, s, (tolv));   \
-  __syncthreads();                                   \
-  Team t{0, 1, nullptr, 0, nullptr};                 \
-  const XProblem &P = sP;                            \
-  (void)L;                                           \
-  (void)t;
 
 // y as the first right-hand side operand (A^T y).
 __global__ void __launch_bounds__(MR_VT) mr_init0_kernel(MrhsDesc D) {
-  const int s = blockIdx.x;
-  Team t{0, 1, nullptr, 0, nullptr};
-  mr_quant(t, D, D.y + (long)s * D.m, nullptr, D.m, D.rb, D.sr, s);
+  __shared__ WgSlots W;
+  int bank = 0;
+  const long s = blockIdx.x;
+  mr_quant(D, W, bank, [&](int q) { return mr_ld4(D.y + s * D.m, 4 * q); }, D.m, D.rb, D.sr, s);
+}
+
+// Scalars of a support selection.
+struct MrSel {
+  int k_bin, sum, max_bin;
+  float alpha_bin, min_val, slope;
+};
+
+// FindSupportSet's binning branch (functions.cu:404-428) on x (LDS or memory,
+// visible to the workgroup) with max |x| = max_value: the threshold, and the new
+// support bits.  Returns whether an entry left.  Ends with __syncthreads.
+__device__ __forceinline__ bool mr_select(const MrhsDesc &D, float *x, unsigned long long *mask,
+                                          int *hist, int *counters, float max_value, MrSel &S) {
+  const int nt = blockDim.x, lane = threadIdx.x & (WAVE - 1);
+  S.slope = (float)(D.num_bins - 1) / max_value;
+  const float slope = S.slope, inter = max_value;
+  const int mb = S.max_bin;
+  const bool lds = D.num_bins <= MR_HIST;
+  for (int b = threadIdx.x; b < mb; b += nt)
+    if (lds)
+      hist[b] = 0;
+    else
+      counters[b] = 0;
+  __syncthreads();
+  for (int j = threadIdx.x; j < D.n; j += nt) {
+    const float v = x[j];
+    const int b = linear_bin(v, slope, inter);
+    if ((double)fabsf(v) > (double)inter * .000001 && b < mb) {
+      if (lds)
+        atomicAdd(&hist[b], 1);
+      else
+        atomicAdd(&counters[b], 1);
+    }
+  }
+  __syncthreads();
+  int kb = -1, sum = 0;
+  if (D.k > 0) {
+    if (lds)
+      kb = sp_walk([&](int b) { return hist[b]; }, 0, mb, 0, D.k, &sum);
+    else
+      kb = sp_walk([&](int b) { return ((volatile int *)counters)[b]; }, 0, mb, 0, D.k, &sum);
+  }
+  if (sum < D.k) {
+    S.alpha_bin = S.alpha_bin * 0.5f;
+    S.max_bin = (int)((float)D.num_bins * (1.0f - S.alpha_bin));
+  }
+  S.min_val = __fsub_rn(inter, __fdiv_rn((float)(kb + 1), slope));
+  S.sum = sum;
+  S.k_bin = kb;
+  int left = 0;
+  for (int j = threadIdx.x; j < D.n; j += nt) {  // n and nt are multiples of 64: whole waves
+    const bool in = linear_bin(x[j], slope, inter) <= kb;
+    if (!in) x[j] = 0.f;
+    const unsigned long long bits = __ballot(in);
+    if (lane == 0) {
+      if (mask[j >> 6] & ~bits) left = 1;
+      mask[j >> 6] = bits;
+    }
+  }
+  return __syncthreads_or(left) != 0;
 }
 
 // x = A^T y, first support (algorithms.cu:3752-3790 with solve_instance's init).
+template <bool XL>
 __global__ void __launch_bounds__(MR_VT) mr_init1_kernel(MrhsDesc D, float c_lp) {
-  MR_PROLOGUE(D.tol);
-  XState S;
-  __builtin_memset(&S, 0, sizeof(S));
-  S.alpha_bin = 0.25f;
-  S.max_bin = (int)((float)P.num_bins * (1.0f - S.alpha_bin));
-  S.max_change = 1.0f;
-  S.diff = 1.f;
-  S.cycle = 1;
-  S.beta_to_zero = 1;
-  S.supp_change = 1;
-  for (int j = 0; j < 16; j++) S.evo[j] = 1.f;
-  const float *G = D.g + (long)s * D.n;
-  double e2 = 0.0;
-  for (int i = threadIdx.x; i < P.m; i += blockDim.x) {
-    const float r = P.y[i];
-    P.resid[i] = r;
-    e2 += (double)r * (double)r;
+  __shared__ WgSlots W;
+  __shared__ int hist[MR_HIST];
+  __shared__ __attribute__((aligned(16))) float xs[XL ? MR_XLDS : 4];
+  int bank = 0;
+  const long s = blockIdx.x;
+  const int n = D.n, nt = blockDim.x;
+  float *x = XL ? xs : D.x + s * n;
+  double e2[1] = {0.0};
+  float xm[1] = {0.f};
+  for (int q = threadIdx.x; q < D.m / 4; q += nt) {
+    const float4 r = mr_ld4(D.y + s * D.m, 4 * q);
+    e2[0] += (double)r.x * (double)r.x + (double)r.y * (double)r.y + (double)r.z * (double)r.z +
+             (double)r.w * (double)r.w;
   }
-  zero_counters(t, P);
-  float xm = 0.f;
-  for (int j = threadIdx.x; j < P.n; j += blockDim.x) {
-    const float v = G[j];
-    P.x[j] = v;
-    xm = fmaxf(xm, fabsf(v));
+  for (int q = threadIdx.x; q < n / 4; q += nt) {
+    const float4 v = mr_sum4(D.g, D.st_g, D.ks_g, s * n + 4 * q);
+    *reinterpret_cast<float4 *>(x + 4 * q) = v;
+    xm[0] = mr_max4(v, xm[0]);
   }
-  double v[2] = {e2, xm};
-  const int op[2] = {0, 1};
-  team_reduce<double, 2>(t, v, op);
-  S.err = (float)sqrt(v[0]);
-  S.err_start = S.err;
-  S.max_value = (float)v[1];
+  for (int w = threadIdx.x; w < D.words; w += nt) D.mask[s * D.words + w] = 0ull;
+  wg_reduce<1, 1>(W, bank, e2, xm);
+  MrSel S{0, 0, (int)((float)D.num_bins * (1.0f - 0.25f)), 0.25f, 0.f, 0.f};
+  const bool zero = xm[0] == 0.f;
+  if (!zero)
+    (void)mr_select(D, x, D.mask + s * D.words, hist, D.counters + s * D.cstride, xm[0], S);
+  else
+    __syncthreads();
+  if (XL)
+    for (int q = threadIdx.x; q < n / 4; q += nt)
+      *reinterpret_cast<float4 *>(D.x + s * n + 4 * q) = *reinterpret_cast<float4 *>(x + 4 * q);
+  if (!zero)
+    mr_quant(D, W, bank, [&](int q) { return mr_pre4(D, *reinterpret_cast<float4 *>(x + 4 * q), q); },
+             n, D.xb, D.sx, s);
   if (threadIdx.x == 0) {
-    D.tol_lp[s] = fmaxf(D.tol, c_lp * S.err);
-    D.ref[4 * s + 2] = v[0];
+    const float err = (float)sqrt(e2[0]);
+    D.tol_lp[s] = fmaxf(D.tol, c_lp * err);
+    D.ref[4 * s + 2] = e2[0];
+    D.stage[s] = zero ? 1 : 0;
+    XState T;
+    __builtin_memset(&T, 0, sizeof(T));
+    T.initialized = 1;
+    T.done = zero ? 1 : 0;
+    T.max_change = 1.0f;
+    T.diff = 1.f;
+    T.cycle = 1;
+    T.beta_to_zero = 1;
+    T.supp_change = 1;
+    for (int j = 0; j < 16; j++) T.evo[j] = 1.f;
+    T.err = T.err_start = err;
+    T.max_value = xm[0];
+    T.k_bin = S.k_bin;
+    T.sum = S.sum;
+    T.max_bin = S.max_bin;
+    T.alpha_bin = S.alpha_bin;
+    T.min_val = S.min_val;
+    T.slope = S.slope;
+    D.st[s] = T;
   }
-  S.initialized = 1;
-  if (S.max_value == 0.f) {
-    S.done = 1;
-    if (threadIdx.x == 0) {
-      D.stage[s] = 1;
-      *P.st = S;
-    }
-    return;
+}
+
+// r = y - A x of one signal (product column pos) as the next A^T operand; returns |r|^2.
+__device__ __forceinline__ double mr_residual(const MrhsDesc &D, WgSlots &W, int &bank, long s,
+                                              long pos) {
+  double e2[1] = {0.0};
+  float mx[1] = {0.f};
+  auto r4 = [&](int q) {
+    const float4 y = mr_ld4(D.y + s * D.m, 4 * q);
+    const float4 a = mr_sum4(D.ax, D.st_ax, D.ks_ax, pos * D.m + 4 * q);
+    return make_float4(__fsub_rn(y.x, a.x), __fsub_rn(y.y, a.y), __fsub_rn(y.z, a.z),
+                       __fsub_rn(y.w, a.w));
+  };
+  const bool bf = D.fmt == FMT_BF16;
+  uint2 *ob = reinterpret_cast<uint2 *>(D.rb + s * D.m * 2);
+  for (int q = threadIdx.x; q < D.m / 4; q += blockDim.x) {
+    const float4 r = r4(q);
+    e2[0] += (double)r.x * (double)r.x + (double)r.y * (double)r.y + (double)r.z * (double)r.z +
+             (double)r.w * (double)r.w;
+    mx[0] = mr_max4(r, mx[0]);
+    if (bf) ob[q] = mr_bf4(r);
   }
-  S.slope = (float)(P.num_bins - 1) / S.max_value;
-  find_support_bin(t, L, P, P.x, P.bins, S, S.slope, S.max_value, &S.k_bin);
-  threshold_x(t, P, S.k_bin);
-  __syncthreads();
-  mr_quant(t, D, (const float *)P.x, mr_pre(D), P.n, D.xb, D.sx, s);
-  if (threadIdx.x == 0) {
-    D.stage[s] = 0;
-    *P.st = S;
+  wg_reduce<1, 1>(W, bank, e2, mx);
+  if (!bf) {
+    const float sc = mr_fp8_scale(mx[0]);
+    uint32_t *o = reinterpret_cast<uint32_t *>(D.rb + s * D.m);
+    for (int q = threadIdx.x; q < D.m / 4; q += blockDim.x) o[q] = mr_fp84(r4(q), sc);
+    if (threadIdx.x == 0) D.sr[s] = sc;
   }
+  return e2[0];
 }
 
 // r^0 = y - A x (algorithms.cu:3791-3800).
 __global__ void __launch_bounds__(MR_VT) mr_init2_kernel(MrhsDesc D) {
-  MR_PROLOGUE(D.tol);
+  __shared__ WgSlots W;
+  int bank = 0;
+  const long s = blockIdx.x;
   if (D.stage[s] != 0) return;
-  XState S = *P.st;
-  const float *AX = D.ax + (long)s * D.m;
-  double e2 = 0.0;
-  for (int i = threadIdx.x; i < P.m; i += blockDim.x) {
-    const float r = __fsub_rn(P.y[i], AX[i]);
-    P.resid[i] = r;
-    e2 += (double)r * (double)r;
-  }
-  double v[1] = {e2};
-  const int op[1] = {0};
-  team_reduce<double, 1>(t, v, op);
-  S.err = (float)sqrt(v[0]);
-  S.prev[15] = S.err;
-  mr_quant(t, D, (const float *)P.resid, nullptr, P.m, D.rb, D.sr, s);
-  if (threadIdx.x == 0) *P.st = S;
-}
-
-// first gradient and its restriction (algorithms.cu:3801-3808); loop entry test.
-__global__ void __launch_bounds__(MR_VT) mr_init3_kernel(MrhsDesc D) {
-  MR_PROLOGUE(D.tol_lp[blockIdx.x]);
-  if (D.stage[s] != 0) return;
-  XState S = *P.st;
-  const float *G = D.g + (long)s * D.n;
-  for (int j = threadIdx.x; j < P.n; j += blockDim.x) {
-    const float gj = G[j];
-    P.gprev[j] = gj;
-    P.gprev_thres[j] = (P.bins[j] <= S.k_bin) ? gj : 0.f;
-  }
-  for (int j = 0; j < 15; j++) S.evo[j] = S.evo[j + 1];
-  S.evo[15] = S.prev[14] - S.prev[15];
-  S.beta_to_zero = 1;
-  S.supp_change = 1;
-  int reason;
-  if (!should_continue(S, P, &reason)) {
-    S.done = 1;
-    S.stop_reason = reason;
-  }
-  __syncthreads();
+  const float err = (float)sqrt(mr_residual(D, W, bank, s, s));
   if (threadIdx.x == 0) {
-    if (S.done) D.stage[s] = 1;
-    *P.st = S;
+    D.st[s].err = err;
+    D.st[s].prev[15] = err;
   }
 }
 
-// Active signals (stage 0) and the ones taking an unrestricted step, in
-// ascending order; one workgroup.
+__device__ __forceinline__ ResStop mr_stop(const XState &T) {
+  return ResStop{T.err, T.err_start, T.diff, T.iter, T.fail, T.cycle};
+}
+// The stop rules for one signal at its low-precision tolerance.
+__device__ __forceinline__ bool mr_continue(const MrhsDesc &D, long s, const ResStop &S,
+                                            int *reason) {
+  XProblem P;
+  P.tol = D.tol_lp[s];
+  P.maxiter = D.maxiter;
+  return res_continue(S, P, reason);
+}
+
+// first gradient (algorithms.cu:3801-3808); loop entry test.
+__global__ void __launch_bounds__(MR_VT) mr_init3_kernel(MrhsDesc D) {
+  const long s = blockIdx.x;
+  if (D.stage[s] != 0) return;
+  for (int q = threadIdx.x; q < D.n / 4; q += blockDim.x)
+    *reinterpret_cast<float4 *>(D.gprev + s * D.n + 4 * q) =
+        mr_sum4(D.g, D.st_g, D.ks_g, s * D.n + 4 * q);
+  if (threadIdx.x < WAVE) {
+    XState &T = D.st[s];
+    const int lane = threadIdx.x;
+    float evo = lane < 16 ? T.evo[lane] : 0.f;
+    evo = hist_push(evo, __fsub_rn(T.prev[14], T.prev[15]));
+    if (lane < 16) T.evo[lane] = evo;
+    if (lane == 0) {
+      int reason;
+      if (!mr_continue(D, s, mr_stop(T), &reason)) {
+        T.done = 1;
+        T.stop_reason = reason;
+        D.stage[s] = 1;
+      }
+    }
+  }
+}
+
+// Active signals (stage 0) in ascending order, and the columns of the step's
+// product: the active signals' directions, then the gradients (columns from
+// count on) of those taking an unrestricted step, whose place wpos records; one
+// workgroup.
 __global__ void __launch_bounds__(MR_THREADS) mr_list_kernel(MrhsDesc D) {
   __shared__ int base_a, base_u;
   if (threadIdx.x == 0) base_a = base_u = 0;
   __syncthreads();
-  for (int c0 = 0; c0 < D.count; c0 += blockDim.x) {
-    const int s = c0 + threadIdx.x;
-    int act = 0, u = 0;
-    if (s < D.count && D.stage[s] == 0) {
-      act = 1;
-      u = (!D.restart && D.st[s].supp_change) ? 1 : 0;
-      D.mode[s] = u;
+  for (int pass = 0; pass < 2; pass++) {  // the second list starts where the first ends
+    for (int c0 = 0; c0 < D.count; c0 += blockDim.x) {
+      const int s = c0 + threadIdx.x;
+      const int act = s < D.count && D.stage[s] == 0;
+      const int u = act && !D.restart && D.st[s].supp_change;
+      const int f = pass ? u : act;
+      int tot;
+      const int pos = (pass ? base_u : base_a) + wg_exclusive_scan(f, &tot);
+      if (act && !pass) {
+        D.mode[s] = u;
+        D.active[pos] = s;
+        D.wlist[pos] = s;
+      }
+      if (u && pass) {
+        D.wlist[base_a + pos] = D.count + s;
+        D.wpos[s] = base_a + pos;
+      }
+      __syncthreads();
+      if (threadIdx.x == 0) (pass ? base_u : base_a) += tot;
+      __syncthreads();
     }
-    int ta, tu;
-    const int pa = wg_exclusive_scan(act, &ta);
-    const int pu = wg_exclusive_scan(u, &tu);
-    if (act) D.active[base_a + pa] = s;
-    if (u) D.ulist[base_u + pu] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      base_a += ta;
-      base_u += tu;
-    }
-    __syncthreads();
   }
   if (threadIdx.x == 0) {
-    *D.nactive = base_a;
-    *D.nu = base_u;
+    D.nactive[0] = base_a;
+    D.nactive[1] = base_a + base_u;
   }
 }
 
-// Step part 1: r = y - A x (into resid for the restricted step, resid_update
-// for the unrestricted one), ||r|| into the history.
+// The signal of this workgroup, or -1: the blockIdx-th active one (sel), or
+// signal blockIdx itself.
+__device__ __forceinline__ int mr_signal(const MrhsDesc &D, int sel, int b) {
+  if (!sel) return b;
+  return b < D.nactive[0] ? D.active[b] : -1;
+}
+
+// Step part 1: r = y - A x, ||r|| into the history.
 __global__ void __launch_bounds__(MR_VT) mr_k1_kernel(MrhsDesc D) {
-  MR_PROLOGUE(D.tol_lp[blockIdx.x]);
-  if (D.stage[s] != 0) return;
-  XState S = *P.st;
-  const bool u = D.mode[s] != 0;
-  const float *AX = D.ax + (long)s * D.m;
-  float *r = u ? (float *)P.resid_update : (float *)P.resid;
-  double e2 = 0.0;
-  for (int i = threadIdx.x; i < P.m; i += blockDim.x) {
-    const float v = __fsub_rn(P.y[i], AX[i]);
-    r[i] = v;
-    e2 += (double)v * (double)v;
+  __shared__ WgSlots W;
+  int bank = 0;
+  const int s = mr_signal(D, 1, blockIdx.x);
+  if (s < 0) return;
+  const float norm = (float)sqrt(mr_residual(D, W, bank, s, blockIdx.x));
+  if (threadIdx.x < WAVE) {
+    float prev = threadIdx.x < 16 ? D.st[s].prev[threadIdx.x] : 0.f;
+    prev = hist_push(prev, norm);
+    if (threadIdx.x < 16) D.st[s].prev[threadIdx.x] = prev;
   }
-  double v[1] = {e2};
-  const int op[1] = {0};
-  team_reduce<double, 1>(t, v, op);
-  push16(S.prev, (float)sqrt(v[0]));
-  mr_quant(t, D, r, nullptr, P.m, D.rb, D.sr, s);
-  if (threadIdx.x == 0) *P.st = S;
 }
 
 // Step part 2 (after g = A^T r): restricted: beta and the new direction,
 // whose restriction is the next product's operand (functions.cu:1004-1060);
 // unrestricted: the old restricted direction and the restricted gradient
-// are the operands (functions.cu:1107-1160).
+// are the operands (functions.cu:1107-1160).  The gradient stays in its product
+// (not copied), restrictions come from the support bits: the pass is bound by
+// memory, and each vector is read or written once.
 __global__ void __launch_bounds__(MR_VT) mr_k2_kernel(MrhsDesc D) {
-  MR_PROLOGUE(D.tol_lp[blockIdx.x]);
-  if (D.stage[s] != 0) return;
-  XState S = *P.st;
-  const int kb = S.k_bin;
-  const float *G = D.g + (long)s * D.n;
+  __shared__ WgSlots W;
+  int bank = 0;
+  const int pos = blockIdx.x, s = mr_signal(D, 1, pos);
+  if (s < 0) return;
+  const int n = D.n, nt = blockDim.x;
+  const unsigned long long *mask = D.mask + (long)s * D.words;
+  float *gp = D.gprev + (long)s * n;
+  auto g4 = [&](int q) { return mr_sum4(D.g, D.st_g, D.ks_g, (long)pos * n + 4 * q); };
+  const bool bf = D.fmt == FMT_BF16;
   if (D.mode[s] == 0) {
-    float th2 = 0.f;
-    for (int j = threadIdx.x; j < P.n; j += blockDim.x) {
-      const float gj = G[j];
-      P.grad[j] = gj;
-      const float th = (P.bins[j] <= kb) ? gj : 0.f;
-      P.thres[j] = th;
-      th2 = fmaf(th, th, th2);
+    double none[1];
+    double th2[1] = {0.0};
+    float nonef[1];
+    for (int q = threadIdx.x; q < n / 4; q += nt) {
+      const unsigned bits = mr_bits4(mask, q);
+      if (!bits) continue;
+      const float4 g = mr_keep4(g4(q), bits);
+      th2[0] += (double)fmaf(g.x, g.x, fmaf(g.y, g.y, fmaf(g.z, g.z, g.w * g.w)));
     }
-    float beta;
-    {
-      double v[1] = {th2};
-      const int op[1] = {0};
-      team_reduce<double, 1>(t, v, op);
-      const float mu_new = (float)v[0];
-      if (S.beta_to_zero == 1) {
-        beta = 0.f;
-        S.mu = mu_new;
-      } else {
-        beta = S.mu;
-        S.mu = mu_new;
-        beta = (S.mu < 1000.0f * beta) ? S.mu / beta : 0.f;
-      }
+    wg_reduce<1, 0>(W, bank, th2, nonef);
+    const float mu_old = D.st[s].mu, mu_new = (float)th2[0];
+    float beta = 0.f;
+    if (D.st[s].beta_to_zero != 1) beta = (mu_new < 1000.0f * mu_old) ? mu_new / mu_old : 0.f;
+    float mx[2] = {0.f, 0.f};  // max |p|, max of the operand
+    uint2 *ob = reinterpret_cast<uint2 *>(D.vb + (long)s * n * 2);
+    for (int q = threadIdx.x; q < n / 4; q += nt) {
+      const float4 g = g4(q), o = mr_ld4(gp, 4 * q);
+      const float4 v = make_float4(__fadd_rn(__fmul_rn(beta, o.x), g.x), __fadd_rn(__fmul_rn(beta, o.y), g.y),
+                                   __fadd_rn(__fmul_rn(beta, o.z), g.z), __fadd_rn(__fmul_rn(beta, o.w), g.w));
+      *reinterpret_cast<float4 *>(gp + 4 * q) = v;
+      mx[0] = mr_max4(v, mx[0]);
+      const float4 k = mr_keep4(v, mr_bits4(mask, q));
+      if (bf)
+        ob[q] = mr_bf4(k);
+      else
+        mx[1] = mr_max4(mr_pre4(D, k, q), mx[1]);
     }
-    float pmax = 0.f;
-    for (int j = threadIdx.x; j < P.n; j += blockDim.x) {
-      const float gp = __fadd_rn(__fmul_rn(beta, P.gprev[j]), P.grad[j]);
-      P.gprev[j] = gp;
-      P.gprev_thres[j] = (P.bins[j] <= kb) ? gp : 0.f;
-      pmax = fmaxf(pmax, fabsf(gp));
+    wg_reduce<0, 2>(W, bank, none, mx);
+    if (!bf) {
+      const float sc = mr_fp8_scale(mx[1]);
+      uint32_t *o = reinterpret_cast<uint32_t *>(D.vb + (long)s * n);
+      for (int q = threadIdx.x; q < n / 4; q += nt)
+        o[q] = mr_fp84(mr_pre4(D, mr_keep4(mr_ld4(gp, 4 * q), mr_bits4(mask, q)), q), sc);
+      if (threadIdx.x == 0) D.sv[s] = sc;
     }
-    double v[1] = {pmax};
-    const int op[1] = {1};
-    team_reduce<double, 1>(t, v, op);
-    if (threadIdx.x == 0) D.aux[4 * s] = (float)v[0];
-    mr_quant(t, D, (const float *)P.gprev_thres, mr_pre(D), P.n, D.vb1, D.sv1, s);
+    if (threadIdx.x == 0) {
+      D.aux[4 * (long)s] = mx[0];
+      D.st[s].mu = mu_new;
+    }
   } else {
-    for (int j = threadIdx.x; j < P.n; j += blockDim.x) {
-      const float gj = G[j];
-      P.grad[j] = gj;
-      P.thres[j] = (P.bins[j] <= kb) ? gj : 0.f;
-    }
-    __syncthreads();
-    mr_quant(t, D, (const float *)P.gprev_thres, mr_pre(D), P.n, D.vb1, D.sv1, s);
-    mr_quant(t, D, (const float *)P.thres, mr_pre(D), P.n, D.vb2, D.sv2, s);
+    mr_quant(D, W, bank,
+             [&](int q) { return mr_pre4(D, mr_keep4(mr_ld4(gp, 4 * q), mr_bits4(mask, q)), q); }, n,
+             D.vb, D.sv, s);
+    mr_quant(D, W, bank,
+             [&](int q) {
+               const unsigned bits = mr_bits4(mask, q);
+               const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+               return bits ? mr_pre4(D, mr_keep4(g4(q), bits), q) : z;
+             },
+             n, D.vb, D.sv, (long)D.count + s);
   }
-  if (threadIdx.x == 0) *P.st = S;
 }
 
 // Step part 3 (after the A p products): step length, x update, support
-// update and stopping rules (algorithms.cu:3835-3942).
+// update and stopping rules (algorithms.cu:3835-3942).  x is held in LDS where it
+// fits (XL): the selection passes over it three times.
+template <bool XL>
 __global__ void __launch_bounds__(MR_VT) mr_k3_kernel(MrhsDesc D) {
-  MR_PROLOGUE(D.tol_lp[blockIdx.x]);
-  if (D.stage[s] != 0) return;
-  XState S = *P.st;
-  const int n = P.n, m = P.m;
-  const float *W1 = D.w1 + (long)s * m, *W2 = D.w2 + (long)s * m;
-  float xm = 0.f;
+  __shared__ WgSlots W;
+  __shared__ int hist[MR_HIST];
+  __shared__ __attribute__((aligned(16))) float xs[XL ? MR_XLDS : 4];
+  int bank = 0;
+  const int pos = blockIdx.x, s = mr_signal(D, 1, pos);
+  if (s < 0) return;
+  const int n = D.n, m = D.m, nt = blockDim.x;
+  unsigned long long *mask = D.mask + (long)s * D.words;
+  float *gp = D.gprev + (long)s * n, *xg = D.x + (long)s * n;
+  float *x = XL ? xs : xg;
+  XState &T = D.st[s];
+  float mu = T.mu, max_change, alpha;
+  float mx[1] = {0.f};
+  float nonef[1];
+  double none[1];
+  auto w4 = [&](long col, int q) { return mr_sum4(D.w, D.st_w, D.ks_w, col * m + 4 * q); };
   if (D.mode[s] == 0) {
-    float a2 = 0.f;
-    for (int i = threadIdx.x; i < m; i += blockDim.x) {
-      const float w = W1[i];
-      P.resid_update[i] = w;
-      a2 = fmaf(w, w, a2);
+    double a2[1] = {0.0};
+    for (int q = threadIdx.x; q < m / 4; q += nt) {
+      const float4 v = w4(pos, q);
+      a2[0] += (double)fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w)));
     }
-    double v[1] = {a2};
-    const int op[1] = {0};
-    team_reduce<double, 1>(t, v, op);
-    float alpha = (float)v[0];
-    alpha = (S.mu < 1000.0f * alpha) ? S.mu / alpha : 0.f;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-      const float xn = fmaf(alpha, P.gprev[j], P.x[j]);
-      P.x[j] = xn;
-      xm = fmaxf(xm, fabsf(xn));
-    }
-    S.max_change = 2.0f * alpha * D.aux[4 * s];
+    wg_reduce<1, 0>(W, bank, a2, nonef);
+    alpha = (float)a2[0];
+    alpha = (mu < 1000.0f * alpha) ? mu / alpha : 0.f;
+    max_change = 2.0f * alpha * D.aux[4 * (long)s];
   } else {
-    const int kb = S.k_bin;
+    const long c2 = D.wpos[s];
     float beta = 0.f;
-    if (S.beta_to_zero != 1) {
-      float num = 0.f, den = 0.f;
-      for (int i = threadIdx.x; i < m; i += blockDim.x) {
-        num = fmaf(W1[i], W2[i], num);
-        den = fmaf(W1[i], W1[i], den);
+    if (T.beta_to_zero != 1) {
+      double v[2] = {0.0, 0.0};
+      for (int q = threadIdx.x; q < m / 4; q += nt) {
+        const float4 a = w4(pos, q), b = w4(c2, q);
+        v[0] += (double)fmaf(a.x, b.x, fmaf(a.y, b.y, fmaf(a.z, b.z, a.w * b.w)));
+        v[1] += (double)fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, a.w * a.w)));
       }
-      double v[2] = {num, den};
-      const int op[2] = {0, 0};
-      team_reduce<double, 2>(t, v, op);
+      wg_reduce<2, 0>(W, bank, v, nonef);
       beta = -((float)v[0]) / (float)v[1];
     }
-    float pmax = 0.f, an = 0.f, mu2 = 0.f, ad = 0.f;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-      const float gp = __fadd_rn(__fmul_rn(beta, P.gprev[j]), P.grad[j]);
-      P.gprev[j] = gp;
-      const float gpt = (P.bins[j] <= kb) ? gp : 0.f;
-      P.gprev_thres[j] = gpt;
-      pmax = fmaxf(pmax, fabsf(gp));
-      const float th = P.thres[j];
-      an = fmaf(gpt, th, an);
-      mu2 = fmaf(th, th, mu2);
+    double v[3] = {0.0, 0.0, 0.0};  // p.g_S, |g_S|^2, |A p_S|^2
+    float pm[1] = {0.f};
+    for (int q = threadIdx.x; q < n / 4; q += nt) {
+      const float4 g = mr_sum4(D.g, D.st_g, D.ks_g, (long)pos * n + 4 * q), o = mr_ld4(gp, 4 * q);
+      const float4 p = make_float4(__fadd_rn(__fmul_rn(beta, o.x), g.x), __fadd_rn(__fmul_rn(beta, o.y), g.y),
+                                   __fadd_rn(__fmul_rn(beta, o.z), g.z), __fadd_rn(__fmul_rn(beta, o.w), g.w));
+      *reinterpret_cast<float4 *>(gp + 4 * q) = p;
+      pm[0] = mr_max4(p, pm[0]);
+      const float4 h = mr_keep4(g, mr_bits4(mask, q));
+      v[0] += (double)fmaf(p.x, h.x, fmaf(p.y, h.y, fmaf(p.z, h.z, p.w * h.w)));
+      v[1] += (double)fmaf(h.x, h.x, fmaf(h.y, h.y, fmaf(h.z, h.z, h.w * h.w)));
     }
-    for (int i = threadIdx.x; i < m; i += blockDim.x) {
-      const float r = __fadd_rn(__fmul_rn(beta, W1[i]), W2[i]);
-      P.resid[i] = r;
-      ad = fmaf(r, r, ad);
-    }
-    double v[4] = {an, ad, pmax, mu2};
-    const int op[4] = {0, 0, 1, 0};
-    team_reduce<double, 4>(t, v, op);
-    const float alpha = (float)v[0] / (float)v[1];
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-      const float xn = fmaf(alpha, P.gprev[j], P.x[j]);
-      P.x[j] = xn;
-      xm = fmaxf(xm, fabsf(xn));
-    }
-    S.mu = (float)v[3];
-    S.max_change = 2.0f * alpha * (float)v[2];
-  }
-  __syncthreads();
-  S.beta_to_zero = 0;
-  if (S.min_val <= S.max_change) {
-    const int kb_prev = S.k_bin;
-    rebin_x(t, L, P, S, xm, true);
-    float ch = 0.f;
-    for (int j = threadIdx.x; j < n; j += blockDim.x)
-      if (P.bins2[j] <= kb_prev && P.bins[j] > S.k_bin) ch = 1.f;
-    double v[1] = {ch};
-    const int op[1] = {1};
-    team_reduce<double, 1>(t, v, op);
-    S.supp_change = v[0] > 0.0 ? 1 : 0;
-    if (S.supp_change) {
-      if (P.restart) {
-        S.beta_to_zero = 1;
-      } else {
-        for (int j = threadIdx.x; j < n; j += blockDim.x)
-          P.gprev_thres[j] = (P.bins[j] <= S.k_bin) ? P.gprev[j] : 0.f;
+    for (int q = threadIdx.x; q < m / 4; q += nt) {
+      const float4 a = w4(pos, q), b = w4(c2, q);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float r = __fadd_rn(__fmul_rn(beta, mr_get(a, e)), mr_get(b, e));
+        v[2] += (double)r * (double)r;
       }
     }
-  } else {
-    S.supp_change = 0;
-    S.min_val = S.min_val - S.max_change;
+    wg_reduce<3, 1>(W, bank, v, pm);
+    alpha = (float)v[0] / (float)v[2];
+    mu = (float)v[1];
+    max_change = 2.0f * alpha * pm[0];
   }
-  threshold_x(t, P, S.k_bin);
-  __syncthreads();
-  S.err = S.prev[15];
-  stop_update(S, 749);
-  S.iter++;
-  int reason;
-  if (!should_continue(S, P, &reason)) {
-    S.done = 1;
-    S.stop_reason = reason;
-  } else {
-    mr_quant(t, D, (const float *)P.x, mr_pre(D), n, D.xb, D.sx, s);
+  for (int q = threadIdx.x; q < n / 4; q += nt) {
+    const float4 p = mr_ld4(gp, 4 * q), o = mr_ld4(xg, 4 * q);
+    const float4 v = make_float4(fmaf(alpha, p.x, o.x), fmaf(alpha, p.y, o.y), fmaf(alpha, p.z, o.z),
+                                 fmaf(alpha, p.w, o.w));
+    *reinterpret_cast<float4 *>(x + 4 * q) = v;
+    mx[0] = mr_max4(v, mx[0]);
   }
-  __syncthreads();
+  wg_reduce<0, 1>(W, bank, none, mx);
+  MrSel S{T.k_bin, T.sum, T.max_bin, T.alpha_bin, T.min_val, T.slope};
+  float max_value = T.max_value;
+  bool left = false;
+  if (S.min_val <= max_change) {
+    max_value = mx[0];
+    left = mr_select(D, x, mask, hist, D.counters + (long)s * D.cstride, max_value, S);
+  } else {
+    S.min_val = S.min_val - max_change;
+    for (int q = threadIdx.x; q < n / 4; q += nt) {
+      float4 *o = reinterpret_cast<float4 *>(x + 4 * q);
+      *o = mr_keep4(*o, mr_bits4(mask, q));
+    }
+    __syncthreads();
+  }
+  // every wave applies the stopping rules to its own copy of the history
+  const int lane = threadIdx.x & (WAVE - 1);
+  const float prev = lane < 16 ? T.prev[lane] : 0.f;
+  float evo = lane < 16 ? T.evo[lane] : 0.f;
+  ResStop Q = mr_stop(T);
+  Q.err = lane_f(prev, 15);
+  res_stop_update(Q, prev, &evo, 749);
+  Q.iter++;
+  int reason = 0;
+  const bool go = mr_continue(D, s, Q, &reason);
+  __syncthreads();  // every wave has read the state
+  if (XL)
+    for (int q = threadIdx.x; q < n / 4; q += nt)
+      *reinterpret_cast<float4 *>(xg + 4 * q) = *reinterpret_cast<float4 *>(x + 4 * q);
+  if (go)
+    mr_quant(D, W, bank, [&](int q) { return mr_pre4(D, *reinterpret_cast<float4 *>(x + 4 * q), q); },
+             n, D.xb, D.sx, s);
+  if (threadIdx.x < 16) T.evo[threadIdx.x] = evo;
   if (threadIdx.x == 0) {
-    if (S.done) D.stage[s] = 1;
-    *P.st = S;
+    T.mu = mu;
+    T.max_change = max_change;
+    T.max_value = max_value;
+    T.k_bin = S.k_bin;
+    T.sum = S.sum;
+    T.max_bin = S.max_bin;
+    T.alpha_bin = S.alpha_bin;
+    T.min_val = S.min_val;
+    T.slope = S.slope;
+    T.supp_change = left ? 1 : 0;
+    T.beta_to_zero = left && D.restart ? 1 : 0;
+    T.err = Q.err;
+    T.diff = Q.diff;
+    T.iter = Q.iter;
+    T.fail = Q.fail;
+    T.cycle = Q.cycle;
+    if (!go) {
+      T.done = 1;
+      T.stop_reason = reason;
+      D.stage[s] = 1;
+    }
   }
 }
 
 // FP8 phase finished: continue every signal in BF16 (D.fmt is BF16 here).
 __global__ void __launch_bounds__(MR_VT) mr_switch_kernel(MrhsDesc D, float c_lp) {
-  MR_PROLOGUE(D.tol);
-  XState S = *P.st;
-  if (S.max_value == 0.f) return;  // A^T y = 0: nothing to continue
-  S.done = 0;
-  S.diff = 1.f;
-  S.cycle = 1;
-  S.fail = 0;
-  for (int j = 0; j < 16; j++) S.evo[j] = 1.f;
-  mr_quant(t, D, (const float *)P.x, nullptr, P.n, D.xb, D.sx, s);
+  __shared__ WgSlots W;
+  int bank = 0;
+  const long s = blockIdx.x;
+  XState &T = D.st[s];
+  if (T.max_value == 0.f) return;  // A^T y = 0: nothing to continue
+  mr_quant(D, W, bank, [&](int q) { return mr_ld4(D.x + s * D.n, 4 * q); }, D.n, D.xb, D.sx, s);
+  if (threadIdx.x < 16) T.evo[threadIdx.x] = 1.f;
   if (threadIdx.x == 0) {
+    T.done = 0;
+    T.diff = 1.f;
+    T.cycle = 1;
+    T.fail = 0;
     D.tol_lp[s] = fmaxf(D.tol, c_lp * (float)sqrt(D.ref[4 * s + 2]));
     D.stage[s] = 0;
-    *P.st = S;
   }
 }
 
 // ------------------------------------------------------------ refinement ---
-// Support lists.  topk = 0: the nonzeros of x (active signals only).
-// topk = 1: the refinement's support, the k largest
-// |x_j| (all nonzeros when there are at most k; ties at the k-th magnitude
-// taken in index order); x is cut to it and bins2 = 1 marks it.  The k-th
-// magnitude is found by a bitwise search on the IEEE bits of |x| (monotone
-// for non-negative floats).
-__global__ void __launch_bounds__(MR_VT) mr_ref_supp_kernel(MrhsDesc D, int topk, int sel) {
-  const int s = blockIdx.x;
-  if ((!topk || sel) && D.stage[s] != 0) return;
-  const long n = D.n;
-  float *x = D.x + s * n;
-  int *mask = D.bins2 + s * n, *sup = D.supp + s * n;
-  __shared__ int base;
-  __shared__ int cnt_s[MAX_WAVES];
-  auto count_ge = [&](uint32_t thr) {
-    int c = 0;
-    for (int j = threadIdx.x; j < D.n; j += blockDim.x) {
-      const uint32_t u = __float_as_uint(x[j]) & 0x7FFFFFFFu;
-      c += (u >= thr) ? 1 : 0;
-    }
-    c = wave_sum_i(c);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) cnt_s[threadIdx.x >> 6] = c;
-    __syncthreads();
-    int t = 0;
-    for (int w = 0; w < (int)blockDim.x / 64; w++) t += cnt_s[w];
-    return t;
-  };
-  uint32_t thr = 0u;
-  int quota = 0;  // entries equal to thr that may still be taken
-  const bool all_nz = !(topk && count_ge(1u) > D.k);
-  if (!all_nz) {
-    uint32_t t = 0;
-    for (int bit = 30; bit >= 0; bit--) {
-      const uint32_t cand = t | (1u << bit);
-      if (count_ge(cand) >= D.k) t = cand;
-    }
-    thr = t;
-    quota = D.k - count_ge(t + 1u);
+// The refinement's support: the k largest |x_j| (all nonzeros when there are at
+// most k; ties at the k-th magnitude taken in index order), as support bits and
+// an ascending list; x is cut to it.  The k-th magnitude is found by a radix
+// select on the IEEE bits of |x| (monotone for non-negative floats), four digits
+// of 8 bits.  The signal's column of the step operand is cleared: the
+// refinement writes the support's entries only.
+template <bool XL>
+__global__ void __launch_bounds__(MR_VT) mr_ref_supp_kernel(MrhsDesc D, int sel) {
+  __shared__ int hist[256];
+  __shared__ int s_cnt[MAX_WAVES];
+  __shared__ uint32_t xs[XL ? MR_XLDS : 4];
+  const int s = mr_signal(D, sel, blockIdx.x);
+  if (s < 0) return;
+  const int n = D.n, nt = blockDim.x, lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+  const int nw = nt / WAVE;
+  float *x = D.x + (long)s * n;
+  auto mag = [&](int j) { return XL ? xs[j] : (__float_as_uint(x[j]) & 0x7FFFFFFFu); };
+  int c = 0;
+  for (int j = threadIdx.x; j < n; j += nt) {
+    const uint32_t u = __float_as_uint(x[j]) & 0x7FFFFFFFu;
+    if (XL) xs[j] = u;
+    c += u != 0u;
   }
-  if (threadIdx.x == 0) base = 0;
+  c = wave_sum_i(c);
+  if (lane == 0) s_cnt[wave] = c;
+  {
+    uint4 *o = reinterpret_cast<uint4 *>(D.vb + (long)s * n * 2);
+    for (int q = threadIdx.x; q < n / 8; q += nt) o[q] = make_uint4(0u, 0u, 0u, 0u);
+  }
   __syncthreads();
-  int eq_taken = 0;
-  for (int j0 = 0; j0 < D.n; j0 += blockDim.x) {
-    const int j = j0 + threadIdx.x;
-    const uint32_t u = j < D.n ? (__float_as_uint(x[j]) & 0x7FFFFFFFu) : 0u;
-    const int eq = (!all_nz && j < D.n && u == thr) ? 1 : 0;
-    int eq_tot;
-    const int eq_pos = wg_exclusive_scan(eq, &eq_tot);
-    const int in = j < D.n && (all_nz ? (u != 0u) : ((u > thr) || (eq && eq_taken + eq_pos < quota)));
-    eq_taken += eq_tot;
-    if (j < D.n && topk) {
-      mask[j] = in;
-      if (!in) x[j] = 0.f;
+  int nnz = 0;
+  for (int w = 0; w < nw; w++) nnz += s_cnt[w];
+  uint32_t thr = 0u;
+  int quota = 0;  // entries equal to thr that are taken (thr = 0: none)
+  if (nnz > D.k) {
+    quota = D.k;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+      for (int d = threadIdx.x; d < 256; d += nt) hist[d] = 0;
+      __syncthreads();
+      const uint32_t above = shift == 24 ? 0u : thr >> (shift + 8);
+      for (int j = threadIdx.x; j < n; j += nt) {
+        const uint32_t u = mag(j);
+        if (shift == 24 || (u >> (shift + 8)) == above) atomicAdd(&hist[(u >> shift) & 255u], 1);
+      }
+      __syncthreads();
+      // digits from the largest down, four per lane, by every wave for itself
+      int h[4], t = 0;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        h[e] = hist[255 - (4 * lane + e)];
+        t += h[e];
+      }
+      const int incl = wscan_i(t);
+      const int l = __ffsll((unsigned long long)__ballot(incl >= quota)) - 1;
+      int need = quota - (incl - t), d = 255 - 4 * lane;
+#pragma unroll
+      for (int e = 0; e < 3; e++)
+        if (need > h[e]) {
+          need -= h[e];
+          d--;
+        } else {
+          break;
+        }
+      thr |= (uint32_t)__builtin_amdgcn_readlane(d, l) << shift;
+      quota = __builtin_amdgcn_readlane(need, l);
+      __syncthreads();
     }
-    int tot;
-    const int pos = wg_exclusive_scan(in, &tot);
-    if (in) sup[base + pos] = j;
-    __syncthreads();
-    if (threadIdx.x == 0) base += tot;
-    __syncthreads();
+  }
+  unsigned long long *gt = D.mask2 + (long)s * D.words, *eq = D.mask3 + (long)s * D.words;
+  for (int j = threadIdx.x; j < n; j += nt) {
+    const uint32_t u = mag(j);
+    const unsigned long long bg = __ballot(u > thr), be = __ballot(u == thr && quota > 0);
+    if (lane == 0) {
+      gt[j >> 6] = bg;
+      eq[j >> 6] = be;
+    }
+  }
+  __syncthreads();
+  unsigned long long *mask = D.mask + (long)s * D.words;
+  int *sup = D.supp + (long)s * n;
+  int base = 0, eq_base = 0;
+  for (int b = 0; b < D.words; b += WAVE) {
+    unsigned long long m = 0ull, e = 0ull;
+    if (b + lane < D.words) {
+      m = gt[b + lane];
+      e = eq[b + lane];
+    }
+    const int ce = __popcll(e);
+    const int pre = eq_base + wscan_i(ce) - ce;  // equal entries before this word
+    for (int over = ce - max(0, min(ce, quota - pre)); over > 0; over--)
+      e &= ~(1ull << (63 - __clzll(e)));  // the last ones are beyond the quota
+    m |= e;
+    const int cm = __popcll(m), incl = wscan_i(cm);
+    for (int w = wave; w < WAVE && b + w < D.words; w += nw) {
+      const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)m, w);
+      const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(m >> 32), w);
+      const unsigned long long mw = ((unsigned long long)hi << 32) | lo;
+      const int at = base + __builtin_amdgcn_readlane(incl, w) - __popcll(mw);
+      const int j = 64 * (b + w) + lane;
+      if ((mw >> lane) & 1ull)
+        sup[at + __popcll(mw & ((1ull << lane) - 1ull))] = j;
+      else if (mag(j) != 0u)
+        x[j] = 0.f;
+      if (lane == 0) mask[b + w] = mw;
+    }
+    base += __builtin_amdgcn_readlane(incl, 63);
+    eq_base += __builtin_amdgcn_readlane(wscan_i(ce), 63);
   }
   if (threadIdx.x == 0) D.supp_cnt[s] = base;
 }
 
 // r = y - A_S x_S from the FP32 A with FP64 sums over the support list of
-// each selected signal.  Pass 1: one workgroup per (slice z of MR_SLICES,
+// each selected signal.  Pass 1: one workgroup per (slice z of `slices`,
 // signal) streams whole columns (contiguous m floats): support chunks z,
-// z + MR_SLICES, ... of MR_CHUNK entries are staged through LDS, and each
+// z + slices, ... of MR_CHUNK entries are staged through LDS, and each
 // thread owns rows 4t + 1024q (float4 loads), keeping FP64 row sums in
-// registers; the slice's sums go to rowpart.  Pass 2 (mr_resid_sum_kernel):
-// slices summed in order, r and the FP64 partial of ||r||^2 of each 256-row
-// block (part[s * nblk + block]).  Needs m <= 1024 * MR_MAXQ.
+// registers; the slice's sums go to rowpart.  The next column's loads are issued
+// before this one's products (NQ float4 per thread and column; NQ = 4 for m <=
+// 4096 leaves room for both).  Pass 2 (mr_resid_sum_kernel): slices summed in
+// order, r (FP32, and BF16 as the next A^T operand) and the FP64 partial of
+// ||r||^2 of each 256-row block (part[s * nblk + block]).  Needs m <= 1024 *
+// MR_MAXQ.
 constexpr int MR_SLICES = 64;
 constexpr int MR_CHUNK = 16;
 constexpr int MR_MAXQ = 8;
+template <int NQ>
 __global__ void __launch_bounds__(MR_THREADS) mr_exact_resid_kernel(MrhsDesc D, double *rowpart,
-                                                                    int sel) {
+                                                                    int slices, int sel) {
   __shared__ int sj[MR_CHUNK];
   __shared__ float sv[MR_CHUNK];
-  const int z = blockIdx.x, s = blockIdx.y;
-  if (sel && D.stage[s] != 0) return;
-  const int slices = MR_SLICES;
+  const int z = blockIdx.x, s = mr_signal(D, sel, blockIdx.y);
+  if (s < 0) return;
   const long n = D.n, m = D.m;
   const int cnt = D.supp_cnt[s];
   if (z * MR_CHUNK >= cnt) return;
   const float *x = D.x + s * n;
   const int *sup = D.supp + s * n;
-  const int nq = (D.m + 4 * MR_THREADS - 1) / (4 * MR_THREADS);
-  double acc[MR_MAXQ][4];
+  double acc[NQ][4];
 #pragma unroll
-  for (int q = 0; q < MR_MAXQ; q++)
+  for (int q = 0; q < NQ; q++)
 #pragma unroll
     for (int e = 0; e < 4; e++) acc[q][e] = 0.0;
+  auto load = [&](int c, float4 (&v)[NQ]) {
+    const float *col = D.A32 + (long)sj[c] * m;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const int i = 4 * (int)threadIdx.x + 4 * MR_THREADS * q;
+      v[q] = i < D.m ? *(const float4 *)(col + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  auto add = [&](const float4 (&v)[NQ], float x1) {
+    const double xv = (double)x1;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      acc[q][0] = fma((double)v[q].x, xv, acc[q][0]);
+      acc[q][1] = fma((double)v[q].y, xv, acc[q][1]);
+      acc[q][2] = fma((double)v[q].z, xv, acc[q][2]);
+      acc[q][3] = fma((double)v[q].w, xv, acc[q][3]);
+    }
+  };
   for (int c0 = z * MR_CHUNK; c0 < cnt; c0 += slices * MR_CHUNK) {
     __syncthreads();
     if (threadIdx.x < MR_CHUNK && c0 + (int)threadIdx.x < cnt) {
@@ -591,46 +792,35 @@ __global__ void __launch_bounds__(MR_THREADS) mr_exact_resid_kernel(MrhsDesc D, 
     }
     __syncthreads();
     const int c1 = min(MR_CHUNK, cnt - c0);
-    for (int c = 0; c < c1; c++) {
-      const float *col = D.A32 + (long)sj[c] * m;
-      const double xv = (double)sv[c];
-      float4 v[MR_MAXQ];
-#pragma unroll
-      for (int q = 0; q < MR_MAXQ; q++) {
-        const int i = 4 * (int)threadIdx.x + 4 * MR_THREADS * q;
-        if (q < nq && i < D.m) v[q] = *(const float4 *)(col + i);
-      }
-#pragma unroll
-      for (int q = 0; q < MR_MAXQ; q++) {
-        const int i = 4 * (int)threadIdx.x + 4 * MR_THREADS * q;
-        if (q < nq && i < D.m) {
-          acc[q][0] = fma((double)v[q].x, xv, acc[q][0]);
-          acc[q][1] = fma((double)v[q].y, xv, acc[q][1]);
-          acc[q][2] = fma((double)v[q].z, xv, acc[q][2]);
-          acc[q][3] = fma((double)v[q].w, xv, acc[q][3]);
-        }
+    float4 v0[NQ], v1[NQ];
+    load(0, v0);
+    for (int c = 0; c < c1; c += 2) {
+      if (c + 1 < c1) load(c + 1, v1);
+      add(v0, sv[c]);
+      if (c + 1 < c1) {
+        if (c + 2 < c1) load(c + 2, v0);
+        add(v1, sv[c + 1]);
       }
     }
   }
   double *o = rowpart + ((long)s * slices + z) * m;
 #pragma unroll
-  for (int q = 0; q < MR_MAXQ; q++) {
+  for (int q = 0; q < NQ; q++) {
     const int i = 4 * (int)threadIdx.x + 4 * MR_THREADS * q;
-    if (q < nq && i < D.m) {
-      o[i] = acc[q][0];
-      o[i + 1] = acc[q][1];
-      o[i + 2] = acc[q][2];
-      o[i + 3] = acc[q][3];
+    if (i < D.m) {
+      *(double2 *)(o + i) = make_double2(acc[q][0], acc[q][1]);
+      *(double2 *)(o + i + 2) = make_double2(acc[q][2], acc[q][3]);
     }
   }
 }
 
 __global__ void __launch_bounds__(MR_THREADS) mr_resid_sum_kernel(MrhsDesc D,
                                                                   const double *rowpart,
-                                                                  double *part, int sel) {
+                                                                  double *part, int slices,
+                                                                  int sel) {
   __shared__ double red[MR_THREADS / 64];
-  const int s = blockIdx.y, slices = MR_SLICES;
-  if (sel && D.stage[s] != 0) return;
+  const int s = mr_signal(D, sel, blockIdx.y);
+  if (s < 0) return;
   const long m = D.m;
   const int cnt = D.supp_cnt[s];
   const int used = min(slices, (cnt + MR_CHUNK - 1) / MR_CHUNK);  // slices that wrote
@@ -638,9 +828,12 @@ __global__ void __launch_bounds__(MR_THREADS) mr_resid_sum_kernel(MrhsDesc D,
   double e2 = 0.0;
   if (i < D.m) {
     double a = 0.0;
+#pragma unroll 8
     for (int z = 0; z < used; z++) a += rowpart[((long)s * slices + z) * m + i];
     const double ri = (double)D.y[s * m + i] - a;
-    D.resid[s * m + i] = (float)ri;
+    const float rf = (float)ri;
+    D.resid[s * m + i] = rf;
+    reinterpret_cast<uint16_t *>(D.rb)[s * m + i] = f2bf16_rne(rf);
     e2 = ri * ri;
   }
   e2 = wave_sum(e2);
@@ -653,138 +846,141 @@ __global__ void __launch_bounds__(MR_THREADS) mr_resid_sum_kernel(MrhsDesc D,
   }
 }
 
-__device__ __forceinline__ double mr_part_sum(const double *part, int s, int nblk) {
+// ||r||^2 of the selected signals (after the exact residual) into ref; with mark
+// (the support corrections' entry) the signals with ||r|| > tol become active.
+__global__ void __launch_bounds__(MR_THREADS) mr_norm_kernel(MrhsDesc D, const double *part,
+                                                             int nblk, int sel, int mark) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= D.count) return;
+  const int s = mr_signal(D, sel, b);
+  if (s < 0) return;
   double t = 0.0;
-  for (int b = 0; b < nblk; b++) t += part[(long)s * nblk + b];
-  return t;
-}
-
-// Refinement residual (after mr_exact_resid_kernel): ||r||^2 into
-// ref; d = 0; r as the next A^T operand (BF16).
-__global__ void __launch_bounds__(MR_VT) mr_ref_resid_kernel(MrhsDesc D, const double *part,
-                                                                  int nblk, int sel) {
-  const int s = blockIdx.x;
-  if (sel && D.stage[s] != 0) return;
-  const long n = D.n, m = D.m;
-  float *d = D.thres + s * n;
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x) d[j] = 0.f;
-  if (threadIdx.x == 0) D.ref[4 * s + 1] = mr_part_sum(part, s, nblk);
-  __syncthreads();
-  Team t{0, 1, nullptr, 0, nullptr};
-  mr_quant(t, D, D.resid + s * m, nullptr, D.m, D.rb, D.sr, s);
+  for (int q = 0; q < nblk; q++) t += part[(long)s * nblk + q];
+  D.ref[4 * (long)s + 1] = t;
+  if (mark) D.stage[s] = (D.st[s].max_value != 0.f && sqrt(t) > (double)D.tol) ? 0 : 1;
 }
 
 // Support correction on the exact residual (after a refinement, whose final
-// pass left r in resid and its BF16 copy in rb): mr_htp_mark_kernel makes the
-// signals with ||r|| > tol active (stage 0); after g = A^T r over them, g
-// restricted to the current support (bins2) is the operand of the step-size
-// product.
-__global__ void __launch_bounds__(MR_THREADS) mr_htp_mark_kernel(MrhsDesc D) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= D.count) return;
-  const double rn = sqrt(D.ref[4 * s + 1]);
-  D.stage[s] = (D.st[s].max_value != 0.f && rn > (double)D.tol) ? 0 : 1;
-}
+// pass left r's BF16 copy in rb): after g = A^T r over the active signals, g
+// restricted to the current support is the operand of the step-size product.
 __global__ void __launch_bounds__(MR_VT) mr_htp_grad_kernel(MrhsDesc D) {
-  const int s = blockIdx.x;
+  __shared__ WgSlots W;
+  int bank = 0;
+  const int pos = blockIdx.x, s = mr_signal(D, 1, pos);
+  if (s < 0) return;
   const long n = D.n;
-  if (D.stage[s] != 0) return;
-  const float *G = D.g + s * n;
-  const int *mask = D.bins2 + s * n;
-  float *gs = D.grad + s * n;
-  double g2 = 0.0;
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x) {
-    const float v = mask[j] ? G[j] : 0.f;
-    gs[j] = v;
-    g2 += (double)v * (double)v;
+  const int *sup = D.supp + s * n;
+  uint16_t *vb = reinterpret_cast<uint16_t *>(D.vb) + s * n;
+  double g2[1] = {0.0};
+  float nonef[1];
+  for (int c = threadIdx.x; c < D.supp_cnt[s]; c += blockDim.x) {
+    const int j = sup[c];
+    const float v = mr_sum1(D.g, D.st_g, D.ks_g, pos * n + j);
+    vb[j] = f2bf16_rne(v);
+    g2[0] += (double)v * (double)v;
   }
-  Team t{0, 1, nullptr, 0, nullptr};
-  double v[1] = {g2};
-  const int op[1] = {0};
-  team_reduce<double, 1>(t, v, op);
-  if (threadIdx.x == 0) D.ref[4 * s] = v[0];
-  mr_quant(t, D, gs, nullptr, D.n, D.vb1, D.sv1, s);
+  wg_reduce<1, 0>(W, bank, g2, nonef);
+  if (threadIdx.x == 0) D.ref[4 * (long)s] = g2[0];
 }
 
 // x += mu g with the NIHT step mu = ||g_S||^2 / ||A g_S||^2 (active signals);
 // the refinement that follows keeps the k largest entries (hard thresholding
 // pursuit with an exact k-term threshold).
 __global__ void __launch_bounds__(MR_VT) mr_htp_step_kernel(MrhsDesc D) {
-  const int s = blockIdx.x;
-  if (D.stage[s] != 0) return;
+  __shared__ WgSlots W;
+  int bank = 0;
+  const int pos = blockIdx.x, s = mr_signal(D, 1, pos);
+  if (s < 0) return;
   const long n = D.n, m = D.m;
-  const float *w = D.w1 + s * m, *G = D.g + s * n;
   float *x = D.x + s * n;
-  double a2 = 0.0;
-  for (int i = threadIdx.x; i < D.m; i += blockDim.x) a2 += (double)w[i] * (double)w[i];
-  Team t{0, 1, nullptr, 0, nullptr};
-  double v[1] = {a2};
-  const int op[1] = {0};
-  team_reduce<double, 1>(t, v, op);
-  const float mu = v[0] > 0.0 ? (float)(D.ref[4 * s] / v[0]) : 0.f;
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x) x[j] = fmaf(mu, G[j], x[j]);
+  double a2[1] = {0.0};
+  float nonef[1];
+  for (int q = threadIdx.x; q < D.m / 4; q += blockDim.x) {
+    const float4 w = mr_sum4(D.w, D.st_w, D.ks_w, pos * m + 4 * q);
+    a2[0] += (double)w.x * (double)w.x + (double)w.y * (double)w.y + (double)w.z * (double)w.z +
+             (double)w.w * (double)w.w;
+  }
+  wg_reduce<1, 0>(W, bank, a2, nonef);
+  const float mu = a2[0] > 0.0 ? (float)(D.ref[4 * (long)s] / a2[0]) : 0.f;
+  for (int q = threadIdx.x; q < D.n / 4; q += blockDim.x) {
+    const float4 g = mr_sum4(D.g, D.st_g, D.ks_g, pos * n + 4 * q);
+    float4 v = mr_ld4(x, 4 * q);
+    v = make_float4(fmaf(mu, g.x, v.x), fmaf(mu, g.y, v.y), fmaf(mu, g.z, v.z), fmaf(mu, g.w, v.w));
+    *reinterpret_cast<float4 *>(x + 4 * q) = v;
+  }
 }
-
 
 // CG on A_S^T A_S d = A_S^T r, part 1 (after s = A^T r): gamma = ||s_S||^2,
-// p = s_S + beta p (beta = 0 on the first step); p as the next A operand.
-__global__ void __launch_bounds__(MR_VT) mr_ref_dir_kernel(MrhsDesc D, int first, int sel) {
-  const int s = blockIdx.x;
-  if (sel && D.stage[s] != 0) return;
+// p = s_S + beta p (beta = 0 and d = 0 on the first step); p as the next A operand.
+// The CG vectors have one entry per list position.
+__global__ void __launch_bounds__(MR_THREADS) mr_ref_dir_kernel(MrhsDesc D, int first, int sel) {
+  __shared__ WgSlots W;
+  int bank = 0;
+  const int pos = blockIdx.x, s = mr_signal(D, sel, pos);
+  if (s < 0) return;
   const long n = D.n;
-  const float *G = D.g + s * n;
-  const int *mask = D.bins2 + s * n;
-  float *p = D.gprev_thres + s * n, *sg = D.grad + s * n;
-  Team t{0, 1, nullptr, 0, nullptr};
-  double g2 = 0.0;
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x) {
-    const float v = mask[j] ? G[j] : 0.f;
-    sg[j] = v;
-    g2 += (double)v * (double)v;
+  const int cnt = D.supp_cnt[s];
+  const int *sup = D.supp + s * n;
+  float *p = D.cp + (long)s * D.k, *d = D.cd + (long)s * D.k;
+  uint16_t *vb = reinterpret_cast<uint16_t *>(D.vb) + s * n;
+  double g2[1] = {0.0};
+  float nonef[1];
+  for (int c = threadIdx.x; c < cnt; c += blockDim.x) {
+    const float v = mr_sum1(D.g, D.st_g, D.ks_g, pos * n + sup[c]);
+    g2[0] += (double)v * (double)v;
   }
-  double v[1] = {g2};
-  const int op[1] = {0};
-  team_reduce<double, 1>(t, v, op);
-  const double gold = D.ref[4 * s];
-  const float beta = (first || gold == 0.0) ? 0.f : (float)(v[0] / gold);
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x) p[j] = fmaf(beta, first ? 0.f : p[j], sg[j]);
-  __syncthreads();
-  if (threadIdx.x == 0) D.ref[4 * s] = v[0];
-  mr_quant(t, D, p, nullptr, D.n, D.vb1, D.sv1, s);
+  wg_reduce<1, 0>(W, bank, g2, nonef);
+  const double gold = D.ref[4 * (long)s];
+  const float beta = (first || gold == 0.0) ? 0.f : (float)(g2[0] / gold);
+  for (int c = threadIdx.x; c < cnt; c += blockDim.x) {
+    const int j = sup[c];
+    const float v = mr_sum1(D.g, D.st_g, D.ks_g, pos * n + j);
+    const float q = fmaf(beta, first ? 0.f : p[c], v);
+    p[c] = q;
+    if (first) d[c] = 0.f;
+    vb[j] = f2bf16_rne(q);
+  }
+  __syncthreads();  // gamma of the last step has been read
+  if (threadIdx.x == 0) D.ref[4 * (long)s] = g2[0];
 }
 
-// CG part 2 (after q = A p): alpha = gamma / ||q||^2, d += alpha p,
-// r -= alpha q; r as the next A^T operand.
-__global__ void __launch_bounds__(MR_VT) mr_ref_step_kernel(MrhsDesc D, int sel) {
-  const int s = blockIdx.x;
-  if (sel && D.stage[s] != 0) return;
+// CG part 2 (after q = A p): alpha = gamma / ||q||^2, d += alpha p; then r -=
+// alpha q as the next A^T operand, or, on the last step, x_S += d.
+__global__ void __launch_bounds__(MR_THREADS) mr_ref_step_kernel(MrhsDesc D, int last, int sel) {
+  __shared__ WgSlots W;
+  int bank = 0;
+  const int pos = blockIdx.x, s = mr_signal(D, sel, pos);
+  if (s < 0) return;
   const long n = D.n, m = D.m;
-  const float *q = D.w1 + s * m, *p = D.gprev_thres + s * n;
-  float *r = D.resid + s * m, *d = D.thres + s * n;
-  Team t{0, 1, nullptr, 0, nullptr};
-  double q2 = 0.0;
-  for (int i = threadIdx.x; i < D.m; i += blockDim.x) q2 += (double)q[i] * (double)q[i];
-  double v[1] = {q2};
-  const int op[1] = {0};
-  team_reduce<double, 1>(t, v, op);
-  const double gam = D.ref[4 * s];
-  const float alpha = v[0] > 0.0 ? (float)(gam / v[0]) : 0.f;
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x) d[j] = fmaf(alpha, p[j], d[j]);
-  for (int i = threadIdx.x; i < D.m; i += blockDim.x) r[i] = fmaf(-alpha, q[i], r[i]);
-  __syncthreads();
-  mr_quant(t, D, r, nullptr, D.m, D.rb, D.sr, s);
-}
-
-// x_S += d.
-__global__ void __launch_bounds__(MR_VT) mr_ref_update_kernel(MrhsDesc D, int sel) {
-  const int s = blockIdx.x;
-  if (sel && D.stage[s] != 0) return;
-  const long n = D.n;
-  float *x = D.x + s * n;
-  const float *d = D.thres + s * n;
-  const int *mask = D.bins2 + s * n;
-  for (int j = threadIdx.x; j < D.n; j += blockDim.x)
-    if (mask[j]) x[j] = __fadd_rn(x[j], d[j]);
+  const int cnt = D.supp_cnt[s], nt = blockDim.x;
+  const int *sup = D.supp + s * n;
+  const float *p = D.cp + (long)s * D.k;
+  float *r = D.resid + s * m, *d = D.cd + (long)s * D.k, *x = D.x + s * n;
+  double q2[1] = {0.0};
+  float nonef[1];
+  for (int i = threadIdx.x; i < D.m / 4; i += nt) {
+    const float4 q = mr_sum4(D.w, D.st_w, D.ks_w, pos * m + 4 * i);
+    q2[0] += (double)q.x * (double)q.x + (double)q.y * (double)q.y + (double)q.z * (double)q.z +
+             (double)q.w * (double)q.w;
+  }
+  wg_reduce<1, 0>(W, bank, q2, nonef);
+  const double gam = D.ref[4 * (long)s];
+  const float alpha = q2[0] > 0.0 ? (float)(gam / q2[0]) : 0.f;
+  for (int c = threadIdx.x; c < cnt; c += nt) {
+    const float v = fmaf(alpha, p[c], d[c]);
+    d[c] = v;
+    if (last) x[sup[c]] = __fadd_rn(x[sup[c]], v);
+  }
+  if (last) return;
+  uint2 *rb = reinterpret_cast<uint2 *>(D.rb + s * m * 2);
+  for (int i = threadIdx.x; i < D.m / 4; i += nt) {
+    const float4 q = mr_sum4(D.w, D.st_w, D.ks_w, pos * m + 4 * i);
+    float4 v = mr_ld4(r, 4 * i);
+    v = make_float4(fmaf(-alpha, q.x, v.x), fmaf(-alpha, q.y, v.y), fmaf(-alpha, q.z, v.z),
+                    fmaf(-alpha, q.w, v.w));
+    *reinterpret_cast<float4 *>(r + 4 * i) = v;
+    rb[i] = mr_bf4(v);
+  }
 }
 
 // y = A x_true for every signal from the FP32 A, FP64 sums.
@@ -930,44 +1126,83 @@ struct xcs_mrhs {
   }
 };
 
-// One product for the active signals: transpose: G = A^T R (M = n, K = m);
-// else C = A V (M = m, K = n, split over K then summed in split order).
-static int mr_gemm(xcs_mrhs *h, int fmt, bool transpose, const uint8_t *B, float *C,
-                   const float *bscale, const int *ncols, const int *map) {
+// Block tile and number of K slices of one product (M x N, kbytes of K per row):
+// about one workgroup per CU, at least two 128-byte K stages each.  A product
+// whose 256 x 128 tiles fill the chip with at most four slices takes that tile;
+// else the 128 x 128 tile with as many slices as it takes.  The slices are added
+// by the kernel that reads the product, so they cost no pass of their own; they
+// matter for narrow products (few active signals) and small matrices, which
+// leave most of the chip idle unsplit.  Measured on MI355X: BF16 A^T R of 16384 x
+// 4096 with up to 128 columns 61 us unsplit, 24 with its four slices.
+static void mr_gemm_shape(int forced, int M, int N, long kbytes, int *tile, int *ks) {
+  const long stages = kbytes / GT_KB;
+  auto fits = [&](int k) { return stages % k == 0 && stages / k >= 2; };
+  const long t128 = (long)(M / 128) * ((N + 127) / 128);
+  if (M % 256 == 0 && forced != 0) {
+    for (int k = 1; k <= 4; k *= 2)
+      if (fits(k) && gemm_tile(M, N, k)) {
+        *tile = 1;
+        *ks = k;
+        if (forced < 0 || forced == 1) return;
+        break;
+      }
+  }
+  *tile = forced > 0 && M % 256 == 0 ? forced : 0;
+  *ks = 1;
+  while (*ks < MR_KMAX && t128 * *ks < 256 && fits(2 * *ks)) *ks *= 2;
+}
+
+enum { MR_AX = 0, MR_G = 1, MR_W = 2 };
+// One product over `cols` columns at most (the first *ncols of `map`, or all):
+// MR_AX: ax = A x, MR_G: g = A^T r, MR_W: w = A v.
+static int mr_gemm(xcs_mrhs *h, int fmt, int which, int cols, const int *ncols, const int *map) {
   const int esz = fmt == FMT_BF16 ? 2 : 1;
+  MrhsDesc &D = h->D;
+  const bool transpose = which == MR_G;
   GemmArgs g{};
   if (transpose) {
     g.A = fmt == FMT_BF16 ? h->a16cm : h->a8cm;
     g.M = h->n;
     g.K = h->m;
-    g.ldc = h->n;
-    g.ksplit = 1;
+    g.B = D.rb;
+    g.C = D.g;
     g.row_scale = fmt == FMT_FP8 ? h->cs : nullptr;
   } else {
     g.A = fmt == FMT_BF16 ? h->a16rm : h->a8rm;
     g.M = h->m;
     g.K = h->n;
-    g.ldc = h->m;
-    g.ksplit = MR_KSPLIT;
-    g.split_stride = (long)h->count * h->m;
+    g.B = which == MR_AX ? D.xb : D.vb;
+    g.C = which == MR_AX ? D.ax : D.w;
   }
-  g.lda_bytes = (long)g.K * esz;
-  g.B = B;
-  g.ldb_bytes = (long)g.K * esz;
-  g.C = C;
-  g.N = h->count;
+  g.ldc = g.M;
+  g.lda_bytes = g.ldb_bytes = (long)g.K * esz;
+  g.N = cols;
   g.ncols = ncols;
   g.col_map = map;
-  g.col_scale = fmt == FMT_FP8 ? bscale : nullptr;
-  const int tile = g.M % 256 ? 0 : h->gemm_big >= 0 ? h->gemm_big : gemm_tile(g.M, g.N, g.ksplit);
+  g.c_by_pos = 1;
+  g.col_scale = fmt == FMT_FP8 ? (transpose ? D.sr : which == MR_AX ? D.sx : D.sv) : nullptr;
+  int tile;
+  mr_gemm_shape(h->gemm_big, g.M, cols, (long)g.K * esz, &tile, &g.ksplit);
+  g.split_stride = (long)cols * g.M;
+  int &ks = transpose ? D.ks_g : which == MR_AX ? D.ks_ax : D.ks_w;
+  long &st = transpose ? D.st_g : which == MR_AX ? D.st_ax : D.st_w;
+  ks = g.ksplit;
+  st = g.split_stride;
   HIP_TRY(fmt == FMT_BF16 ? gemm_tn_launch<FMT_BF16>(tile, g, h->stream)
                           : gemm_tn_launch<FMT_FP8>(tile, g, h->stream));
-  if (g.ksplit > 1) {
-    hipLaunchKernelGGL(gemm_split_sum_kernel, dim3(2048), dim3(256), 0, h->stream, C, g.ldc,
-                       g.split_stride, g.ksplit, g.M, h->count, ncols, map);
-    HIP_TRY(hipGetLastError());
-  }
   return XCS_OK;
+}
+// Floats a product buffer needs for any number of columns up to `cols`.
+static size_t mr_product_floats(int M, int cols, int K) {
+  size_t most = 0;
+  for (int N = 1; N <= cols; N++)
+    for (int esz = 1; esz <= 2; esz++)
+      for (int forced = -1; forced <= 2; forced++) {
+        int tile, ks;
+        mr_gemm_shape(forced, M, N, (long)K * esz, &tile, &ks);
+        most = std::max(most, (size_t)ks * N * M);
+      }
+  return most;
 }
 
 static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *precision,
@@ -1021,8 +1256,9 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   D.n = n;
   D.k = k;
   D.count = count;
+  D.words = n / 64;
   D.num_bins = o->num_bins > 0 ? o->num_bins : std::max(n / 20, 1000);
-  D.cstride = round_up(D.num_bins + 64, 64);
+  D.cstride = D.num_bins > MR_HIST ? round_up(D.num_bins, 64) : 0;
   D.restart = o->restart;
   D.maxiter = o->maxiter > 0 ? o->maxiter : 5000;
   D.tol = o->tol_reference_default ? (float)(10 ^ (-4)) : o->tol;
@@ -1032,39 +1268,35 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   XCS_TRY(h->alloc(&y, S * m));
   D.y = y;
   XCS_TRY(h->alloc(&D.x, S * n));
-  XCS_TRY(h->alloc(&D.grad, S * n));
-  XCS_TRY(h->alloc(&D.thres, S * n));
   XCS_TRY(h->alloc(&D.gprev, S * n));
-  XCS_TRY(h->alloc(&D.gprev_thres, S * n));
   XCS_TRY(h->alloc(&D.resid, S * m));
-  XCS_TRY(h->alloc(&D.resid_update, S * m));
   XCS_TRY(h->alloc(&D.aux, 4 * S));
   XCS_TRY(h->alloc(&D.tol_lp, S));
-  XCS_TRY(h->alloc(&D.bins, S * n));
-  XCS_TRY(h->alloc(&D.bins2, S * n));
+  XCS_TRY(h->alloc(&D.mask, S * D.words));
+  XCS_TRY(h->alloc(&D.mask2, S * D.words));
+  XCS_TRY(h->alloc(&D.mask3, S * D.words));
   XCS_TRY(h->alloc(&D.counters, S * D.cstride));
   XCS_TRY(h->alloc(&D.stage, S));
   XCS_TRY(h->alloc(&D.mode, S));
+  XCS_TRY(h->alloc(&D.wpos, S));
   XCS_TRY(h->alloc(&D.st, S));
   XCS_TRY(h->alloc(&D.xb, 2 * S * n));
-  XCS_TRY(h->alloc(&D.vb1, 2 * S * n));
-  XCS_TRY(h->alloc(&D.vb2, 2 * S * n));
+  XCS_TRY(h->alloc(&D.vb, 4 * S * n));
   XCS_TRY(h->alloc(&D.rb, 2 * S * m));
   XCS_TRY(h->alloc(&D.sx, S));
   XCS_TRY(h->alloc(&D.sr, S));
-  XCS_TRY(h->alloc(&D.sv1, S));
-  XCS_TRY(h->alloc(&D.sv2, S));
-  XCS_TRY(h->alloc(&D.ax, MR_KSPLIT * S * m));
-  XCS_TRY(h->alloc(&D.w1, MR_KSPLIT * S * m));
-  XCS_TRY(h->alloc(&D.w2, MR_KSPLIT * S * m));
-  XCS_TRY(h->alloc(&D.g, S * n));
+  XCS_TRY(h->alloc(&D.sv, 2 * S));
+  XCS_TRY(h->alloc(&D.ax, mr_product_floats(m, count, n)));
+  XCS_TRY(h->alloc(&D.w, mr_product_floats(m, 2 * count, n)));
+  XCS_TRY(h->alloc(&D.g, mr_product_floats(n, count, m)));
   XCS_TRY(h->alloc(&D.active, S));
-  XCS_TRY(h->alloc(&D.ulist, S));
+  XCS_TRY(h->alloc(&D.wlist, 2 * S));
   XCS_TRY(h->alloc(&D.nactive, 64));
-  XCS_TRY(h->alloc(&D.nu, 64));
   XCS_TRY(h->alloc(&D.ref, 4 * S));
   XCS_TRY(h->alloc(&D.supp, S * n));
   XCS_TRY(h->alloc(&D.supp_cnt, S));
+  XCS_TRY(h->alloc(&D.cp, S * k));
+  XCS_TRY(h->alloc(&D.cd, S * k));
   h->nblk = (m + MR_THREADS - 1) / MR_THREADS;
   XCS_TRY(h->alloc(&h->part, S * h->nblk));
   XCS_TRY(h->alloc(&h->rowpart, S * MR_SLICES * m));
@@ -1110,29 +1342,56 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   return XCS_OK;
 }
 
+// Workgroups a per-signal kernel needs: the signals known to be active (sel) or
+// all; the active signals only ever get fewer within a phase.
+static dim3 mr_grid(const xcs_mrhs *h, int sel) { return dim3(sel ? *h->h_nactive : h->count); }
+
 static int mr_exact_resid(xcs_mrhs *h, int sel) {
-  hipLaunchKernelGGL(mr_exact_resid_kernel, dim3(MR_SLICES, h->count), dim3(MR_THREADS), 0,
-                     h->stream, h->D, h->rowpart, sel);
-  hipLaunchKernelGGL(mr_resid_sum_kernel, dim3(h->nblk, h->count), dim3(MR_THREADS), 0, h->stream,
-                     h->D, h->rowpart, h->part, sel);
+  // Slices per signal: every slice's row sums go through memory (m doubles written
+  // and read), so as few as still give about 16 workgroups per CU; a few signals
+  // take all MR_SLICES.  512 signals, k = 400, m = 4096: 8 slices 471 us and 28 for
+  // their sum, where 25 slices of one chunk each moved 840 MB of row sums (and the
+  // single-buffered loads took 600 us).
+  const int cols = (int)mr_grid(h, sel).x;
+  int slices = MR_SLICES;
+  while (slices > 4 && (long)slices * cols > 4096) slices /= 2;
+  const dim3 g(slices, cols);
+  if (h->m <= 4 * 4 * MR_THREADS)
+    hipLaunchKernelGGL(mr_exact_resid_kernel<4>, g, dim3(MR_THREADS), 0, h->stream, h->D,
+                       h->rowpart, slices, sel);
+  else
+    hipLaunchKernelGGL(mr_exact_resid_kernel<MR_MAXQ>, g, dim3(MR_THREADS), 0, h->stream, h->D,
+                       h->rowpart, slices, sel);
+  hipLaunchKernelGGL(mr_resid_sum_kernel, dim3(h->nblk, cols), dim3(MR_THREADS), 0, h->stream, h->D,
+                     h->rowpart, h->part, slices, sel);
   HIP_TRY(hipGetLastError());
   return XCS_OK;
 }
 
-// One lock-step CGIHT iteration over the active signals (format D.fmt).
+// One lock-step CGIHT iteration over the active signals (format D.fmt); ends
+// with the lists for the next one.
 static int mr_iteration(xcs_mrhs *h) {
   MrhsDesc &D = h->D;
-  const int f = D.fmt;
-  const dim3 gs(h->count), bs(MR_VT);
-  hipLaunchKernelGGL(mr_list_kernel, dim3(1), dim3(MR_THREADS), 0, h->stream, D);
-  XCS_TRY(mr_gemm(h, f, false, D.xb, D.ax, D.sx, D.nactive, D.active));
+  const int f = D.fmt, na = *h->h_nactive;
+  const dim3 gs(na), bs(MR_VT);
+  XCS_TRY(mr_gemm(h, f, MR_AX, na, D.nactive, D.active));
   hipLaunchKernelGGL(mr_k1_kernel, gs, bs, 0, h->stream, D);
-  XCS_TRY(mr_gemm(h, f, true, D.rb, D.g, D.sr, D.nactive, D.active));
+  XCS_TRY(mr_gemm(h, f, MR_G, na, D.nactive, D.active));
   hipLaunchKernelGGL(mr_k2_kernel, gs, bs, 0, h->stream, D);
-  XCS_TRY(mr_gemm(h, f, false, D.vb1, D.w1, D.sv1, D.nactive, D.active));
-  XCS_TRY(mr_gemm(h, f, false, D.vb2, D.w2, D.sv2, D.nu, D.ulist));
-  hipLaunchKernelGGL(mr_k3_kernel, gs, bs, 0, h->stream, D);
+  XCS_TRY(mr_gemm(h, f, MR_W, 2 * na, D.nactive + 1, D.wlist));
+  if (D.n <= MR_XLDS)
+    hipLaunchKernelGGL(mr_k3_kernel<true>, gs, bs, 0, h->stream, D);
+  else
+    hipLaunchKernelGGL(mr_k3_kernel<false>, gs, bs, 0, h->stream, D);
+  hipLaunchKernelGGL(mr_list_kernel, dim3(1), dim3(MR_THREADS), 0, h->stream, D);
   HIP_TRY(hipGetLastError());
+  return XCS_OK;
+}
+
+// The number of active signals into h_nactive (the lists are up to date).
+static int mr_count_active(xcs_mrhs *h) {
+  HIP_TRY(hipMemcpyAsync(h->h_nactive, h->D.nactive, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
   return XCS_OK;
 }
 
@@ -1142,10 +1401,10 @@ static int mr_phase(xcs_mrhs *h, int *issued) {
   MrhsDesc &D = h->D;
   int it = 0;
   const int cap = D.maxiter + 2;
+  hipLaunchKernelGGL(mr_list_kernel, dim3(1), dim3(MR_THREADS), 0, h->stream, D);
+  HIP_TRY(hipGetLastError());
   while (it < cap) {
-    hipLaunchKernelGGL(mr_list_kernel, dim3(1), dim3(MR_THREADS), 0, h->stream, D);
-    HIP_TRY(hipMemcpyAsync(h->h_nactive, D.nactive, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    XCS_TRY(mr_count_active(h));
     if (*h->h_nactive == 0) break;
     for (int q = 0; q < 4 && it < cap; q++, it++) XCS_TRY(mr_iteration(h));
   }
@@ -1154,32 +1413,31 @@ static int mr_phase(xcs_mrhs *h, int *issued) {
 }
 
 // sel = 0: every signal; sel = 1: the active signals only (stage 0, listed in
-// D.active).  Signals are independent, and each column of a GEMM is the same
-// K-ordered sum whichever columns share its tile, so a selected signal gets
-// the same bits either way.
-static int mr_refine(xcs_mrhs *h, int sel) {
+// D.active).  mark: afterwards the signals above tol are the active ones.
+static int mr_refine(xcs_mrhs *h, int sel, int mark) {
   MrhsDesc &D = h->D;
   D.fmt = FMT_BF16;
-  const dim3 gs(h->count), bs(MR_VT);
+  const dim3 gs = mr_grid(h, sel);
+  const int cols = (int)gs.x;
   const int *nc = sel ? D.nactive : nullptr, *map = sel ? D.active : nullptr;
-  hipLaunchKernelGGL(mr_ref_supp_kernel, gs, bs, 0, h->stream, D, 1, sel);
+  if (D.n <= MR_XLDS)
+    hipLaunchKernelGGL(mr_ref_supp_kernel<true>, gs, dim3(MR_VT), 0, h->stream, D, sel);
+  else
+    hipLaunchKernelGGL(mr_ref_supp_kernel<false>, gs, dim3(MR_VT), 0, h->stream, D, sel);
   for (int o = 0; o < h->ref_outer; o++) {
     XCS_TRY(mr_exact_resid(h, sel));
-    hipLaunchKernelGGL(mr_ref_resid_kernel, gs, bs, 0, h->stream, D, h->part, h->nblk, sel);
-    XCS_TRY(mr_gemm(h, FMT_BF16, true, D.rb, D.g, nullptr, nc, map));
-    hipLaunchKernelGGL(mr_ref_dir_kernel, gs, bs, 0, h->stream, D, 1, sel);
     for (int j = 0; j < h->ref_inner; j++) {
-      XCS_TRY(mr_gemm(h, FMT_BF16, false, D.vb1, D.w1, nullptr, nc, map));
-      hipLaunchKernelGGL(mr_ref_step_kernel, gs, bs, 0, h->stream, D, sel);
-      if (j + 1 == h->ref_inner) break;
-      XCS_TRY(mr_gemm(h, FMT_BF16, true, D.rb, D.g, nullptr, nc, map));
-      hipLaunchKernelGGL(mr_ref_dir_kernel, gs, bs, 0, h->stream, D, 0, sel);
+      XCS_TRY(mr_gemm(h, FMT_BF16, MR_G, cols, nc, map));
+      hipLaunchKernelGGL(mr_ref_dir_kernel, gs, dim3(MR_THREADS), 0, h->stream, D, j == 0 ? 1 : 0, sel);
+      XCS_TRY(mr_gemm(h, FMT_BF16, MR_W, cols, nc, map));
+      hipLaunchKernelGGL(mr_ref_step_kernel, gs, dim3(MR_THREADS), 0, h->stream, D,
+                         j + 1 == h->ref_inner ? 1 : 0, sel);
     }
-    hipLaunchKernelGGL(mr_ref_update_kernel, gs, bs, 0, h->stream, D, sel);
   }
   // final FP64 residual
   XCS_TRY(mr_exact_resid(h, sel));
-  hipLaunchKernelGGL(mr_ref_resid_kernel, gs, bs, 0, h->stream, D, h->part, h->nblk, sel);
+  hipLaunchKernelGGL(mr_norm_kernel, dim3((cols + MR_THREADS - 1) / MR_THREADS), dim3(MR_THREADS),
+                     0, h->stream, D, h->part, h->nblk, sel, mark);
   HIP_TRY(hipGetLastError());
   return XCS_OK;
 }
@@ -1193,11 +1451,14 @@ static int mr_solve(xcs_mrhs *h, float *ms) {
   D.fmt = h->prec;
   const float c_lp = h->prec == FMT_FP8 ? h->c8 : h->c16;
   hipLaunchKernelGGL(mr_init0_kernel, gs, bs, 0, h->stream, D);
-  XCS_TRY(mr_gemm(h, D.fmt, true, D.rb, D.g, D.sr, nullptr, nullptr));
-  hipLaunchKernelGGL(mr_init1_kernel, gs, bs, 0, h->stream, D, c_lp);
-  XCS_TRY(mr_gemm(h, D.fmt, false, D.xb, D.ax, D.sx, nullptr, nullptr));
+  XCS_TRY(mr_gemm(h, D.fmt, MR_G, h->count, nullptr, nullptr));
+  if (D.n <= MR_XLDS)
+    hipLaunchKernelGGL(mr_init1_kernel<true>, gs, bs, 0, h->stream, D, c_lp);
+  else
+    hipLaunchKernelGGL(mr_init1_kernel<false>, gs, bs, 0, h->stream, D, c_lp);
+  XCS_TRY(mr_gemm(h, D.fmt, MR_AX, h->count, nullptr, nullptr));
   hipLaunchKernelGGL(mr_init2_kernel, gs, bs, 0, h->stream, D);
-  XCS_TRY(mr_gemm(h, D.fmt, true, D.rb, D.g, D.sr, nullptr, nullptr));
+  XCS_TRY(mr_gemm(h, D.fmt, MR_G, h->count, nullptr, nullptr));
   hipLaunchKernelGGL(mr_init3_kernel, gs, bs, 0, h->stream, D);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(ev[1], h->stream));
@@ -1211,24 +1472,23 @@ static int mr_solve(xcs_mrhs *h, float *ms) {
     XCS_TRY(mr_phase(h, &h->lp_iters[1]));
   }
   HIP_TRY(hipEventRecord(ev[3], h->stream));
-  XCS_TRY(mr_refine(h, 0));
+  XCS_TRY(mr_refine(h, 0, 1));
   HIP_TRY(hipEventRecord(ev[4], h->stream));
   // signals above tol after the refinement: support corrections on the
   // exact residual, each followed by the refinement
   D.fmt = FMT_BF16;
   for (int c = 0; c < h->polish_max; c++) {
-    hipLaunchKernelGGL(mr_htp_mark_kernel, dim3((h->count + MR_THREADS - 1) / MR_THREADS),
-                       dim3(MR_THREADS), 0, h->stream, D);
     hipLaunchKernelGGL(mr_list_kernel, dim3(1), dim3(MR_THREADS), 0, h->stream, D);
-    HIP_TRY(hipMemcpyAsync(h->h_nactive, D.nactive, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    if (*h->h_nactive == 0) break;
-    XCS_TRY(mr_gemm(h, FMT_BF16, true, D.rb, D.g, nullptr, D.nactive, D.active));
-    hipLaunchKernelGGL(mr_htp_grad_kernel, gs, bs, 0, h->stream, D);
-    XCS_TRY(mr_gemm(h, FMT_BF16, false, D.vb1, D.w1, nullptr, D.nactive, D.active));
-    hipLaunchKernelGGL(mr_htp_step_kernel, gs, bs, 0, h->stream, D);
     HIP_TRY(hipGetLastError());
-    XCS_TRY(mr_refine(h, 1));
+    XCS_TRY(mr_count_active(h));
+    const int na = *h->h_nactive;
+    if (na == 0) break;
+    XCS_TRY(mr_gemm(h, FMT_BF16, MR_G, na, D.nactive, D.active));
+    hipLaunchKernelGGL(mr_htp_grad_kernel, dim3(na), bs, 0, h->stream, D);
+    XCS_TRY(mr_gemm(h, FMT_BF16, MR_W, na, D.nactive, D.active));
+    hipLaunchKernelGGL(mr_htp_step_kernel, dim3(na), bs, 0, h->stream, D);
+    HIP_TRY(hipGetLastError());
+    XCS_TRY(mr_refine(h, 1, 1));
     h->lp_iters[2]++;
   }
   HIP_TRY(hipEventRecord(ev[5], h->stream));
@@ -1305,17 +1565,27 @@ int xcs_mrhs_gemm_timed(xcs_mrhs *h, int transpose, const char *fmt, int reps, f
   if (f == FMT_FP8 && !h->a8cm) return set_err(XCS_EINVAL, "fp8 copies exist only for fp8 handles");
   HIP_TRY(hipSetDevice(h->dev));
   MrhsDesc &D = h->D;
-  const uint8_t *B = transpose ? D.rb : D.vb1;
-  float *C = transpose ? D.g : D.w1;
-  float *bs = transpose ? D.sr : D.sv1;
   std::vector<float> ones((size_t)h->count, 1.0f);
-  HIP_TRY(h2d(bs, ones.data(), 4 * ones.size(), nullptr));
-  XCS_TRY(mr_gemm(h, f, transpose != 0, B, C, bs, nullptr, nullptr));
+  HIP_TRY(h2d(transpose ? D.sr : D.sv, ones.data(), 4 * ones.size(), nullptr));
+  // the product and, where its K is split, the slices' sum (in a solve the kernel
+  // that uses the product adds them)
+  auto product = [&]() -> int {
+    XCS_TRY(mr_gemm(h, f, transpose ? MR_G : MR_W, h->count, nullptr, nullptr));
+    const int ks = transpose ? D.ks_g : D.ks_w, M = transpose ? h->n : h->m;
+    if (ks > 1) {
+      hipLaunchKernelGGL(gemm_split_sum_kernel, dim3(2048), dim3(256), 0, h->stream,
+                         transpose ? D.g : D.w, (long)M, transpose ? D.st_g : D.st_w, ks, M,
+                         h->count, (const int *)nullptr, (const int *)nullptr);
+      HIP_TRY(hipGetLastError());
+    }
+    return XCS_OK;
+  };
+  XCS_TRY(product());
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   HIP_TRY(hipEventRecord(e0, h->stream));
-  for (int r = 0; r < reps; r++) XCS_TRY(mr_gemm(h, f, transpose != 0, B, C, bs, nullptr, nullptr));
+  for (int r = 0; r < reps; r++) XCS_TRY(product());
   HIP_TRY(hipEventRecord(e1, h->stream));
   HIP_TRY(hipEventSynchronize(e1));
   float ms = 0.f;

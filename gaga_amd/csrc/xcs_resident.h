@@ -130,7 +130,7 @@ __device__ __forceinline__ int wscan_i(int v) {
 // __syncthreads: consecutive calls alternate between two banks of LDS slots,
 // and a bank is written again only after the barrier of the call between.
 struct WgSlots {
-  double d[2][2][MAX_WAVES];
+  double d[2][3][MAX_WAVES];
   float m[2][2][MAX_WAVES];
 };
 template <int ND, int NM>
