@@ -334,8 +334,8 @@ class Plan:
         it = ctypes.c_int(0)
         rate = ctypes.c_float(0)
         reason = ctypes.c_int(0)
-        x = np.zeros(self.n, np.float32)
-        xt = np.zeros(self.n, np.float32)
+        x = np.empty(self.n, np.float32)  # both filled by the call
+        xt = np.empty(self.n, np.float32)
         _ck(load().xcs_plan_results(self._h, _p(norms), ctypes.byref(it), _p(sup),
                                     ctypes.byref(rate), ctypes.byref(reason), _p(x), _p(xt)))
         return dict(norms=norms, iters=it.value, support=sup, conv_rate=rate.value,
@@ -447,8 +447,8 @@ class Batch:
         return dict(norms=norms, iters=it, stop_reason=reason, conv_rate=rate)
 
     def x(self, i):
-        x = np.zeros(int(self.n[i]), np.float32)
-        xt = np.zeros(int(self.n[i]), np.float32)
+        x = np.empty(int(self.n[i]), np.float32)  # both filled by the call
+        xt = np.empty(int(self.n[i]), np.float32)
         _ck(load().xcs_batch_x(self._h, i, _p(x), _p(xt)))
         return x, xt
 
@@ -568,9 +568,9 @@ class ManyRHS:
         return dict(norms=norms, iters=it, resid_rel=rr)
 
     def x(self, s):
-        x = np.zeros(self.n, np.float32)
-        xt = np.zeros(self.n, np.float32)
-        y = np.zeros(self.m, np.float32)
+        x = np.empty(self.n, np.float32)  # all filled by the call
+        xt = np.empty(self.n, np.float32)
+        y = np.empty(self.m, np.float32)
         _ck(load().xcs_mrhs_x(self._h, int(s), _p(x), _p(xt), _p(y)))
         return x, xt, y
 
@@ -647,7 +647,7 @@ class MLP:
     def grad(self, X, labels, pos_w=1.0):
         X = np.ascontiguousarray(X, np.float32)
         labels = np.ascontiguousarray(labels, np.float32)
-        g = np.zeros(self.nparams, np.float32)
+        g = np.empty(self.nparams, np.float32)  # filled by the call
         loss = ctypes.c_float(0)
         _ck(load().xcs_mlp_grad(self._h, _p(X), _p(labels), len(labels), float(pos_w), _p(g),
                                 ctypes.byref(loss)))

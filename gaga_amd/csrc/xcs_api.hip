@@ -175,6 +175,8 @@ static int set_err(int code, const char *fmt, ...) {
     if (r_ != XCS_OK) return r_; \
   } while (0)
 
+#include "xcs_host.h"
+
 // ----------------------------------------------------------------- kernels --
 // One instance, the whole (cooperatively launched) grid is its team.
 // The descriptor is copied to LDS: its fields then cannot alias the global
@@ -524,9 +526,29 @@ static const char *const SMV_FAIL =
     "smv generation: a column needed more than 2^20 draws (p too close to m)";
 
 // ------------------------------------------------------------------- plans --
+// Everything a solve starts from, in one launch: the descriptor, x = 0, a fresh
+// state and cleared barrier words (a copy and three fills before: 4 of the
+// runtime's calls, each with a launch of its own behind it).
+__global__ void plan_reset_kernel(XProblem P, XProblem *d, unsigned *bar) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  if (t == 0) *d = P;
+  for (int i = t; i < P.n; i += stride) P.x[i] = 0.f;
+  int *st = (int *)(XState *)P.st;
+  for (int i = t; i < (int)(sizeof(XState) / sizeof(int)); i += stride) st[i] = 0;
+  for (int i = t; i < BAR_WORDS; i += stride) bar[i] = 0u;
+}
+
+// Device memory of a plan: its vectors come out of one block (one allocation,
+// one fill) as long as they fit, the rest one by one.  A given-problem call of
+// 256 x 1024 made 23 allocations and as many fills, 0.2 ms of its 0.65.
+constexpr size_t PLAN_SLAB_MAX = (size_t)16 << 20;
+
 struct xcs_plan {
   int dev = 0;
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr;  // the lane's
+  HostLane lane;
+  char *slab = nullptr;
+  size_t slab_left = 0;
   XProblem h{};         // host copy (device pointers)
   XProblem *d = nullptr;
   int team = 1, block = 256, mode = 0;
@@ -542,16 +564,39 @@ struct xcs_plan {
   float *warm_g = nullptr;  // learned warm start: A^T y and the starting support
   int *warm_mask = nullptr;
   float *warm_score = nullptr;
+  float *xt_dev = nullptr;  // the planted vector, where the plan was generated
   ~xcs_plan() {
     // nothing of this plan may still run on memory that is about to be freed
     if (stream) (void)hipStreamSynchronize(stream);
     for (void *p : allocs) (void)hipFree(p);
-    if (stream) (void)hipStreamDestroy(stream);
+    lane_put(&lane);
+  }
+  // The device is current: the plan's stream, events and staging memory.
+  int open() {
+    HIP_TRY(hipGetDevice(&dev));
+    XCS_TRY(lane_get(&lane));
+    stream = lane.stream;
+    return XCS_OK;
+  }
+  // One cleared block for the allocations that follow.
+  int reserve(size_t bytes) {
+    if (bytes > PLAN_SLAB_MAX) return XCS_OK;
+    char *q = nullptr;
+    XCS_TRY(alloc(&q, bytes));
+    slab = q;
+    slab_left = bytes;
+    return XCS_OK;
   }
   template <class T>
   int alloc(T **p, size_t count) {
     void *q = nullptr;
-    const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+    const size_t bytes = std::max<size_t>(count, 1) * sizeof(T), need = (bytes + 255) / 256 * 256;
+    if (need <= slab_left) {
+      *p = (T *)slab;
+      slab += need;
+      slab_left -= need;
+      return XCS_OK;
+    }
     hipError_t e = dev_malloc(&q, bytes);
     if (e != hipSuccess)
       return set_err(XCS_ENOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
@@ -764,6 +809,13 @@ static int plan_alloc(xcs_plan *pl, int alg, int ens, int k, int m, int n, int p
   // found; it stays off until it is.
   if (alg == ALG_CSMPSP) return set_err(XCS_EINVAL, CSMPSP_OFF);
   const size_t nn = (size_t)n, ml = (size_t)P.lda;
+  // the allocations below and those that a generated or given problem adds (y, the
+  // rows of a dct, a planted vector); the matrices have blocks of their own
+  const size_t words = 9 * nn + (ens == ENS_DCT ? 7 * nn + ml : 0) + 6 * ml +
+                       (ens == ENS_GEN ? 2 * (size_t)MAXCH * ml : 0) + P.num_bins + pl->team +
+                       (P.timing ? 10 : 2) * ((size_t)P.maxiter + 2) +
+                       4 * (size_t)RED_SLOTS * (pl->team + 1) + BAR_WORDS + std::max(k, 1);
+  XCS_TRY(pl->reserve(4 * words + 32 * 256 + sizeof(XState) + sizeof(XProblem) + 1024));
   XCS_TRY(pl->alloc(&P.x, nn));
   XCS_TRY(pl->alloc(&P.thres, nn));
   XCS_TRY(pl->alloc(&P.grad, nn));
@@ -886,12 +938,8 @@ static int plan_generate(xcs_plan *pl, int alg, int ens, int k, int m, int n, in
   XCS_TRY(validate(alg, ens, k, m, n));
   if (k > n) return set_err(XCS_EINVAL, "k must be <= n");
   XCS_TRY(use_device(o->gpu_number));
-  HIP_TRY(hipGetDevice(&pl->dev));
-  HIP_TRY(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking));
-  hipEvent_t e0, e1;
-  HIP_TRY(hipEventCreate(&e0));
-  HIP_TRY(hipEventCreate(&e1));
-  HIP_TRY(hipEventRecord(e0, pl->stream));
+  XCS_TRY(pl->open());
+  HIP_TRY(hipEventRecord(pl->lane.e0, pl->stream));
   const uint32_t seed = o->seed, inst = o->instance;
   int *smv_tmp = nullptr;
   int nz = 0;
@@ -956,11 +1004,10 @@ static int plan_generate(xcs_plan *pl, int alg, int ens, int k, int m, int n, in
   XCS_TRY(plan_make_y(pl, d_supp, k, d_xt, y));
   pl->x_true.resize((size_t)n);
   HIP_TRY(d2h(pl->x_true.data(), d_xt, sizeof(float) * n, nullptr));
-  HIP_TRY(hipEventRecord(e1, pl->stream));
-  HIP_TRY(hipEventSynchronize(e1));
-  HIP_TRY(hipEventElapsedTime(&pl->gen_ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  pl->xt_dev = d_xt;
+  HIP_TRY(hipEventRecord(pl->lane.e1, pl->stream));
+  HIP_TRY(hipEventSynchronize(pl->lane.e1));
+  HIP_TRY(hipEventElapsedTime(&pl->gen_ms, pl->lane.e0, pl->lane.e1));
   if (smv_tmp) {
     int fl[2];
     HIP_TRY(d2h(fl, smv_tmp + 4 * (size_t)m, sizeof(fl), nullptr));
@@ -982,17 +1029,14 @@ static int launch_solve(xcs_plan *pl, int budget) {
   return XCS_OK;
 }
 
-static int plan_run(xcs_plan *pl, float *ms) {
+// One solve; x_out (where not null) takes the solution.
+static int plan_run(xcs_plan *pl, float *ms, float *x_out = nullptr) {
   XProblem &P = pl->h;
-  // reset: x = 0 and a fresh state (inputs stay resident)
-  HIP_TRY(hipMemsetAsync(P.x, 0, sizeof(float) * P.n, pl->stream));
-  HIP_TRY(hipMemsetAsync(P.st, 0, sizeof(XState), pl->stream));
-  HIP_TRY(hipMemsetAsync(pl->bar, 0, sizeof(unsigned) * BAR_WORDS, pl->stream));
-  XCS_TRY(plan_upload_desc(pl));
-  hipEvent_t e0, e1;
-  HIP_TRY(hipEventCreate(&e0));
-  HIP_TRY(hipEventCreate(&e1));
-  HIP_TRY(hipEventRecord(e0, pl->stream));
+  // inputs stay resident
+  hipLaunchKernelGGL(plan_reset_kernel, dim3(std::max(1, std::min(256, (P.n + 1023) / 1024))), dim3(256),
+                     0, pl->stream, P, pl->d, pl->bar);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipEventRecord(pl->lane.e0, pl->stream));
   if (pl->mode == 1) {
     // plain form: one outer iteration per launch, host reads the stop flag
     // (an aborted team marks the instance done, so launching stops there too)
@@ -1008,15 +1052,29 @@ static int plan_run(xcs_plan *pl, float *ms) {
     int budget = P.maxiter + 4;
     XCS_TRY(launch_solve(pl, budget));
   }
-  HIP_TRY(hipEventRecord(e1, pl->stream));
-  HIP_TRY(hipEventSynchronize(e1));
-  HIP_TRY(hipEventElapsedTime(&pl->last_ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  HIP_TRY(d2h(&pl->last, P.st, sizeof(XState), nullptr));
-  unsigned abort_flag = 0;
-  HIP_TRY(d2h(&abort_flag, pl->bar + 2, sizeof(unsigned), nullptr));
-  if (abort_flag) return set_err(XCS_EHIP, "team barrier timed out (results invalid)");
+  HIP_TRY(hipEventRecord(pl->lane.e1, pl->stream));
+  // the state, the abort flag and a solution that the staging memory holds come
+  // back in one launch behind the solve, for one synchronisation
+  struct Back {
+    XState st;
+    unsigned abort_flag;
+  };
+  static_assert(sizeof(XState) % sizeof(float) == 0 && LANE_X + sizeof(Back) <= LANE_BYTES, "staging memory");
+  Back *back = (Back *)(pl->lane.pin + LANE_X);
+  const bool x_too = x_out && sizeof(float) * (size_t)P.n <= LANE_X;
+  XferList L;
+  L.add((XState *)P.st, &back->st, sizeof(XState) / sizeof(float));
+  L.add(pl->bar + 2, &back->abort_flag, 1);
+  if (x_too) L.add((float *)P.x, pl->lane.pin, P.n);
+  HIP_TRY(xfer(L, pl->stream));
+  HIP_TRY(hipStreamSynchronize(pl->stream));
+  HIP_TRY(hipEventElapsedTime(&pl->last_ms, pl->lane.e0, pl->lane.e1));
+  pl->last = back->st;
+  if (back->abort_flag) return set_err(XCS_EHIP, "team barrier timed out (results invalid)");
+  if (x_too)
+    memcpy(x_out, pl->lane.pin, sizeof(float) * (size_t)P.n);
+  else if (x_out)
+    HIP_TRY(d2h(x_out, P.x, sizeof(float) * (size_t)P.n, pl->stream));
   if (ms) *ms = pl->last_ms;
   return XCS_OK;
 }
@@ -1140,6 +1198,7 @@ struct xcs_batch {
   std::vector<XState> last;
   std::vector<int> order;  // order[q] = caller index of queue slot q
   std::vector<int> slot_of;  // slot_of[i] = queue slot of caller index i
+  ReadAhead ahead;           // solution vectors read in order
   unsigned long long *phase = nullptr;  // XCS_PHASE_TIMING builds only
   float gen_ms = 0.f, last_ms = 0.f;
   void drop_graph() {
@@ -1879,13 +1938,30 @@ int xcs_plan_results(xcs_plan *pl, float norms[3], int *iterations, int support[
   if (!pl) return set_err(XCS_EINVAL, "NULL plan");
   HIP_TRY(hipSetDevice(pl->dev));
   const int n = pl->h.n;
-  std::vector<float> xo((size_t)n);
-  HIP_TRY(d2h(xo.data(), pl->h.x, sizeof(float) * n, nullptr));
-  if (!pl->x_true.empty()) host_norms(pl->x_true, xo.data(), pl->k_planted, norms, support);
+  const bool x_pin = x_out && sizeof(float) * (size_t)n <= LANE_X;
+  const bool planted = pl->xt_dev && (norms || support);
+  if (x_pin || planted) {
+    float *xh = x_pin ? (float *)pl->lane.pin : nullptr;
+    NormPart *part = (NormPart *)(pl->lane.pin + LANE_X);
+    const int wgs = norm_wgs(n);
+    static_assert(LANE_X + NORM_WGS * sizeof(NormPart) <= LANE_BYTES, "staging memory");
+    if (planted) {
+      hipLaunchKernelGGL(norms_kernel, dim3(wgs), dim3(256), 0, pl->stream, (const float *)(float *)pl->h.x,
+                         (const float *)pl->xt_dev, n, xh, part);
+      HIP_TRY(hipGetLastError());
+    } else {
+      XferList L;
+      L.add((float *)pl->h.x, xh, n);
+      HIP_TRY(xfer(L, pl->stream));
+    }
+    HIP_TRY(hipStreamSynchronize(pl->stream));
+    if (planted) norms_finish(part, wgs, n, pl->k_planted, norms, support);
+    if (x_pin) memcpy(x_out, xh, sizeof(float) * (size_t)n);
+  }
+  if (x_out && !x_pin) HIP_TRY(d2h(x_out, pl->h.x, sizeof(float) * (size_t)n, pl->stream));
   if (iterations) *iterations = pl->last.iter;
   if (conv_rate) *conv_rate = conv_rate_results(pl->last);
   if (stop_reason) *stop_reason = pl->last.stop_reason;
-  if (x_out) memcpy(x_out, xo.data(), sizeof(float) * n);
   if (x_true && !pl->x_true.empty()) memcpy(x_true, pl->x_true.data(), sizeof(float) * n);
   return XCS_OK;
 }
@@ -2175,8 +2251,7 @@ static int given_solve(xcs_plan *pl, const float *y, float *x_out, int *iteratio
   XCS_TRY(pl->alloc(&d_y, (size_t)P.lda));
   HIP_TRY(h2d(d_y, y, sizeof(float) * P.m, pl->stream));
   xset(P.y, d_y);
-  XCS_TRY(plan_run(pl, nullptr));
-  if (x_out) HIP_TRY(d2h(x_out, P.x, sizeof(float) * P.n, nullptr));
+  XCS_TRY(plan_run(pl, nullptr, x_out));
   if (iterations) *iterations = pl->last.iter;
   if (conv_rate) *conv_rate = conv_rate_given(pl->last);
   return XCS_OK;
@@ -2184,9 +2259,7 @@ static int given_solve(xcs_plan *pl, const float *y, float *x_out, int *iteratio
 
 static int given_begin(xcs_plan *pl, int gpu) {
   XCS_TRY(use_device(gpu));
-  HIP_TRY(hipGetDevice(&pl->dev));
-  HIP_TRY(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking));
-  return XCS_OK;
+  return pl->open();
 }
 
 int xcs_cs_gen(const char *alg, const float *y, const float *A, int m, int n, int k,
@@ -2530,7 +2603,7 @@ int xcs_generate_gen(int m, int n, unsigned int seed, unsigned int instance, flo
   if (m <= 0 || n <= 0 || !A) return set_err(XCS_EINVAL, "bad arguments");
   XCS_TRY(use_device(0));
   xcs_plan pl;
-  HIP_TRY(hipStreamCreateWithFlags(&pl.stream, hipStreamNonBlocking));
+  XCS_TRY(pl.open());
   float *dA;
   XCS_TRY(pl.alloc(&dA, (size_t)m * n));
   const size_t total = (size_t)m * n;
@@ -2571,7 +2644,7 @@ int xcs_generate_smv(int m, int n, int p, int ens, unsigned int seed, unsigned i
   XCS_TRY(smv_check(m, n, p, ens));
   XCS_TRY(use_device(0));
   xcs_plan pl;
-  HIP_TRY(hipStreamCreateWithFlags(&pl.stream, hipStreamNonBlocking));
+  XCS_TRY(pl.open());
   const size_t nz = (size_t)n * p;
   SmvOut d;
   int *tmp;
@@ -2614,6 +2687,7 @@ int xcs_batch_create(const char *alg, int count, const int *ens, const int *k, c
 int xcs_batch_solve(xcs_batch *B, float *ms) {
   if (!B) return set_err(XCS_EINVAL, "NULL batch");
   HIP_TRY(hipSetDevice(B->dev));
+  B->ahead.drop();
   return batch_run(B, ms);
 }
 
@@ -2652,7 +2726,14 @@ int xcs_batch_x(xcs_batch *B, int idx, float *x_out, float *x_true) {
   HIP_TRY(hipSetDevice(B->dev));
   const int q = B->slot_of[idx];
   const XProblem &P = B->hP[q];
-  if (x_out) HIP_TRY(d2h(x_out, B->xs + B->xoff[q], sizeof(float) * P.n, nullptr));
+  float *const out[2] = {x_out, nullptr};
+  auto piece = [B](int i, int, const float **src, long *n) {
+    const int s = B->slot_of[i];
+    *src = B->xs + B->xoff[s];
+    *n = B->hP[s].n;
+  };
+  if (x_out && !B->ahead.get(idx, B->count, 1, piece, out, B->stream))
+    HIP_TRY(d2h(x_out, B->xs + B->xoff[q], sizeof(float) * P.n, nullptr));
   if (x_true) memcpy(x_true, B->x_true[q].data(), sizeof(float) * P.n);
   return XCS_OK;
 }
@@ -2660,6 +2741,7 @@ int xcs_batch_x(xcs_batch *B, int idx, float *x_out, float *x_true) {
 int xcs_batch_configure(xcs_batch *B, int team_size, int block_size, int big_count) {
   if (!B) return set_err(XCS_EINVAL, "NULL batch");
   HIP_TRY(hipSetDevice(B->dev));
+  B->ahead.drop();
   return batch_configure(B, team_size, block_size, big_count);
 }
 
@@ -2673,6 +2755,7 @@ int xcs_batch_schedule(xcs_batch *B, int phases, const int *team_sizes, const in
     if (team_sizes[p] < 1) return set_err(XCS_EINVAL, "phase team sizes must be >= 1");
   if (B->alg == ALG_CSMPSP) return set_err(XCS_EINVAL, CSMPSP_OFF);
   HIP_TRY(hipSetDevice(B->dev));
+  B->ahead.drop();
   HIP_TRY(hipStreamSynchronize(B->stream));
   B->drop_graph();
   B->sched_team.assign(team_sizes, team_sizes + phases);
@@ -2701,6 +2784,7 @@ int xcs_batch_schedule_mode(xcs_batch *B, int adaptive, int split_team) {
   if (split_team < 0 || split_team > BAR_MAX_TEAM)
     return set_err(XCS_EINVAL, "split_team must be in [0, %d]", BAR_MAX_TEAM);
   HIP_TRY(hipSetDevice(B->dev));
+  B->ahead.drop();
   HIP_TRY(hipStreamSynchronize(B->stream));
   B->drop_graph();
   B->adaptive = adaptive != 0;
@@ -2721,6 +2805,7 @@ int xcs_batch_tune(xcs_batch *B, int probe_iters, const char *cache_path, int ve
     return set_err(XCS_EINVAL, "NULL argument");
   if (probe_iters < 0) return set_err(XCS_EINVAL, "probe_iters must be >= 0");
   HIP_TRY(hipSetDevice(B->dev));
+  B->ahead.drop();
   return batch_tune(B, probe_iters, cache_path, verbose, team_size, block_size, big_count,
                     probe_ms);
 }
@@ -2737,6 +2822,7 @@ int xcs_batch_info(xcs_batch *B, int *teams, int *team_size, int *block, float *
 int xcs_batch_apply_timed(xcs_batch *B, int reps, float *ms_per, double *bytes) {
   if (!B || reps <= 0 || !ms_per) return set_err(XCS_EINVAL, "bad arguments");
   HIP_TRY(hipSetDevice(B->dev));
+  B->ahead.drop();
   int per_cu, cus;
   XCS_TRY(batch_occupancy(B->block, &per_cu, &cus));
   const int grid = std::min(B->count, B->nteams);  // works[] has one entry per team
