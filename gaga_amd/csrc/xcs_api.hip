@@ -730,9 +730,10 @@ static int plan_split(xcs_plan *pl, int alg, const xcs_options *o) {
   if (team <= 0) {
     // As for the dense form the optimum grows with the square root of the size:
     // half of sqrt(n), in powers of two.  Measured on MI355X, ms per solve:
-    // NIHT smv 1000 x 4001 0.294 / 0.259 / 0.279 at 8 / 16 / 32 workgroups; NIHT smv
-    // 4999 x 20001 0.546 / 0.495 / 0.543 at 32 / 64 / 128 (general form 1.64); CGIHT
-    // smv 2^15 x 2^18 4.48 / 3.03 / 2.58 at 64 / 128 / 256 (6.6); NIHT dct n = 2^17
+    // NIHT smv 1500 x 8000 0.238 / 0.253 / 0.273 at 16 / 32 / 64 workgroups; CGIHT smv
+    // 6000 x 30011 0.357 / 0.324 / 0.384 at 32 / 64 / 128, NIHT 15000 x 65536 0.944 /
+    // 0.921 / 1.158 at 64 / 128 / 256, CGIHT 2^15 x 2^18 2.93 / 1.91 / 1.76 at 64 /
+    // 128 / 256 (general form 6.6); NIHT dct n = 2^17
     // 0.785 / 0.619 / 0.552 at 32 / 64 / 128; CGIHT dct n = 2^14 0.366 / 0.302 / 0.307
     // at 8 / 16 / 32; NIHT dct n = 2^20 1.66 at 256 (5.7; fewer do not fit its LDS).
     team = 2;

@@ -10,10 +10,17 @@
 // about twelve fenced barriers, and each carries the scalar sums pending at
 // that point:
 //   * one per matrix product: smv publishes the operand (device-scope stores),
-//     then gathers it through the L2s (one cache invalidation per workgroup;
-//     lanes share a row, so its loads are in flight together); the DCT publishes
-//     its half-transformed data (below);
+//     then gathers it through the L2s (one cache invalidation per workgroup); the
+//     DCT publishes its half-transformed data (below);
 //   * the step length, max |x| and the histogram of the support selection.
+//
+// smv: the matrix entries of the own rows and columns do not change during a solve
+// and stay in LDS as far as it has room, and the operand of every A product is
+// zero off the support, so a row's entries are tested against the support's bits
+// (all n of them in LDS, exchanged once per selection) and only the few that hit
+// are gathered.  An iteration of 2^15 x 2^18 (CGIHT, 256 workgroups) 76 -> 51 us: A x
+// gathers 28 -> 6 us, A^T r 10.7 -> 6.2; what is left is six exchanges (20 us), the
+// A^T gather's random loads and the selection (5).
 //
 // DCT: a transform of n reals is an FFT of N = n / 2 complex values by N = N1 N2
 // (half the work and half the exchanged bytes of the complex transform of the
@@ -27,7 +34,7 @@
 // column transforms are decimation in time from bit-reversed slots and the row
 // transforms decimation in frequency into them, so no permutation is ever made.
 //
-// Measured on MI355X: smv 2^15 x 2^18 CGIHT 6.6 -> 2.58 ms (34 iterations), dct
+// Measured on MI355X: smv 2^15 x 2^18 CGIHT 6.6 -> 1.75 ms (34 iterations), dct
 // n = 2^20 NIHT 5.7 -> 1.66 ms (20 iterations); a DCT product costs about 15 us
 // there where the complex transform in fenced passes took 65 (plan_split has
 // the other sizes and the teams).
@@ -43,11 +50,14 @@ constexpr int SP_LDS = 150 * 1024;    // bytes of LDS for the slices and tables
 constexpr int SP_HIST = 4096;         // histogram bins held in LDS
 constexpr int SP_PAD = 64;            // slices of n-vectors: multiples of a wave
 
+// Histogram bins held in LDS: all of them or none.
+__host__ __device__ inline int sp_hist(int num_bins) { return num_bins <= SP_HIST ? num_bins : 0; }
 // Layout of an instance over `size` workgroups.
 struct SplitGeom {
   int nl, rl;          // floats per workgroup of an n-vector and of an m-vector
   int b1, b2;          // dct: N1 = 2^b1 rows, N2 = 2^b2 columns
   size_t lds;          // bytes
+  bool filter;         // smv: room for the support bits of all columns besides
 };
 __host__ __device__ inline SplitGeom split_geom(int ens, int alg, int m, int n, int log2n,
                                                 int num_bins, int size) {
@@ -65,7 +75,8 @@ __host__ __device__ inline SplitGeom split_geom(int ens, int alg, int m, int n, 
     G.rl = ((m + size - 1) / size + 3) / 4 * 4;
   }
   G.lds += vecs * res_up16(4 * (size_t)G.nl) + 3 * res_up16(4 * (size_t)G.rl) +
-           res_up16((size_t)G.nl / 8 + 8) + res_up16(4 * (size_t)(num_bins < SP_HIST ? num_bins : SP_HIST));
+           res_up16((size_t)G.nl / 8 + 8) + res_up16(4 * (size_t)sp_hist(num_bins));
+  G.filter = ens == ENS_SMV && G.lds + res_up16((size_t)n / 8 + 8) <= (size_t)SP_LDS;
   return G;
 }
 inline bool split_fits(int alg, int ens, int m, int n, int log2n, int num_bins, int timing,
@@ -97,31 +108,41 @@ struct Sp {
   int mid;                     // dct: parity of the exchange buffer
   int nl, nlv, rl, rlv;        // slice lengths and how much of them is in range
   int j0, i0;                  // smv: first column and row
+  unsigned long long *fmask;   // smv: the support bits of all columns, or null (not enough LDS)
+  bool fnew;                   // smv: the own bits have changed since fmask was read
+  // smv: the own rows' and columns' entries, where LDS has room for them (else null);
+  // pointers relative to the first entry
+  const int *lrp, *lcols, *lcp, *lrows;
+  const float *lvals;
+  int rbase;                   // first entry of the own rows
   int b1, b2;
 };
 
 __device__ __forceinline__ bool sp_in(const Sp &R, int i) {
   return (R.mask[i >> 6] >> (i & 63)) & 1ull;
 }
+__device__ __forceinline__ void st_dev_w(XG(unsigned long long) p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long ld_dev_w(XG(const unsigned long long) p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void st_dev2(XG(float2) p, float2 v) {
-  const unsigned long long b =
-      ((unsigned long long)__float_as_uint(v.y) << 32) | (unsigned long long)__float_as_uint(v.x);
-  __hip_atomic_store(reinterpret_cast<XG(unsigned long long)>(p), b, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
+  st_dev_w(reinterpret_cast<XG(unsigned long long)>(p),
+           ((unsigned long long)__float_as_uint(v.y) << 32) | (unsigned long long)__float_as_uint(v.x));
 }
 __device__ __forceinline__ float2 ld_dev2(XG(const float2) p) {
-  const unsigned long long b = __hip_atomic_load(reinterpret_cast<XG(const unsigned long long)>(p),
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long b = ld_dev_w(reinterpret_cast<XG(const unsigned long long)>(p));
   return make_float2(__uint_as_float((unsigned)b), __uint_as_float((unsigned)(b >> 32)));
 }
 
 // ------------------------------------------------------------------ smv ----
 // dst[r] = sum over the entries of row (column) first + r, r < cnt, of
 // val * v[idx], LPR lanes per row: a lane takes every LPR-th entry, eight loads
-// in flight, then the lanes' sums.  NV vectors share the index loads.
-template <int LPR, int NV>
-__device__ __forceinline__ void sp_gather_l(XG(const int) ptr, XG(const int) idx,
-                                            XG(const float) val, int first, int cnt,
+// in flight, then the lanes' sums.  NV vectors share the index loads.  ptr, idx
+// and val are in memory or in LDS.
+template <int LPR, int NV, class PI, class PV>
+__device__ __forceinline__ void sp_gather_l(PI ptr, PI idx, PV val, int first, int cnt,
                                             XG(const float) v0, XG(const float) v1, float *d0,
                                             float *d1) {
   const int sub = threadIdx.x % LPR;
@@ -160,18 +181,127 @@ __device__ __forceinline__ void sp_gather_l(XG(const int) ptr, XG(const int) idx
     }
   }
 }
-template <int NV>
-__device__ __forceinline__ void sp_gather(XG(const int) ptr, XG(const int) idx,
-                                          XG(const float) val, int first, int cnt, int avg,
+// One vector, one lane per row, two rows at a time, and only the loads of
+// entries that exist.
+template <class PI, class PV>
+__device__ __forceinline__ void sp_gather_pair(PI ptr, PI idx, PV val, int first, int cnt,
+                                               XG(const float) v, float *d) {
+  const int nt = blockDim.x;
+  for (int r = threadIdx.x; r < cnt; r += 2 * nt) {
+    const int rb = r + nt < cnt ? r + nt : r;
+    const int ea = ptr[first + r], ea1 = ptr[first + r + 1];
+    const int eb = ptr[first + rb], eb1 = rb == r ? eb : ptr[first + rb + 1];
+    float s[2] = {0.f, 0.f};
+    for (int o = 0; o < max(ea1 - ea, eb1 - eb); o += 8) {
+      int c[2][8];
+      float a[2][8], x[2][8];
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          const int e = (h ? eb : ea) + o + u;
+          c[h][u] = -1;
+          a[h][u] = 0.f;
+          if (e < (h ? eb1 : ea1)) {
+            c[h][u] = idx[e];
+            a[h][u] = val[e];
+          }
+        }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          x[h][u] = 0.f;
+          if (c[h][u] >= 0) x[h][u] = v[c[h][u]];
+        }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (c[h][u] >= 0) s[h] = fmaf(a[h][u], x[h][u], s[h]);
+    }
+    d[r] = s[0];
+    if (rb != r) d[rb] = s[1];
+  }
+}
+template <int NV, class PI, class PV>
+__device__ __forceinline__ void sp_gather(PI ptr, PI idx, PV val, int first, int cnt, int avg,
                                           XG(const float) v0, XG(const float) v1, float *d0,
                                           float *d1) {
-  // as many lanes as leave each about eight entries
+  // as many lanes as leave each about eight entries; two rows at a time where a
+  // thread has that many (A^T r of 2^15 x 2^18: 7.8 us one by one, 6.2 in pairs; of
+  // 2^15 x 2^20, from memory, an iteration 227 and 199 us; with a single row a thread the
+  // pairs are slower, 2.7 against 1.4 us at 3001 x 30011)
   if (avg > 32)
     sp_gather_l<8, NV>(ptr, idx, val, first, cnt, v0, v1, d0, d1);
   else if (avg > 12)
     sp_gather_l<4, NV>(ptr, idx, val, first, cnt, v0, v1, d0, d1);
+  else if (NV == 1 && cnt > (int)blockDim.x)
+    sp_gather_pair(ptr, idx, val, first, cnt, v0, d0);
   else
     sp_gather_l<1, NV>(ptr, idx, val, first, cnt, v0, v1, d0, d1);
+  __syncthreads();
+}
+// The same sums for operands that are zero outside the support, whose bits are
+// in LDS: a lane tests its entries' bits (up to 64 at a time), then reads value
+// and operand of the few that are set, two in flight.  An entry costs two LDS
+// reads instead of a random load through the L2, which is what bounds the
+// product: smv 2^15 x 2^18 (1.8 million entries, k = 3277) 12 us unfiltered, under
+// 3 filtered.  The lanes per row fill the workgroup in one pass over the rows.
+template <int NV, class PI>
+__device__ __forceinline__ void sp_gather_supp(PI ptr, PI idx, XG(const float) val, int first,
+                                               int cnt, const unsigned long long *mask,
+                                               XG(const float) v0, XG(const float) v1, float *d0,
+                                               float *d1) {
+  int lpr = 1;
+  while (lpr < 16 && 2 * lpr * cnt <= (int)blockDim.x) lpr *= 2;
+  const unsigned *mw = reinterpret_cast<const unsigned *>(mask);
+  const int sub = threadIdx.x & (lpr - 1), nr = blockDim.x / lpr;
+  for (int r = threadIdx.x / lpr; r < cnt; r += nr) {
+    const int e0 = ptr[first + r], e1 = ptr[first + r + 1];
+    float s0 = 0.f, s1 = 0.f;
+    for (int e = e0 + sub; e < e1; e += 64 * lpr) {
+      unsigned long long hits = 0ull;
+      for (int u0 = 0; u0 < 64 && e + u0 * lpr < e1; u0 += 8) {
+        int c[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) c[u] = idx[min(e + (u0 + u) * lpr, e1 - 1)];
+        unsigned h = 0;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (e + (u0 + u) * lpr < e1) h |= ((mw[c[u] >> 5] >> (c[u] & 31)) & 1u) << u;
+        hits |= (unsigned long long)h << u0;
+      }
+      while (hits) {
+        const int ea = e + (__ffsll(hits) - 1) * lpr;
+        hits &= hits - 1;
+        const bool two = hits != 0ull;
+        const int eb = two ? e + (__ffsll(hits) - 1) * lpr : ea;
+        hits &= hits - 1;
+        const int ca = idx[ea], cb = idx[eb];
+        const float aa = val[ea], ab = val[eb], xa = v0[ca], xb = v0[cb];
+        float pa = 0.f, pb = 0.f;
+        if (NV == 2) {
+          pa = v1[ca];
+          pb = v1[cb];
+        }
+        s0 = fmaf(aa, xa, s0);
+        if (NV == 2) s1 = fmaf(aa, pa, s1);
+        if (two) {
+          s0 = fmaf(ab, xb, s0);
+          if (NV == 2) s1 = fmaf(ab, pb, s1);
+        }
+      }
+    }
+    for (int o = 1; o < lpr; o <<= 1) {
+      s0 += __shfl_xor(s0, o);
+      if (NV == 2) s1 += __shfl_xor(s1, o);
+    }
+    if (sub == 0) {
+      d0[r] = s0;
+      if (NV == 2) d1[r] = s1;
+    }
+  }
   __syncthreads();
 }
 
@@ -317,7 +447,8 @@ struct SpOp;
 
 template <>
 struct SpOp<ENS_SMV> {
-  // d0 = A s0 (and d1 = A s1); operands cut to the support where m is set
+  // d0 = A s0 (and d1 = A s1); operands cut to the support where m is set, zero
+  // outside it where not
   template <int NV, int K, int MAXES = 0>
   static __device__ __forceinline__ void A(RTeam &t, Sp &R, const XProblem &P, const float *s0,
                                            bool m0, const float *s1, bool m1, float *d0, float *d1,
@@ -329,10 +460,28 @@ struct SpOp<ENS_SMV> {
       st_dev(b0 + R.j0 + i, (m0 && !in) ? 0.f : s0[i]);
       if (NV == 2) st_dev(b1 + R.j0 + i, (m1 && !in) ? 0.f : s1[i]);
     }
+    // the support bits go along the first time after they have changed (P.bins is
+    // written at the end of a solve and read at the start of a continued one)
+    const bool bits = R.fmask && R.fnew;
+    XG(unsigned long long) fw = reinterpret_cast<XG(unsigned long long)>(P.bins);
+    if (bits)
+      for (int w = threadIdx.x; 64 * w < R.nlv; w += blockDim.x)
+        st_dev_w(fw + (R.j0 >> 6) + w, R.mask[w]);
     rt_allreduce<K, MAXES>(t, *R.rt, v, o);
     if (threadIdx.x < WAVE) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (bits) {
+      ld_dev_vec((float *)R.fmask, reinterpret_cast<XG(const float)>(P.bins), 2 * ((P.n + 63) >> 6));
+      R.fnew = false;
+    }
     __syncthreads();
-    sp_gather<NV>(P.row_ptr, P.cols, P.rvals, R.i0, R.rlv, P.nz / P.m, b0, b1, d0, d1);
+    XG(const float) v0 = b0;
+    XG(const float) v1 = b1;
+    if (R.lcols)
+      sp_gather_supp<NV>(R.lrp, R.lcols, P.rvals + R.rbase, 0, R.rlv, R.fmask, v0, v1, d0, d1);
+    else if (R.fmask)
+      sp_gather_supp<NV>(P.row_ptr, P.cols, P.rvals, R.i0, R.rlv, R.fmask, v0, v1, d0, d1);
+    else
+      sp_gather<NV>(P.row_ptr, P.cols, P.rvals, R.i0, R.rlv, P.nz / P.m, v0, v1, d0, d1);
   }
   // d = A^T s
   template <int K, int MAXES = 0>
@@ -343,7 +492,11 @@ struct SpOp<ENS_SMV> {
     rt_allreduce<K, MAXES>(t, *R.rt, v, o);
     if (threadIdx.x < WAVE) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();
-    sp_gather<1>(P.col_ptr, P.rows, P.vals, R.j0, R.nlv, P.nz / P.n, b, nullptr, d, nullptr);
+    XG(const float) r = b;
+    if (R.lrows)
+      sp_gather<1>(R.lcp, R.lrows, R.lvals, 0, R.nlv, P.nz / P.n, r, r, d, nullptr);
+    else
+      sp_gather<1>(P.col_ptr, P.rows, P.vals, R.j0, R.nlv, P.nz / P.n, r, r, d, nullptr);
   }
 };
 
@@ -669,6 +822,7 @@ __device__ __forceinline__ double sp_rebin(RTeam &t, Sp &R, const XProblem &P, R
       R.mask[i >> 6] = bits;
     }
   }
+  R.fnew = true;
   __syncthreads();
   return left;
 }
@@ -806,7 +960,7 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
     R.t0 = (float *)take(4 * (size_t)G.rl);
     R.t1 = (float *)take(4 * (size_t)G.rl);
     R.mask = (unsigned long long *)take((size_t)G.nl / 8 + 8);
-    R.hist = (int *)take(4 * (size_t)min(P.num_bins, SP_HIST));
+    R.hist = (int *)take(4 * (size_t)sp_hist(P.num_bins));
     R.rmask = nullptr;
     R.w1 = R.w2 = nullptr;
     if (ENS == ENS_DCT) {
@@ -821,6 +975,12 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
       R.w2 = w2;
     }
   }
+  R.fmask = nullptr;
+  R.fnew = true;
+  R.lrp = R.lcols = R.lcp = R.lrows = nullptr;
+  R.lvals = nullptr;
+  R.rbase = 0;
+  if (G.filter) R.fmask = (unsigned long long *)(lds + G.lds);
   R.slots = &slots;
   R.rt = &rt;
   R.bank = R.par = R.mid = 0;
@@ -850,7 +1010,40 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
   } else {
     for (int i = threadIdx.x; i < R.rlv; i += nt) R.y[i] = P.y[R.i0 + i];
   }
-  for (int b = threadIdx.x; b < min(P.num_bins, SP_HIST); b += nt) R.hist[b] = 0;
+  if (ENS == ENS_SMV && G.filter) {
+    // the matrix entries do not change during a solve: what LDS has left takes the
+    // own rows' columns, then the own columns' rows and values
+    unsigned char *q = lds + G.lds + res_up16((size_t)n / 8 + 8), *end = lds + SP_LDS;
+    auto room = [&](int words) { return (size_t)(end - q) >= res_up16(4 * (size_t)words); };
+    auto take = [&](int words) {
+      unsigned char *r = q;
+      q += res_up16(4 * (size_t)words);
+      return r;
+    };
+    R.rbase = P.row_ptr[R.i0];
+    const int rn = P.row_ptr[R.i0 + R.rlv] - R.rbase;
+    if (room(R.rlv + 1 + rn + 8)) {
+      int *rp = (int *)take(R.rlv + 1), *cols = (int *)take(rn);
+      for (int i = threadIdx.x; i <= R.rlv; i += nt) rp[i] = P.row_ptr[R.i0 + i] - R.rbase;
+      for (int e = threadIdx.x; e < rn; e += nt) cols[e] = P.cols[R.rbase + e];
+      R.lrp = rp;
+      R.lcols = cols;
+    }
+    const int cbase = P.col_ptr[R.j0], cn = P.col_ptr[R.j0 + R.nlv] - cbase;
+    if (room(R.nlv + 1 + 2 * cn + 12)) {
+      int *cp = (int *)take(R.nlv + 1), *rows = (int *)take(cn);
+      float *vals = (float *)take(cn);
+      for (int i = threadIdx.x; i <= R.nlv; i += nt) cp[i] = P.col_ptr[R.j0 + i] - cbase;
+      for (int e = threadIdx.x; e < cn; e += nt) {
+        rows[e] = P.rows[cbase + e];
+        vals[e] = P.vals[cbase + e];
+      }
+      R.lcp = cp;
+      R.lrows = rows;
+      R.lvals = vals;
+    }
+  }
+  for (int b = threadIdx.x; b < sp_hist(P.num_bins); b += nt) R.hist[b] = 0;
   for (int w = threadIdx.x; w <= R.nl / 64; w += nt) R.mask[w] = 0ull;
   {  // both counter arrays start at zero (read after the first exchanges)
     const int cb = (P.num_bins + t.size - 1) / t.size, lo = t.rank * cb;
