@@ -59,7 +59,7 @@ struct MrhsDesc {
   double *ref;  // per signal: gamma, |r|^2, |y|^2, spare
   int *supp, *supp_cnt;
   float *cp, *cd;  // refinement: CG direction and correction, by list position
-  const float *A32;
+  const float *A32b;  // A in FP32, in blocks of MR_RB rows
 };
 
 __device__ __forceinline__ float4 mr_ld4(const float *p, long o) {
@@ -734,128 +734,133 @@ __global__ void __launch_bounds__(MR_VT) mr_ref_supp_kernel(MrhsDesc D, int sel)
   if (threadIdx.x == 0) D.supp_cnt[s] = base;
 }
 
-// r = y - A_S x_S from the FP32 A with FP64 sums over the support list of
-// each selected signal.  Pass 1: one workgroup per (slice z of `slices`,
-// signal) streams whole columns (contiguous m floats): support chunks z,
-// z + slices, ... of MR_CHUNK entries are staged through LDS, and each
-// thread owns rows 4t + 1024q (float4 loads), keeping FP64 row sums in
-// registers; the slice's sums go to rowpart.  The next column's loads are issued
-// before this one's products (NQ float4 per thread and column; NQ = 4 for m <=
-// 4096 leaves room for both).  Pass 2 (mr_resid_sum_kernel): slices summed in
-// order, r (FP32, and BF16 as the next A^T operand) and the FP64 partial of
-// ||r||^2 of each 256-row block (part[s * nblk + block]).  Needs m <= 1024 *
-// MR_MAXQ.
-constexpr int MR_SLICES = 64;
-constexpr int MR_CHUNK = 16;
-constexpr int MR_MAXQ = 8;
-template <int NQ>
-__global__ void __launch_bounds__(MR_THREADS) mr_exact_resid_kernel(MrhsDesc D, double *rowpart,
-                                                                    int slices, int sel) {
-  __shared__ int sj[MR_CHUNK];
-  __shared__ float sv[MR_CHUNK];
-  const int z = blockIdx.x, s = mr_signal(D, sel, blockIdx.y);
+// r = y - A x on the support with FP32 A and 64-bit products and sums, for each
+// selected signal, with the FP64 part of ||r||^2 of each block of MR_RB rows
+// (part[s * (m / MR_RB) + block]) and r's BF16 copy (the next A^T operand).  A
+// workgroup takes one signal and row blocks xcd, xcd + 8, ... (its share of
+// them); eight lanes read the 128 bytes of a column's block, so a wave has eight
+// columns per load and a lane MR_RU loads in flight, and the columns' sums
+// meet in the workgroup in a fixed order.  The support list is padded with zero
+// values to whole rounds of 16 columns: no load is conditional.
+// The gathered columns are 4 m k bytes a signal, 3.4 GB for 512 signals of m =
+// 4096, k = 400.  Whole columns at a time they came from beyond the L2s at 7 TB/s
+// (471 us and 20 for adding the slices' sums; now 219).  Workgroups are dealt to the
+// 8 XCDs round robin, so here an XCD's workgroups all work on the same few row
+// blocks (2 MB each at n = 16384), which stay in its L2 while the signals pass: 82%
+// of the loads hit.  From the column-major matrix one row block's lines are 16 KB
+// apart, on few of an L2's channels (420 us), so A lies in row blocks here.  The
+// workgroups have to keep step for that: more loads a lane run them further apart
+// (256 threads with 4 / 2 / 1 loads: 324 / 246 / 286 us at 37 / 71 / 78% hits; 128 with
+// 8 / 4 / 2: 315 / 296 / 219; 64 with 4: 219).
+constexpr int MR_RB = 32;
+constexpr int MR_RT = 128;
+constexpr int MR_RU = 2;
+constexpr int MR_RLIST = 1024;  // support entries held in LDS at a time
+constexpr int MR_MAXM = 8192;
+__global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, double *part,
+                                                                    int groups, int sel) {
+  constexpr int SLOTS = MR_RT / 8, ROWS = MR_RT / 16;
+  static_assert(MR_RLIST % SLOTS == 0, "whole rounds");
+  __shared__ uint2 list[MR_RLIST];  // (byte offset of the column in a block, value)
+  __shared__ double red[ROWS][MR_RB];
+  const int s = mr_signal(D, sel, blockIdx.x >> 3);
   if (s < 0) return;
+  const int sub = threadIdx.x & 7, slot = threadIdx.x >> 3;
   const long n = D.n, m = D.m;
-  const int cnt = D.supp_cnt[s];
-  if (z * MR_CHUNK >= cnt) return;
+  const int cnt = D.supp_cnt[s], blocks = D.m / MR_RB;
   const float *x = D.x + s * n;
   const int *sup = D.supp + s * n;
-  double acc[NQ][4];
+  bool staged = false;
+  for (int b = (blockIdx.x & 7) + 8 * blockIdx.y; b < blocks; b += 8 * groups) {
+    const char *base = reinterpret_cast<const char *>(D.A32b + (long)b * n * MR_RB);
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int c0 = 0; c0 < cnt; c0 += MR_RLIST) {
+      const int c1 = min(MR_RLIST, (cnt - c0 + SLOTS - 1) / SLOTS * SLOTS);
+      if (!staged || cnt > MR_RLIST) {
+        __syncthreads();
+        for (int c = threadIdx.x; c < c1; c += MR_RT) {
+          uint2 e = make_uint2(0u, 0u);
+          if (c0 + c < cnt) {
+            const int j = sup[c0 + c];
+            e = make_uint2((unsigned)j * (4u * MR_RB), __float_as_uint(x[j]));
+          }
+          list[c] = e;
+        }
+        __syncthreads();
+        staged = true;
+      }
+      auto add = [&](const float4 &v, unsigned w) {
+        const double xv = (double)__uint_as_float(w);
+        acc[0] = fma((double)v.x, xv, acc[0]);
+        acc[1] = fma((double)v.y, xv, acc[1]);
+        acc[2] = fma((double)v.z, xv, acc[2]);
+        acc[3] = fma((double)v.w, xv, acc[3]);
+      };
+      int c = slot;
+      for (; c + (MR_RU - 1) * SLOTS < c1; c += MR_RU * SLOTS) {
+        uint2 e[MR_RU];
+        float4 v[MR_RU];
 #pragma unroll
-  for (int q = 0; q < NQ; q++)
+        for (int u = 0; u < MR_RU; u++) e[u] = list[c + u * SLOTS];
 #pragma unroll
-    for (int e = 0; e < 4; e++) acc[q][e] = 0.0;
-  auto load = [&](int c, float4 (&v)[NQ]) {
-    const float *col = D.A32 + (long)sj[c] * m;
+        for (int u = 0; u < MR_RU; u++) v[u] = *(const float4 *)(base + (e[u].x + 16u * sub));
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int i = 4 * (int)threadIdx.x + 4 * MR_THREADS * q;
-      v[q] = i < D.m ? *(const float4 *)(col + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  };
-  auto add = [&](const float4 (&v)[NQ], float x1) {
-    const double xv = (double)x1;
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      acc[q][0] = fma((double)v[q].x, xv, acc[q][0]);
-      acc[q][1] = fma((double)v[q].y, xv, acc[q][1]);
-      acc[q][2] = fma((double)v[q].z, xv, acc[q][2]);
-      acc[q][3] = fma((double)v[q].w, xv, acc[q][3]);
-    }
-  };
-  for (int c0 = z * MR_CHUNK; c0 < cnt; c0 += slices * MR_CHUNK) {
-    __syncthreads();
-    if (threadIdx.x < MR_CHUNK && c0 + (int)threadIdx.x < cnt) {
-      const int j = sup[c0 + threadIdx.x];
-      sj[threadIdx.x] = j;
-      sv[threadIdx.x] = x[j];
-    }
-    __syncthreads();
-    const int c1 = min(MR_CHUNK, cnt - c0);
-    float4 v0[NQ], v1[NQ];
-    load(0, v0);
-    for (int c = 0; c < c1; c += 2) {
-      if (c + 1 < c1) load(c + 1, v1);
-      add(v0, sv[c]);
-      if (c + 1 < c1) {
-        if (c + 2 < c1) load(c + 2, v0);
-        add(v1, sv[c + 1]);
+        for (int u = 0; u < MR_RU; u++) add(v[u], e[u].y);
+      }
+      for (; c < c1; c += SLOTS) {
+        const uint2 e = list[c];
+        add(*(const float4 *)(base + (e.x + 16u * sub)), e.y);
       }
     }
-  }
-  double *o = rowpart + ((long)s * slices + z) * m;
 #pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    const int i = 4 * (int)threadIdx.x + 4 * MR_THREADS * q;
-    if (i < D.m) {
-      *(double2 *)(o + i) = make_double2(acc[q][0], acc[q][1]);
-      *(double2 *)(o + i + 2) = make_double2(acc[q][2], acc[q][3]);
+    for (int e = 0; e < 4; e++) acc[e] += dpp_d<DPP_ROR8, 0xf>(acc[e]);
+    if ((threadIdx.x & 15) < 8) {
+      double *o = &red[threadIdx.x >> 4][4 * sub];
+      *(double2 *)o = make_double2(acc[0], acc[1]);
+      *(double2 *)(o + 2) = make_double2(acc[2], acc[3]);
     }
+    __syncthreads();
+    if (threadIdx.x < MR_RB) {
+      double a = 0.0;
+#pragma unroll
+      for (int q = 0; q < ROWS; q++) a += red[q][threadIdx.x];
+      const long i = s * m + b * MR_RB + threadIdx.x;
+      const double ri = (double)D.y[i] - a;
+      const float rf = (float)ri;
+      D.resid[i] = rf;
+      reinterpret_cast<uint16_t *>(D.rb)[i] = f2bf16_rne(rf);
+      double e2 = ri * ri;
+      for (int o = MR_RB / 2; o; o >>= 1) e2 += __shfl_xor(e2, o);
+      if (threadIdx.x == 0) part[(long)s * blocks + b] = e2;
+    }
+    __syncthreads();
   }
 }
 
-__global__ void __launch_bounds__(MR_THREADS) mr_resid_sum_kernel(MrhsDesc D,
-                                                                  const double *rowpart,
-                                                                  double *part, int slices,
-                                                                  int sel) {
-  __shared__ double red[MR_THREADS / 64];
-  const int s = mr_signal(D, sel, blockIdx.y);
-  if (s < 0) return;
-  const long m = D.m;
-  const int cnt = D.supp_cnt[s];
-  const int used = min(slices, (cnt + MR_CHUNK - 1) / MR_CHUNK);  // slices that wrote
-  const int i = blockIdx.x * MR_THREADS + threadIdx.x;
-  double e2 = 0.0;
-  if (i < D.m) {
-    double a = 0.0;
-#pragma unroll 8
-    for (int z = 0; z < used; z++) a += rowpart[((long)s * slices + z) * m + i];
-    const double ri = (double)D.y[s * m + i] - a;
-    const float rf = (float)ri;
-    D.resid[s * m + i] = rf;
-    reinterpret_cast<uint16_t *>(D.rb)[s * m + i] = f2bf16_rne(rf);
-    e2 = ri * ri;
-  }
-  e2 = wave_sum(e2);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e2;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < MR_THREADS / 64; w++) t += red[w];
-    part[(long)s * gridDim.x + blockIdx.x] = t;
+// A in blocks of MR_RB rows, each block's columns one after the other.
+__global__ void __launch_bounds__(MR_THREADS) mr_blocks_kernel(const float4 *A, int m, int n, float4 *out) {
+  constexpr int Q = MR_RB / 4;
+  const long per = (long)n * Q, total = per * (m / MR_RB);
+  for (long e = (long)blockIdx.x * MR_THREADS + threadIdx.x; e < total; e += (long)gridDim.x * MR_THREADS) {
+    const long b = e / per, j = (e - b * per) / Q;
+    out[e] = A[j * (m / 4) + b * Q + e % Q];
   }
 }
 
 // ||r||^2 of the selected signals (after the exact residual) into ref; with mark
 // (the support corrections' entry) the signals with ||r|| > tol become active.
+// One wave per signal.
 __global__ void __launch_bounds__(MR_THREADS) mr_norm_kernel(MrhsDesc D, const double *part,
-                                                             int nblk, int sel, int mark) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+                                                             int sel, int mark) {
+  const int b = blockIdx.x * (MR_THREADS / 64) + threadIdx.x / 64;
   if (b >= D.count) return;
   const int s = mr_signal(D, sel, b);
   if (s < 0) return;
+  const int lane = threadIdx.x & 63, blocks = D.m / MR_RB;
   double t = 0.0;
-  for (int q = 0; q < nblk; q++) t += part[(long)s * nblk + q];
+  for (int q = lane; q < blocks; q += 64) t += part[(long)s * blocks + q];
+  t = wsum_d(t);
+  if (lane) return;
   D.ref[4 * (long)s + 1] = t;
   if (mark) D.stage[s] = (D.st[s].max_value != 0.f && sqrt(t) > (double)D.tol) ? 0 : 1;
 }
@@ -1091,16 +1096,14 @@ struct xcs_mrhs {
   int ref_outer = 2, ref_inner = 4;
   float c16 = 0.0078125f, c8 = 0.125f;
   MrhsDesc D{};
-  float *A32 = nullptr, *cs = nullptr;
+  float *A32 = nullptr, *A32b = nullptr, *cs = nullptr;
   uint8_t *a16cm = nullptr, *a16rm = nullptr, *a8cm = nullptr, *a8rm = nullptr;
   std::vector<void *> allocs;
   std::vector<std::vector<float>> x_true;
   int lp_iters[3] = {0, 0, 0};
   float last_ms = 0.f, gen_ms = 0.f;
   int *h_nactive = nullptr;  // pinned
-  double *part = nullptr;    // exact-residual partials (count x ceil(m / 256))
-  double *rowpart = nullptr; // exact-residual row sums per slice (count x MR_SLICES x m)
-  int nblk = 1;
+  double *part = nullptr;    // exact-residual partials (count x m / MR_RB)
   int polish_max = 6;  // support-correction steps
   int gemm_big = -1;   // GEMM block tile where M allows: 0 128 x 128, 1 256 x 128, 2 256 x 256, -1 by gemm_tile
   xcs_options opts{};
@@ -1214,7 +1217,7 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
     return set_err(XCS_EINVAL, "need 0 < k <= m, n > 0, count > 0");
   if (m % 128 || n % 512)
     return set_err(XCS_EINVAL, "many-rhs products need m %% 128 == 0 and n %% 512 == 0");
-  if (m > 4 * MR_THREADS * MR_MAXQ) return set_err(XCS_EINVAL, "many-rhs needs m <= %d", 4 * MR_THREADS * MR_MAXQ);
+  if (m > MR_MAXM) return set_err(XCS_EINVAL, "many-rhs needs m <= %d", MR_MAXM);
   XCS_TRY(use_device(o->gpu_number));
   HIP_TRY(hipGetDevice(&h->dev));
   HIP_TRY(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
@@ -1234,6 +1237,10 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   XCS_TRY(h->alloc(&h->A32, mn));
   hipLaunchKernelGGL(gen_matrix_kernel, dim3((int)std::min<size_t>(65536, (mn + 255) / 256)),
                      dim3(256), 0, h->stream, h->A32, m, n, m, o->seed, o->instance);
+  HIP_TRY(hipGetLastError());
+  XCS_TRY(h->alloc(&h->A32b, mn));
+  hipLaunchKernelGGL(mr_blocks_kernel, dim3((int)std::min<size_t>(65536, (mn / 4 + MR_THREADS - 1) / MR_THREADS)),
+                     dim3(MR_THREADS), 0, h->stream, (const float4 *)h->A32, m, n, (float4 *)h->A32b);
   HIP_TRY(hipGetLastError());
   XCS_TRY(h->alloc(&h->cs, (size_t)n));
   XCS_TRY(h->alloc(&h->a16cm, 2 * mn));
@@ -1263,7 +1270,7 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   D.restart = o->restart;
   D.maxiter = o->maxiter > 0 ? o->maxiter : 5000;
   D.tol = o->tol_reference_default ? (float)(10 ^ (-4)) : o->tol;
-  D.A32 = h->A32;
+  D.A32b = h->A32b;
   D.colscale = h->cs;
   float *y;
   XCS_TRY(h->alloc(&y, S * m));
@@ -1298,9 +1305,7 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   XCS_TRY(h->alloc(&D.supp_cnt, S));
   XCS_TRY(h->alloc(&D.cp, S * k));
   XCS_TRY(h->alloc(&D.cd, S * k));
-  h->nblk = (m + MR_THREADS - 1) / MR_THREADS;
-  XCS_TRY(h->alloc(&h->part, S * h->nblk));
-  XCS_TRY(h->alloc(&h->rowpart, S * MR_SLICES * m));
+  XCS_TRY(h->alloc(&h->part, S * (m / MR_RB)));
   // planted signals (supports and values drawn on the device, key (seed,
   // instance + 1 + signal)) and y = A x_true (FP32 A, FP64 sums)
   float *d_vals;
@@ -1348,23 +1353,14 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
 static dim3 mr_grid(const xcs_mrhs *h, int sel) { return dim3(sel ? *h->h_nactive : h->count); }
 
 static int mr_exact_resid(xcs_mrhs *h, int sel) {
-  // Slices per signal: every slice's row sums go through memory (m doubles written
-  // and read), so as few as still give about 16 workgroups per CU; a few signals
-  // take all MR_SLICES.  512 signals, k = 400, m = 4096: 8 slices 471 us and 28 for
-  // their sum, where 25 slices of one chunk each moved 840 MB of row sums (and the
-  // single-buffered loads took 600 us).
-  const int cols = (int)mr_grid(h, sel).x;
-  int slices = MR_SLICES;
-  while (slices > 4 && (long)slices * cols > 4096) slices /= 2;
-  const dim3 g(slices, cols);
-  if (h->m <= 4 * 4 * MR_THREADS)
-    hipLaunchKernelGGL(mr_exact_resid_kernel<4>, g, dim3(MR_THREADS), 0, h->stream, h->D,
-                       h->rowpart, slices, sel);
-  else
-    hipLaunchKernelGGL(mr_exact_resid_kernel<MR_MAXQ>, g, dim3(MR_THREADS), 0, h->stream, h->D,
-                       h->rowpart, slices, sel);
-  hipLaunchKernelGGL(mr_resid_sum_kernel, dim3(h->nblk, cols), dim3(MR_THREADS), 0, h->stream, h->D,
-                     h->rowpart, h->part, slices, sel);
+  const int cols = (int)mr_grid(h, sel).x, per = std::max(1, h->m / MR_RB / 8);  // blocks of an XCD
+  // at least 4096 workgroups (512 signals: one for all blocks of an XCD, 219 us; two
+  // 241, four 272), and no more than there are blocks
+  int groups = 1;
+  while (groups < per && 8L * groups * cols < 4096) groups *= 2;
+  groups = std::min(groups, per);
+  hipLaunchKernelGGL(mr_exact_resid_kernel, dim3(8 * cols, groups), dim3(MR_RT), 0, h->stream, h->D,
+                     h->part, groups, sel);
   HIP_TRY(hipGetLastError());
   return XCS_OK;
 }
@@ -1437,8 +1433,8 @@ static int mr_refine(xcs_mrhs *h, int sel, int mark) {
   }
   // final FP64 residual
   XCS_TRY(mr_exact_resid(h, sel));
-  hipLaunchKernelGGL(mr_norm_kernel, dim3((cols + MR_THREADS - 1) / MR_THREADS), dim3(MR_THREADS),
-                     0, h->stream, D, h->part, h->nblk, sel, mark);
+  hipLaunchKernelGGL(mr_norm_kernel, dim3((cols + MR_THREADS / 64 - 1) / (MR_THREADS / 64)),
+                     dim3(MR_THREADS), 0, h->stream, D, h->part, sel, mark);
   HIP_TRY(hipGetLastError());
   return XCS_OK;
 }
