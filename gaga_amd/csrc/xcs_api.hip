@@ -1183,6 +1183,7 @@ struct xcs_batch {
   XProblem *dP = nullptr;
   float *xs = nullptr;       // every x, contiguous (queue order)
   size_t xs_len = 0;
+  char *back = nullptr;      // pinned: the abort flag, then the states (batch_states)
   float *xs_host = nullptr;  // pinned copy of xs for the results (allocated on first use)
   std::vector<size_t> xoff;
   XState *sts = nullptr;
@@ -1217,6 +1218,7 @@ struct xcs_batch {
     drop_work();
     for (void *q : allocs) (void)hipFree(q);
     if (xs_host) (void)hipHostFree(xs_host);
+    if (back) (void)hipHostFree(back);
     if (stream) (void)hipStreamDestroy(stream);
   }
   int raw(void **q, size_t bytes, bool clear, std::vector<void *> &list) {
@@ -1615,7 +1617,7 @@ static int batch_generate(xcs_batch *B, int alg, int count, const int *ens, cons
 
 // Reset, then solve: the two launches of one batched solve, on B->stream.
 // budget: iterations per instance in this launch.
-static int batch_enqueue(xcs_batch *B, int budget) {
+static int batch_enqueue(xcs_batch *B, int budget, int c, int grid) {
   const int rgrid = (int)std::min<size_t>(4096, (B->xs_len + 255) / 256 + 1);
   hipLaunchKernelGGL(batch_reset_kernel, dim3(rgrid), dim3(256), 0, B->stream, B->xs, B->xs_len,
                      (int *)B->sts, sizeof(XState) / sizeof(int) * (size_t)B->count, B->queue,
@@ -1624,15 +1626,18 @@ static int batch_enqueue(xcs_batch *B, int budget) {
   const int *list = nullptr;
   void *args[] = {(void *)&B->dP, (void *)&B->count, (void *)&B->n_big, (void *)&B->queue,
                   (void *)&B->dW, (void *)&B->slots, (void *)&B->red, (void *)&B->bar,
-                  (void *)&B->c, (void *)&budget, (void *)&list, (void *)&B->spin_limit};
-  if (B->c > 1) {
-    HIP_TRY(hipLaunchCooperativeKernel((const void *)solve_batch_kernel<true>, dim3(B->grid),
+                  (void *)&c, (void *)&budget, (void *)&list, (void *)&B->spin_limit};
+  if (c > 1) {
+    HIP_TRY(hipLaunchCooperativeKernel((const void *)solve_batch_kernel<true>, dim3(grid),
                                        dim3(B->block), args, 0, B->stream));
   } else {
-    HIP_TRY(hipLaunchKernel((const void *)solve_batch_kernel<false>, dim3(B->grid),
+    HIP_TRY(hipLaunchKernel((const void *)solve_batch_kernel<false>, dim3(grid),
                             dim3(B->block), args, 0, B->stream));
   }
   return XCS_OK;
+}
+static int batch_enqueue(xcs_batch *B, int budget) {
+  return batch_enqueue(B, budget, B->c, B->grid);
 }
 
 // Single-workgroup teams: the reset and the persistent solve are captured
@@ -1660,13 +1665,22 @@ static int batch_capture(xcs_batch *B) {
   return XCS_OK;
 }
 
+// Teams of c workgroups for up to `want` instances: whole groups of eight (one
+// per XCD, see batch_team), with a few spare teams where the chip has room for
+// them rather than a few instances that wait.
+static int batch_teams(const xcs_batch *B, int want, int c) {
+  const int most = B->resident / c;
+  int nteams = std::min(want, most);
+  if (c > 1 && nteams >= 8) nteams = (nteams + 7) / 8 * 8 <= most ? (nteams + 7) / 8 * 8 : nteams - nteams % 8;
+  return nteams;
+}
+
 // A later phase of the tail schedule: the `cnt` instances at queue positions
 // B->list[0, cnt) on teams of c workgroups (whole teams per XCD where they
 // fit), at most `budget` more iterations each.  Cooperative launch for c > 1.
 static int batch_enqueue_phase(xcs_batch *B, int cnt, int c, int budget) {
   c = std::max(1, std::min(c, std::min(B->resident, BAR_MAX_TEAM)));
-  int nteams = std::min(cnt, B->resident / c);
-  if (c > 1 && nteams >= 8) nteams -= nteams % 8;
+  const int nteams = batch_teams(B, cnt, c);
   const int grid = nteams * c, n_big = c > 1 ? cnt : 0;
   hipLaunchKernelGGL(batch_reset_kernel, dim3(64), dim3(256), 0, B->stream, B->xs, (size_t)0,
                      (int *)B->sts, (size_t)0, B->queue, B->bar, (size_t)BAR_WORDS * nteams);
@@ -1685,14 +1699,34 @@ static int batch_enqueue_phase(xcs_batch *B, int cnt, int c, int budget) {
   return XCS_OK;
 }
 
-static int batch_check_abort(xcs_batch *B) {
-  // the abort word (word 2) of every team's barrier words, one strided copy
-  std::vector<unsigned> ab((size_t)B->resident);
-  HIP_TRY(hipMemcpy2DAsync(ab.data(), sizeof(unsigned), B->bar + 2, sizeof(unsigned) * BAR_WORDS,
-                           sizeof(unsigned), (size_t)B->resident, hipMemcpyDeviceToHost, B->stream));
+// The solver states of queue slots [0, cnt) and whether a team's abort word (word
+// 2 of its barrier words) is set, straight into pinned memory.
+__global__ void __launch_bounds__(256) batch_back_kernel(const int *st, int words, const unsigned *bar,
+                                                         int teams, int *out, int *aborted) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) out[i] = st[i];
+  if (blockIdx.x == 0) {
+    int bad = 0;
+    for (int t = threadIdx.x; t < teams; t += 256) bad |= bar[(size_t)t * BAR_WORDS + 2] != 0u;
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) *aborted = bad;
+  }
+}
+
+// B->last of slots [0, cnt) after what the stream holds, in one launch and one
+// synchronisation; an aborted team is an error.  (A strided copy of the abort words
+// into pageable memory moved one word at a time: 5 ms for 512 teams.)
+static int batch_states(xcs_batch *B, int cnt) {
+  if (!B->back)
+    HIP_TRY(hipHostMalloc((void **)&B->back, sizeof(XState) * (size_t)B->count + 64, hipHostMallocDefault));
+  XState *st = (XState *)(B->back + 64);
+  const int words = (int)(sizeof(XState) / sizeof(int)) * cnt;
+  hipLaunchKernelGGL(batch_back_kernel, dim3(std::max(1, std::min(64, (words + 1023) / 1024))), dim3(256), 0,
+                     B->stream, (const int *)B->sts, words, (const unsigned *)B->bar, B->resident, (int *)st,
+                     (int *)B->back);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(B->stream));
-  for (int t = 0; t < B->resident; t++)
-    if (ab[t]) return set_err(XCS_EHIP, "team barrier timed out (results invalid)");
+  std::copy(st, st + cnt, B->last.begin());
+  if (*(int *)B->back) return set_err(XCS_EHIP, "team barrier timed out (results invalid)");
   return XCS_OK;
 }
 
@@ -1745,14 +1779,52 @@ static int batch_run_adaptive(xcs_batch *B, float *ms) {
   (void)hipEventDestroy(e1);
   std::vector<int> sw((size_t)SCHED_WORDS);
   HIP_TRY(d2h(sw.data(), B->sw, sizeof(int) * sw.size(), B->stream));
-  HIP_TRY(d2h(B->last.data(), B->sts, sizeof(XState) * B->count, B->stream));
-  XCS_TRY(batch_check_abort(B));
+  XCS_TRY(batch_states(B, B->count));
   if (sw[SW_ABORT * SCHED_LINE]) return set_err(XCS_EHIP, "scheduler wait timed out (results invalid)");
   B->phase_instances.assign(1, B->count);
   for (int l = 1; l < levels; l++) B->phase_instances.push_back(sw[(SW_TAIL + l) * SCHED_LINE]);
   B->phase_instances.push_back(lv.split_c >= 2 ? sw[(SW_TAIL + levels) * SCHED_LINE] : 0);
   if (ms) *ms = B->last_ms;
   return XCS_OK;
+}
+
+// Algorithmic bytes of one product of queue slot q's instance.
+static double batch_bytes1(const xcs_batch *B, int q) {
+  const XProblem &P = B->hP[q];
+  return P.ens == ENS_GEN ? 4.0 * P.lda * (double)P.n : P.ens == ENS_SMV ? 8.0 * P.nz : 24.0 * P.n;
+}
+
+// One solve on the configured geometry (teams of c for the n_big largest, no
+// tail schedule), in larger teams where the chip has room for them.  A workgroup
+// streams about 100 GB/s, so a large instance on a few workgroups takes long after
+// the others are done.  Teams of twice the size are taken, again and again,
+// while every large instance still has its team at once, a workgroup keeps GROW_BYTES
+// a product (below that the team's barriers take the time) and the longest wait
+// shrinks: the bytes a workgroup streams for the largest instance and, where the
+// other instances can't all run beside the teams, for the largest of those after it.
+// Measured on MI355X, ms per solve before and after: instances of both ensembles, n =
+// 1024 to 8192, the largest quarter in teams of 4, CGIHT: 256 of them 21.0 -> 16.6, 128
+// 14.7 -> 10.5, 64 9.4 -> 4.2, 16 5.6 -> 3.6; 20 of 2048 x 8192 in teams of 4 16.2 -> 7.4.
+constexpr double GROW_BYTES = 2e6;
+static int batch_run_teams(xcs_batch *B) {
+  const int big = B->n_big, small = B->count - big;
+  double most = 0.0, most1 = 0.0;
+  for (int q = 0; q < big; q++) most = std::max(most, batch_bytes1(B, q));
+  for (int q = big; q < B->count; q++) most1 = std::max(most1, batch_bytes1(B, q));
+  int c = B->c, grid = B->grid;
+  double wait = 0.0;
+  for (int d = B->c; d <= std::min(B->resident, BAR_MAX_TEAM) && (d == B->c || most / d >= GROW_BYTES); d *= 2) {
+    const int teams = batch_teams(B, big + (small + d - 1) / d, d);
+    const double w = most / d + ((long)teams * d >= (long)big * d + small ? 0.0 : most1);
+    if (d > B->c && teams < big) break;
+    if (d > B->c && w >= wait) continue;
+    wait = w;
+    if (d > B->c) {
+      c = d;
+      grid = teams * d;
+    }
+  }
+  return batch_enqueue(B, B->budget, c, grid);
 }
 
 static int batch_run(xcs_batch *B, float *ms) {
@@ -1764,15 +1836,15 @@ static int batch_run(xcs_batch *B, float *ms) {
   HIP_TRY(hipEventRecord(e0, B->stream));
   if (B->graph) {
     HIP_TRY(hipGraphLaunch(B->graph, B->stream));
+  } else if (B->c > 1 && B->sched_budget.empty() && B->n_big > 0) {
+    XCS_TRY(batch_run_teams(B));
   } else {
     XCS_TRY(batch_enqueue(B, B->sched_budget.empty() ? B->budget : B->sched_budget[0]));
   }
   B->phase_instances.assign(1, B->count);
   // the tail schedule: the instances still running go to larger teams
   for (size_t ph = 1; ph < B->sched_budget.size(); ph++) {
-    XCS_TRY(batch_check_abort(B));
-    HIP_TRY(d2h(B->last.data(), B->sts, sizeof(XState) * B->count, B->stream));
-    HIP_TRY(hipStreamSynchronize(B->stream));
+    XCS_TRY(batch_states(B, B->count));
     std::vector<int> run;
     for (int q = 0; q < B->count; q++)
       if (!B->last[q].done) run.push_back(q);
@@ -1787,8 +1859,7 @@ static int batch_run(xcs_batch *B, float *ms) {
   HIP_TRY(hipEventElapsedTime(&B->last_ms, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  HIP_TRY(d2h(B->last.data(), B->sts, sizeof(XState) * B->count, B->stream));
-  XCS_TRY(batch_check_abort(B));
+  XCS_TRY(batch_states(B, B->count));
   if (ms) *ms = B->last_ms;
   return XCS_OK;
 }
