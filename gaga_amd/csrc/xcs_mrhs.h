@@ -1099,7 +1099,8 @@ struct xcs_mrhs {
   float *A32 = nullptr, *A32b = nullptr, *cs = nullptr;
   uint8_t *a16cm = nullptr, *a16rm = nullptr, *a8cm = nullptr, *a8rm = nullptr;
   std::vector<void *> allocs;
-  std::vector<std::vector<float>> x_true;
+  std::vector<int> sup_true;     // the planted signals, k entries each (written out on request:
+  std::vector<float> val_true;   // dense they are 33 MB for 512 of 16384, 5 ms of first touches)
   int lp_iters[3] = {0, 0, 0};
   float last_ms = 0.f, gen_ms = 0.f;
   int *h_nactive = nullptr;  // pinned
@@ -1114,6 +1115,10 @@ struct xcs_mrhs {
     for (void *q : allocs) (void)hipFree(q);
     if (h_nactive) (void)hipHostFree(h_nactive);
     if (stream) (void)hipStreamDestroy(stream);
+  }
+  void planted(int s, float *out) const {
+    std::fill(out, out + n, 0.f);
+    for (size_t e = (size_t)s * k; e < (size_t)(s + 1) * k; e++) out[sup_true[e]] = val_true[e];
   }
   template <class T>
   int alloc(T **q, size_t cnt) {
@@ -1328,14 +1333,10 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
     XCS_TRY(device_draws(h->stream, jobs, dj, plants, dp));
   }
   {
-    std::vector<float> vals(S * k);
-    std::vector<int> sup_all(S * k);
-    HIP_TRY(d2h(vals.data(), d_vals, 4 * vals.size(), nullptr));
-    HIP_TRY(d2h(sup_all.data(), d_sup, 4 * sup_all.size(), nullptr));
-    h->x_true.assign(S, std::vector<float>((size_t)n, 0.f));
-    for (int s = 0; s < count; s++)
-      for (int c = 0; c < k; c++)
-        h->x_true[s][sup_all[(size_t)s * k + c]] = vals[(size_t)s * k + c];
+    h->val_true.resize(S * k);
+    h->sup_true.resize(S * k);
+    HIP_TRY(d2h(h->val_true.data(), d_vals, 4 * S * k, nullptr));
+    HIP_TRY(d2h(h->sup_true.data(), d_sup, 4 * S * k, nullptr));
   }
   hipLaunchKernelGGL(mr_make_y_kernel, dim3(count), dim3(MR_THREADS), 0, h->stream, h->A32, m,
                      d_vals, d_sup, k, y);
@@ -1533,13 +1534,17 @@ int xcs_mrhs_results(xcs_mrhs *h, float *norms, int *iterations, double *resid_r
   std::vector<double> ref(4 * S);
   HIP_TRY(d2h(st.data(), h->D.st, sizeof(XState) * S, nullptr));
   HIP_TRY(d2h(ref.data(), h->D.ref, sizeof(double) * 4 * S, nullptr));
-  std::vector<float> x;
+  std::vector<float> x, xt;
   if (norms) {
     x.resize(S * n);
+    xt.resize(n);
     HIP_TRY(d2h(x.data(), h->D.x, sizeof(float) * S * n, nullptr));
   }
   for (size_t s = 0; s < S; s++) {
-    if (norms) host_norms(h->x_true[s], x.data() + s * n, h->k, norms + 3 * s, nullptr);
+    if (norms) {
+      h->planted((int)s, xt.data());
+      host_norms(xt, x.data() + s * n, h->k, norms + 3 * s, nullptr);
+    }
     if (iterations) iterations[s] = st[s].iter;
     if (resid_rel) resid_rel[s] = ref[4 * s + 2] > 0 ? sqrt(ref[4 * s + 1] / ref[4 * s + 2]) : 0.0;
   }
@@ -1549,7 +1554,7 @@ int xcs_mrhs_results(xcs_mrhs *h, float *norms, int *iterations, double *resid_r
 int xcs_mrhs_x(xcs_mrhs *h, int s, float *x_out, float *x_true, float *y) {
   if (!h || s < 0 || s >= h->count) return set_err(XCS_EINVAL, "bad signal index");
   HIP_TRY(hipSetDevice(h->dev));
-  if (x_true) memcpy(x_true, h->x_true[s].data(), 4 * (size_t)h->n);
+  if (x_true) h->planted(s, x_true);
   float *const out[2] = {x_out, y};
   auto piece = [h](int i, int p, const float **src, long *n) {
     *src = p ? h->D.y + (size_t)i * h->m : h->D.x + (size_t)i * h->n;
@@ -1615,7 +1620,7 @@ int xcs_mrhs_fp32_solve(xcs_mrhs *h, int first, int cnt, int mode, float *ms_tot
   XCS_TRY(plan_alloc(&pl, ALG_CGIHT, ENS_GEN, h->k, h->m, h->n, 0, 0, &o));
   if (pl.h.lda != h->m) return set_err(XCS_EINVAL, "internal: leading dimension");
   xset(pl.h.A, h->A32);
-  std::vector<float> x((size_t)h->n);
+  std::vector<float> x((size_t)h->n), xt((size_t)h->n);
   float total = 0.f;
   for (int q = 0; q < cnt; q++) {
     const int s = first + q;
@@ -1624,7 +1629,10 @@ int xcs_mrhs_fp32_solve(xcs_mrhs *h, int first, int cnt, int mode, float *ms_tot
     XCS_TRY(plan_run(&pl, &ms));
     total += ms;
     HIP_TRY(d2h(x.data(), pl.h.x, 4 * (size_t)h->n, nullptr));
-    if (norms) host_norms(h->x_true[s], x.data(), h->k, norms + 3 * (size_t)q, nullptr);
+    if (norms) {
+      h->planted(s, xt.data());
+      host_norms(xt, x.data(), h->k, norms + 3 * (size_t)q, nullptr);
+    }
     if (iterations) iterations[q] = pl.last.iter;
   }
   *ms_total = total;
