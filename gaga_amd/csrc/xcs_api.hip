@@ -780,7 +780,8 @@ static int plan_alloc(xcs_plan *pl, int alg, int ens, int k, int m, int n, int p
   XCS_TRY(max_coop_blocks(pl->block, &maxb));
   int team = o->team_size;
   if (team <= 0) {
-    // Bandwidth grows with the team, and so does the cost of its barriers
+    // The general form's team (solve_coop_kernel; plan_resident and plan_split
+    // choose their own).  Bandwidth grows with the team, and so does the cost of its barriers
     // (8-10 team barriers or reductions per iteration).  Teams in proportion
     // to the bytes one product streams, capped where the measured optima on
     // MI355X (512-thread workgroups, CGIHT and NIHT) lie: gen 2048 x 8192 at

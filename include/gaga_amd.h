@@ -206,7 +206,9 @@ int xcs_batch_create(const char *alg, int count, const int *ens, const int *k, c
 int xcs_batch_solve(xcs_batch *batch, float *ms);
 /* Change the team geometry: team_size workgroups of block_size threads per instance for the
  * big_count largest instances (big_count < 0: all of them); the rest run one per workgroup
- * once those are taken.  Recovery does not depend on it (reduction order does). */
+ * once those are taken.  Without a tail schedule a solve takes teams of twice, four times, ...
+ * team_size where the chip has room for all of them at once.  Recovery does not depend on
+ * the geometry (reduction order does). */
 int xcs_batch_configure(xcs_batch *batch, int team_size, int block_size, int big_count);
 /* Tail schedule (no counterpart in the reference, whose sweep driver runs one problem per
  * call): phase 0 solves every instance on the configured geometry for at most budgets[0]
