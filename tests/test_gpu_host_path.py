@@ -99,3 +99,19 @@ def test_given_problems_from_more_threads_than_idle_lanes():
     [t.join() for t in th]
     for i, q in enumerate(probs):
         assert all(np.array_equal(g, want[i]) for g in got[i]), i
+
+
+@pytest.mark.parametrize("n", [1 << 12, 1 << 16, 1 << 17])  # with the staging memory, its last size, past it
+def test_given_problem_solutions_of_every_length(n):
+    from gaga_amd import _capi
+    rng = np.random.default_rng(6)
+    m, k = n // 4, n // 256
+    rows = np.sort(rng.choice(n, m, replace=False)).astype(np.int32)
+    x = np.zeros(n, np.float32)
+    x[rng.choice(n, k, replace=False)] = rng.choice([-1.0, 1.0], k)
+    y = _capi.apply("dct", 0, m, n, x, dct_rows=rows)
+    got, iters, _ = ga.cs("NIHT", "dct", y, rows + 1, k, m, n, ga.options(tol=1e-5))
+    # stops at |r| <= tol; the smallest singular value on 2k columns is above 1 / 4 here
+    # (a quarter of the rows of an orthogonal matrix, scale 1 / 2)
+    assert np.linalg.norm(got - x) <= 8e-5 and iters > 0
+    assert set(np.flatnonzero(np.abs(got) > 0.5)) == set(np.flatnonzero(x))
