@@ -869,14 +869,33 @@ static int launch_apply(xcs_plan *pl, int transpose, const float *in, float *out
   return XCS_OK;
 }
 
-// y = A x for a device x whose support list (cnt entries) is d_supp.
+// y = A x for a device x whose support list (cnt entries, ascending) is d_supp, by the
+// product the plan's solves use.
 static int plan_make_y(xcs_plan *pl, const int *d_supp, int cnt, const float *d_x, float *d_y) {
   XProblem &P = pl->h;
   if (cnt)
     HIP_TRY(hipMemcpyAsync((int *)P.supp, d_supp, sizeof(int) * cnt, hipMemcpyDeviceToDevice,
                            pl->stream));
   XCS_TRY(plan_upload_desc(pl));
-  XCS_TRY(launch_apply(pl, 0, d_x, d_y, cnt));
+  if (pl->kernel && P.ens == ENS_GEN) {
+    if (pl->block <= 512)
+      hipLaunchKernelGGL(resident_y_kernel<512>, dim3(pl->team), dim3(pl->block), 0, pl->stream,
+                         (const XProblem *)pl->d, d_x, cnt, d_y);
+    else
+      hipLaunchKernelGGL(resident_y_kernel<1024>, dim3(pl->team), dim3(pl->block), 0, pl->stream,
+                         (const XProblem *)pl->d, d_x, cnt, d_y);
+    HIP_TRY(hipGetLastError());
+  } else if (pl->kernel) {
+    HIP_TRY(hipMemsetAsync(pl->bar, 0, sizeof(unsigned) * BAR_WORDS, pl->stream));
+    long limit = BAR_SPIN_LIMIT;
+    int alg = P.alg;
+    void *args[] = {(void *)&pl->d, (void *)&alg, (void *)&d_x, (void *)&d_y, (void *)&pl->bar, (void *)&limit};
+    const void *kernel = P.ens == ENS_DCT ? (const void *)split_y_kernel<ENS_DCT>
+                                          : (const void *)split_y_kernel<ENS_SMV>;
+    HIP_TRY(hipLaunchCooperativeKernel(kernel, dim3(pl->team), dim3(pl->block), args, 0, pl->stream));
+  } else {
+    XCS_TRY(launch_apply(pl, 0, d_x, d_y, cnt));
+  }
   HIP_TRY(hipStreamSynchronize(pl->stream));
   return XCS_OK;
 }

@@ -305,12 +305,9 @@ __device__ __forceinline__ void rt_allreduce(RTeam &t, RtSlots &X, const double 
 }
 
 // ------------------------------------------------------------ the state ----
-// The residual history of the stop rules, entry i in lane i < 16 of every wave
-// (each wave keeps its own copy: pushes and the rules are a few DPP moves and
-// ballots, uniform, without barriers).
-struct ResHist {
-  float prev, evo;  // lane i: prev[i], evo[i]
-};
+// The residual history of the stop rules is kept with entry i in lane i < 16 of
+// every wave (each wave keeps its own copy: pushes and the rules are a few DPP
+// moves and ballots, uniform, without barriers).
 __device__ __forceinline__ float hist_push(float h, float v) {
   const int lane = threadIdx.x & (WAVE - 1);
   const float nx = __shfl_down(h, 1);
@@ -1061,6 +1058,38 @@ __global__ void __launch_bounds__(MAXT) solve_resident_kernel(const XProblem *Pp
       bar[1] = t.tag;
     }
   }
+}
+
+// y = A x of a generated instance (x in memory, its support ascending in P.supp)
+// by the solve's own product in the solve's geometry, so that the planted vector
+// leaves no residual: with y from the general form's product, whose sums round
+// differently, a solve cannot come below about ||y|| 2^-23 (CGIHT 1024 x 4096: 7e-7
+// of 7).  One launch of the team, no exchanges.
+template <int MAXT>
+__global__ void __launch_bounds__(MAXT) resident_y_kernel(const XProblem *Pp, const float *x, int cnt,
+                                                          float *y) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RES_LDS];
+  __shared__ XProblem sP;
+  __shared__ float tile[2][RES_TCAP];
+  __shared__ __attribute__((aligned(16))) float wsum[2 * 4 * MAX_WAVES][4 * RES_QB];
+  if (threadIdx.x == 0) sP = *Pp;
+  __syncthreads();
+  const XProblem &P = sP;
+  Res R;
+  R.x = (float *)lds;
+  R.list = (unsigned short *)(lds + res_up16(4 * (size_t)P.n));
+  R.tile = tile;
+  R.wsum = wsum;
+  R.cnt = cnt;
+  res_rows(blockIdx.x, gridDim.x, P.lda, &R.row0, &R.rows);
+  for (int s = threadIdx.x; s < cnt; s += blockDim.x) {
+    const int j = P.supp[s];
+    R.list[s] = (unsigned short)j;
+    R.x[j] = x[j];
+  }
+  __syncthreads();
+  res_gather<1>(R, P.A, P.lda, R.x, nullptr);
+  for (int i = threadIdx.x; i < R.rows; i += blockDim.x) y[R.row0 + i] = tile[0][i];
 }
 
 }  // namespace xcs

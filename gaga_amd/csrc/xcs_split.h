@@ -922,25 +922,20 @@ __device__ __forceinline__ float sp_cg_projection(RTeam &t, Sp &R, const XProble
   return errCG;
 }
 
-// One instance by the whole (cooperatively launched) grid: at most `budget`
-// outer iterations from the saved state.
-template <int ENS, int ALG>
-__global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem *Pp, int budget,
-                                                                 unsigned *bar, long spin_limit) {
-  typedef SpOp<ENS> Op;
-  constexpr bool CG = ALG == ALG_CGIHT;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[SP_LDS];
-  __shared__ XProblem sP;
-  __shared__ WgSlots slots;
-  __shared__ RtSlots rt;
-  if (threadIdx.x == 0) sP = *Pp;
-  __syncthreads();
-  const XProblem &P = sP;
-  if (P.st->done) return;
+// Index of element i of the n-slice in the caller's vectors.
+template <int ENS>
+__device__ __forceinline__ int sp_column(const Sp &R, const RTeam &t, int n, int i) {
+  if (ENS != ENS_DCT) return R.j0 + i;
+  const int z = sp_time(R, t.rank, t.size, i);
+  return z < n / 2 ? 2 * z : 2 * (n - 1 - z) + 1;
+}
+// The workgroup's slices in LDS for an instance of `alg`, with y (slots and rt are
+// the kernel's own); the smv entries are staged by the solve.
+template <int ENS>
+__device__ __forceinline__ SplitGeom sp_open(Sp &R, const RTeam &t, const XProblem &P, int alg,
+                                             unsigned char *lds) {
   const int lane = threadIdx.x & (WAVE - 1), nt = blockDim.x, n = P.n;
-  RTeam t{(int)blockIdx.x, (int)gridDim.x, bar, bar[1], spin_limit, 0};
-  const SplitGeom G = split_geom(ENS, ALG, P.m, n, P.log2n, P.num_bins, t.size);
-  Sp R;
+  const SplitGeom G = split_geom(ENS, alg, P.m, n, P.log2n, P.num_bins, t.size);
   {
     unsigned char *q = lds;
     auto take = [&](size_t b) {
@@ -955,7 +950,7 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
     R.x = (float *)take(4 * (size_t)G.nl);
     R.g = (float *)take(4 * (size_t)G.nl);
     R.p = (float *)take(4 * (size_t)G.nl);
-    R.q = ALG == ALG_HTP ? (float *)take(4 * (size_t)G.nl) : nullptr;
+    R.q = alg == ALG_HTP ? (float *)take(4 * (size_t)G.nl) : nullptr;
     R.y = (float *)take(4 * (size_t)G.rl);
     R.t0 = (float *)take(4 * (size_t)G.rl);
     R.t1 = (float *)take(4 * (size_t)G.rl);
@@ -981,20 +976,12 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
   R.lvals = nullptr;
   R.rbase = 0;
   if (G.filter) R.fmask = (unsigned long long *)(lds + G.lds);
-  R.slots = &slots;
-  R.rt = &rt;
   R.bank = R.par = R.mid = 0;
   // slices: smv contiguous columns and rows, dct the owned packed slots
   R.j0 = min(n, t.rank * G.nl);
   R.i0 = min(P.m, t.rank * G.rl);
   R.nlv = ENS == ENS_DCT ? G.nl : min(G.nl, n - R.j0);
   R.rlv = ENS == ENS_DCT ? G.rl : min(G.rl, P.m - R.i0);
-  // index of element i of the n-slice in the caller's vectors
-  auto column = [&](int i) {
-    if (ENS != ENS_DCT) return R.j0 + i;
-    const int z = sp_time(R, t.rank, t.size, i);
-    return z < n / 2 ? 2 * z : 2 * (n - 1 - z) + 1;
-  };
   if (ENS == ENS_DCT) {
     for (int j0 = 0; j0 < R.rl; j0 += nt) {
       const int i = j0 + threadIdx.x;
@@ -1010,6 +997,31 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
   } else {
     for (int i = threadIdx.x; i < R.rlv; i += nt) R.y[i] = P.y[R.i0 + i];
   }
+  return G;
+}
+
+// One instance by the whole (cooperatively launched) grid: at most `budget`
+// outer iterations from the saved state.
+template <int ENS, int ALG>
+__global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem *Pp, int budget,
+                                                                 unsigned *bar, long spin_limit) {
+  typedef SpOp<ENS> Op;
+  constexpr bool CG = ALG == ALG_CGIHT;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[SP_LDS];
+  __shared__ XProblem sP;
+  __shared__ WgSlots slots;
+  __shared__ RtSlots rt;
+  if (threadIdx.x == 0) sP = *Pp;
+  __syncthreads();
+  const XProblem &P = sP;
+  if (P.st->done) return;
+  const int lane = threadIdx.x & (WAVE - 1), nt = blockDim.x, n = P.n;
+  RTeam t{(int)blockIdx.x, (int)gridDim.x, bar, bar[1], spin_limit, 0};
+  Sp R;
+  const SplitGeom G = sp_open<ENS>(R, t, P, ALG, lds);
+  R.slots = &slots;
+  R.rt = &rt;
+  auto column = [&](int i) { return sp_column<ENS>(R, t, n, i); };
   if (ENS == ENS_SMV && G.filter) {
     // the matrix entries do not change during a solve: what LDS has left takes the
     // own rows' columns, then the own columns' rows and values
@@ -1318,6 +1330,46 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
       st->diff = Q.diff;
       st->mat_bytes = S.bytes;
       bar[1] = t.tag;
+    }
+  }
+}
+
+// y = A x of a generated instance (x in memory) by the solve's own product in the
+// solve's geometry (see resident_y_kernel): the planted vector leaves no residual.
+// dct 2^20, m = 2^18 + 1: with the general form's y an NIHT solve to 1e-5 stalled at
+// 1.15e-5 for 32 iterations, with this one it takes 18.
+template <int ENS>
+__global__ void __launch_bounds__(SP_THREADS) split_y_kernel(const XProblem *Pp, int alg, const float *x,
+                                                             float *y, unsigned *bar, long spin_limit) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[SP_LDS];
+  __shared__ XProblem sP;
+  __shared__ WgSlots slots;
+  __shared__ RtSlots rt;
+  if (threadIdx.x == 0) sP = *Pp;
+  __syncthreads();
+  const XProblem &P = sP;
+  const int n = P.n;
+  RTeam t{(int)blockIdx.x, (int)gridDim.x, bar, bar[1], spin_limit, 0};
+  Sp R;
+  (void)sp_open<ENS>(R, t, P, alg, lds);
+  R.slots = &slots;
+  R.rt = &rt;
+  for (int j0 = 0; j0 < R.nl; j0 += blockDim.x) {
+    const int i = j0 + threadIdx.x;
+    const float v = i < R.nlv ? x[sp_column<ENS>(R, t, n, i)] : 0.f;
+    if (i < R.nl) R.x[i] = v;
+    const unsigned long long bits = __ballot(v != 0.f);
+    if ((threadIdx.x & (WAVE - 1)) == 0 && i < R.nl) R.mask[i >> 6] = bits;
+  }
+  __syncthreads();
+  double z[1] = {0.0};
+  SpOp<ENS>::template A<1, 0>(t, R, P, R.x, false, nullptr, false, R.t0, nullptr, z, z);
+  for (int i = threadIdx.x; i < R.rlv; i += blockDim.x) {
+    if (ENS == ENS_DCT) {
+      const int k = sp_coef(R, t.rank, t.size, i >> 1), pos = P.dct_pos[(i & 1) ? (k ? n - k : n >> 1) : k];
+      if (pos >= 0) y[pos] = R.t0[i];
+    } else {
+      y[R.i0 + i] = R.t0[i];
     }
   }
 }
