@@ -50,6 +50,8 @@ constexpr int SP_LDS = 150 * 1024;    // bytes of LDS for the slices and tables
 constexpr int SP_HIST = 4096;         // histogram bins held in LDS
 constexpr int SP_PAD = 64;            // slices of n-vectors: multiples of a wave
 
+// Twiddles of a length-2^b transform held in LDS: what its radix-4 butterflies read.
+__host__ __device__ inline size_t sp_twiddles(int b) { return b < 2 ? 1 : (size_t)3 << (b - 2); }
 // Histogram bins held in LDS: all of them or none.
 __host__ __device__ inline int sp_hist(int num_bins) { return num_bins <= SP_HIST ? num_bins : 0; }
 // Layout of an instance over `size` workgroups.
@@ -68,7 +70,7 @@ __host__ __device__ inline SplitGeom split_geom(int ens, int alg, int m, int n, 
     G.b1 = ln / 2;
     G.b2 = ln - G.b1;
     G.nl = G.rl = n / size;
-    G.lds = res_up16(8 * ((size_t)1 << G.b1) / 2) + res_up16(8 * ((size_t)1 << G.b2) / 2) +
+    G.lds = res_up16(8 * sp_twiddles(G.b1)) + res_up16(8 * sp_twiddles(G.b2)) +
             res_up16((size_t)G.rl / 8 + 8);
   } else {
     G.nl = ((n + size - 1) / size + SP_PAD - 1) / SP_PAD * SP_PAD;
@@ -101,7 +103,7 @@ struct Sp {
   int *hist;                   // zero between uses
   unsigned long long *mask;    // support bits of the n-slice
   unsigned long long *rmask;   // dct: sampled bits of the m-slice
-  const float2 *w1, *w2;       // dct: w_N1^k and w_N2^k, k < half
+  const float2 *w1, *w2;       // dct: w_N1^k and w_N2^k, k < 3/4 of the length
   WgSlots *slots;
   RtSlots *rt;
   int bank, par;               // wg_reduce bank, histogram parity
@@ -310,28 +312,47 @@ template <int SIGN>
 __device__ __forceinline__ float2 sp_tw(float2 w) {  // tables hold the forward sign
   return SIGN > 0 ? make_float2(w.x, -w.y) : w;
 }
+// Radix-4 butterflies (three twiddle products for four points where two radix-2
+// stages take four) and fused multiply-adds (two roundings a component where
+// separate products take three): the packed transform passes over the spectrum once
+// more than the general form's (xcs_fft.h), and with that form's butterflies its
+// products came out 4-5% further from 64 bits than they; with these 5-10% nearer,
+// and their projection on the support, which is what reaches x, 12-27% nearer.
+__device__ __forceinline__ float2 sp_cmul(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -__fmul_rn(a.y, b.y)), fmaf(a.x, b.y, __fmul_rn(a.y, b.x)));
+}
+__device__ __forceinline__ float2 sp_add(float2 a, float2 b) {
+  return make_float2(__fadd_rn(a.x, b.x), __fadd_rn(a.y, b.y));
+}
+__device__ __forceinline__ float2 sp_sub(float2 a, float2 b) {
+  return make_float2(__fsub_rn(a.x, b.x), __fsub_rn(a.y, b.y));
+}
+// a + s i b with s = SIGN (the quarter turn of the transform's direction).
+template <int SIGN>
+__device__ __forceinline__ float2 sp_turn(float2 a, float2 b) {
+  return SIGN > 0 ? make_float2(__fsub_rn(a.x, b.y), __fadd_rn(a.y, b.x))
+                  : make_float2(__fadd_rn(a.x, b.y), __fsub_rn(a.y, b.x));
+}
 // cnt sequences of length 2^lb, contiguous in f, in place: decimation in time
-// from bit-reversed to natural order, two radix-2 stages per LDS pass.
+// from bit-reversed to natural order.
 template <int SIGN>
 __device__ __forceinline__ void sp_dit(float2 *f, const float2 *tw, int lb, int cnt) {
   const int len = 1 << lb;
   int lh = 0;
   for (; lh + 2 <= lb; lh += 2) {
-    const int h = 1 << lh, lq = lb - 2;
-    const int s1 = len >> (lh + 1), s2 = len >> (lh + 2);
+    const int h = 1 << lh, lq = lb - 2, s2 = len >> (lh + 2);
     for (int b = threadIdx.x; b < (cnt << lq); b += blockDim.x) {
       const int sq = b >> lq, bb = b & ((1 << lq) - 1);
       const int pos = bb & (h - 1), base = (sq << lb) + ((bb >> lh) << (lh + 2)) + pos;
-      float2 x0 = f[base], x1 = f[base + h], x2 = f[base + 2 * h], x3 = f[base + 3 * h];
-      const float2 wa = sp_tw<SIGN>(tw[pos * s1]);
-      bfly(x0, x1, wa);
-      bfly(x2, x3, wa);
-      bfly(x0, x2, sp_tw<SIGN>(tw[pos * s2]));
-      bfly(x1, x3, sp_tw<SIGN>(tw[(pos + h) * s2]));
-      f[base] = x0;
-      f[base + h] = x1;
-      f[base + 2 * h] = x2;
-      f[base + 3 * h] = x3;
+      const int e = pos * s2;
+      const float2 x0 = f[base], t1 = sp_cmul(f[base + h], sp_tw<SIGN>(tw[2 * e]));
+      const float2 t2 = sp_cmul(f[base + 2 * h], sp_tw<SIGN>(tw[e]));
+      const float2 t3 = sp_cmul(f[base + 3 * h], sp_tw<SIGN>(tw[3 * e]));
+      const float2 u = sp_add(x0, t1), v = sp_sub(x0, t1), c = sp_add(t2, t3), d = sp_sub(t2, t3);
+      f[base] = sp_add(u, c);
+      f[base + h] = sp_turn<SIGN>(v, d);
+      f[base + 2 * h] = sp_sub(u, c);
+      f[base + 3 * h] = sp_turn<-SIGN>(v, d);
     }
     __syncthreads();
   }
@@ -339,19 +360,12 @@ __device__ __forceinline__ void sp_dit(float2 *f, const float2 *tw, int lb, int 
     const int h = 1 << lh;
     for (int b = threadIdx.x; b < (cnt << lh); b += blockDim.x) {
       const int sq = b >> lh, pos = b & (h - 1), i0 = (sq << lb) + pos;
-      float2 u = f[i0], v = f[i0 + h];
-      bfly(u, v, sp_tw<SIGN>(tw[pos]));
-      f[i0] = u;
-      f[i0 + h] = v;
+      const float2 u = f[i0], v = sp_cmul(f[i0 + h], sp_tw<SIGN>(tw[pos]));
+      f[i0] = sp_add(u, v);
+      f[i0 + h] = sp_sub(u, v);
     }
     __syncthreads();
   }
-}
-// Decimation-in-frequency butterfly: (u, v) -> (u + v, (u - v) w).
-__device__ __forceinline__ void bflyf(float2 &u, float2 &v, float2 w) {
-  const float2 d = make_float2(__fsub_rn(u.x, v.x), __fsub_rn(u.y, v.y));
-  u = make_float2(__fadd_rn(u.x, v.x), __fadd_rn(u.y, v.y));
-  v = cmul(d, w);
 }
 // The same from natural to bit-reversed order: decimation in frequency.
 template <int SIGN>
@@ -363,29 +377,25 @@ __device__ __forceinline__ void sp_dif(float2 *f, const float2 *tw, int lb, int 
     lh--;
     for (int b = threadIdx.x; b < (cnt << lh); b += blockDim.x) {
       const int sq = b >> lh, pos = b & (h - 1), i0 = (sq << lb) + pos;
-      float2 u = f[i0], v = f[i0 + h];
-      bflyf(u, v, sp_tw<SIGN>(tw[pos]));
-      f[i0] = u;
-      f[i0 + h] = v;
+      const float2 u = f[i0], v = f[i0 + h];
+      f[i0] = sp_add(u, v);
+      f[i0 + h] = sp_cmul(sp_sub(u, v), sp_tw<SIGN>(tw[pos]));
     }
     __syncthreads();
   }
   for (; lh >= 2; lh -= 2) {
     const int l2 = lh - 2, h = 1 << l2, lq = lb - 2;  // spans 2h, then h
-    const int s1 = len >> (l2 + 2), s2 = len >> (l2 + 1);
+    const int s1 = len >> (l2 + 2);
     for (int b = threadIdx.x; b < (cnt << lq); b += blockDim.x) {
       const int sq = b >> lq, bb = b & ((1 << lq) - 1);
       const int pos = bb & (h - 1), base = (sq << lb) + ((bb >> l2) << lh) + pos;
-      float2 x0 = f[base], x1 = f[base + h], x2 = f[base + 2 * h], x3 = f[base + 3 * h];
-      bflyf(x0, x2, sp_tw<SIGN>(tw[pos * s1]));
-      bflyf(x1, x3, sp_tw<SIGN>(tw[(pos + h) * s1]));
-      const float2 wa = sp_tw<SIGN>(tw[pos * s2]);
-      bflyf(x0, x1, wa);
-      bflyf(x2, x3, wa);
-      f[base] = x0;
-      f[base + h] = x1;
-      f[base + 2 * h] = x2;
-      f[base + 3 * h] = x3;
+      const int e = pos * s1;
+      const float2 x0 = f[base], x1 = f[base + h], x2 = f[base + 2 * h], x3 = f[base + 3 * h];
+      const float2 u = sp_add(x0, x2), v = sp_sub(x0, x2), c = sp_add(x1, x3), d = sp_sub(x1, x3);
+      f[base] = sp_add(u, c);
+      f[base + h] = sp_cmul(sp_sub(u, c), sp_tw<SIGN>(tw[2 * e]));
+      f[base + 2 * h] = sp_cmul(sp_turn<SIGN>(v, d), sp_tw<SIGN>(tw[e]));
+      f[base + 3 * h] = sp_cmul(sp_turn<-SIGN>(v, d), sp_tw<SIGN>(tw[3 * e]));
     }
     __syncthreads();
   }
@@ -525,8 +535,8 @@ struct SpOp<ENS_DCT> {
       const int cl = e & (cb - 1), k1 = e >> lcb, c = c0 + cl;
       const float2 w = tw[(2 * c * k1) & (n - 1)];
       const size_t at = ((size_t)k1 << R.b2) + c;
-      st_dev2(buf(P, R.mid, 0) + at, cmul(((float2 *)d0)[(cl << R.b1) + k1], w));
-      if (NV == 2) st_dev2(buf(P, R.mid, 1) + at, cmul(((float2 *)d1)[(cl << R.b1) + k1], w));
+      st_dev2(buf(P, R.mid, 0) + at, sp_cmul(((float2 *)d0)[(cl << R.b1) + k1], w));
+      if (NV == 2) st_dev2(buf(P, R.mid, 1) + at, sp_cmul(((float2 *)d1)[(cl << R.b1) + k1], w));
     }
     rt_allreduce<K, MAXES>(t, *R.rt, v, o);
     const int h = (N1 / t.size) >> 1;
@@ -557,8 +567,8 @@ struct SpOp<ENS_DCT> {
     auto put = [&](int e, float2 c, float2 q) {
       const unsigned long long bits = R.rmask[e >> 5] >> ((2 * e) & 63);
       f[e] = make_float2(
-          (bits & 1) ? __fmul_rn(w, __fadd_rn(__fmul_rn(c.x, q.x), __fmul_rn(c.y, q.y))) : 0.f,
-          (bits & 2) ? __fmul_rn(w, __fsub_rn(__fmul_rn(c.x, q.y), __fmul_rn(c.y, q.x))) : 0.f);
+          (bits & 1) ? __fmul_rn(w, fmaf(c.x, q.x, __fmul_rn(c.y, q.y))) : 0.f,
+          (bits & 2) ? __fmul_rn(w, fmaf(c.x, q.y, -__fmul_rn(c.y, q.x))) : 0.f);
     };
     sp_pairs(
         R, t.rank, t.size,
@@ -567,10 +577,11 @@ struct SpOp<ENS_DCT> {
           // E = (a + conj b) / 2, D = (a - conj b) / 2, C_k = E - i w_n^k D
           const float2 E = make_float2(0.5f * __fadd_rn(a.x, b.x), 0.5f * __fsub_rn(a.y, b.y));
           const float2 D = make_float2(0.5f * __fsub_rn(a.x, b.x), 0.5f * __fadd_rn(a.y, b.y));
-          const float2 u = cmul(tw[k], D);  // -i u = (u.y, -u.x)
-          put(ea, make_float2(__fadd_rn(E.x, u.y), __fsub_rn(E.y, u.x)), qw[k]);
+          const float2 c = tw[k];
+          put(ea, make_float2(fmaf(c.x, D.y, fmaf(c.y, D.x, E.x)), fmaf(-c.x, D.x, fmaf(c.y, D.y, E.y))), qw[k]);
           // C_{N-k} = conj(E + i w_n^k D)
-          put(eb, make_float2(__fsub_rn(E.x, u.y), -__fadd_rn(E.y, u.x)), qw[N - k]);
+          put(eb, make_float2(fmaf(-c.x, D.y, fmaf(-c.y, D.x, E.x)), -fmaf(c.x, D.x, fmaf(-c.y, D.y, E.y))),
+              qw[N - k]);
         },
         [&](int e) {
           const float2 a = f[e];
@@ -592,8 +603,8 @@ struct SpOp<ENS_DCT> {
     const float w0 = (float)sqrt(1.0 / (double)n), w = (float)sqrt(2.0 / (double)n);
     // H = w / 2 ((a cos + b sin) + i (a sin - b cos))
     auto half = [&](float2 d, float2 q) {
-      return make_float2(0.5f * __fmul_rn(w, __fadd_rn(__fmul_rn(d.x, q.x), __fmul_rn(d.y, q.y))),
-                         0.5f * __fmul_rn(w, __fsub_rn(__fmul_rn(d.x, q.y), __fmul_rn(d.y, q.x))));
+      return make_float2(0.5f * __fmul_rn(w, fmaf(d.x, q.x, __fmul_rn(d.y, q.y))),
+                         0.5f * __fmul_rn(w, fmaf(d.x, q.y, -__fmul_rn(d.y, q.x))));
     };
     sp_pairs(
         R, t.rank, t.size,
@@ -601,10 +612,9 @@ struct SpOp<ENS_DCT> {
           const float2 a = half(f[ea], qw[k]), b = half(f[eb], qw[N - k]);
           const float2 S = make_float2(__fadd_rn(a.x, b.x), __fsub_rn(a.y, b.y));
           const float2 D = make_float2(__fsub_rn(a.x, b.x), __fadd_rn(a.y, b.y));
-          const float2 c = tw[k];
-          const float2 u = cmul(make_float2(c.x, -c.y), D);  // e^{2 pi i k / n} D
-          f[ea] = make_float2(__fsub_rn(S.x, u.y), __fadd_rn(S.y, u.x));   // S + i u
-          f[eb] = make_float2(__fadd_rn(S.x, u.y), __fsub_rn(u.x, S.y));   // conj S + i conj u
+          const float2 c = tw[k];  // u = e^{2 pi i k / n} D = conj(c) D
+          f[ea] = make_float2(fmaf(-c.x, D.y, fmaf(c.y, D.x, S.x)), fmaf(c.x, D.x, fmaf(c.y, D.y, S.y)));  // S + i u
+          f[eb] = make_float2(fmaf(c.x, D.y, fmaf(-c.y, D.x, S.x)), fmaf(c.x, D.x, fmaf(c.y, D.y, -S.y)));  // conj S + i conj u
         },
         [&](int e) {
           const float2 d = f[e];
@@ -635,7 +645,7 @@ struct SpOp<ENS_DCT> {
       const int r = sp_class(t.rank, h, a, N1);
       const float2 w = tw[(2 * r * q2) & (n - 1)];
       st_dev2(mid + ((size_t)q2 << R.b1) + t.rank * rb + a,
-              cmul(((float2 *)s)[(a << R.b2) + q2], make_float2(w.x, -w.y)));
+              sp_cmul(((float2 *)s)[(a << R.b2) + q2], make_float2(w.x, -w.y)));
     }
     rt_allreduce<K, MAXES>(t, *R.rt, v, o);
     for (int e = threadIdx.x; e < nc; e += blockDim.x) {
@@ -960,11 +970,11 @@ __device__ __forceinline__ SplitGeom sp_open(Sp &R, const RTeam &t, const XProbl
     R.w1 = R.w2 = nullptr;
     if (ENS == ENS_DCT) {
       R.rmask = (unsigned long long *)take((size_t)G.rl / 8 + 8);
-      float2 *w1 = (float2 *)take(8 * ((size_t)1 << G.b1) / 2);
-      float2 *w2 = (float2 *)take(8 * ((size_t)1 << G.b2) / 2);
-      for (int k = threadIdx.x; k < (1 << G.b1) / 2; k += nt)
+      float2 *w1 = (float2 *)take(8 * sp_twiddles(G.b1));
+      float2 *w2 = (float2 *)take(8 * sp_twiddles(G.b2));
+      for (int k = threadIdx.x; k < (int)sp_twiddles(G.b1); k += nt)
         w1[k] = P.twiddle[(size_t)k << (P.log2n - G.b1)];
-      for (int k = threadIdx.x; k < (1 << G.b2) / 2; k += nt)
+      for (int k = threadIdx.x; k < (int)sp_twiddles(G.b2); k += nt)
         w2[k] = P.twiddle[(size_t)k << (P.log2n - G.b2)];
       R.w1 = w1;
       R.w2 = w2;
@@ -1337,7 +1347,7 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
 // y = A x of a generated instance (x in memory) by the solve's own product in the
 // solve's geometry (see resident_y_kernel): the planted vector leaves no residual.
 // dct 2^20, m = 2^18 + 1: with the general form's y an NIHT solve to 1e-5 stalled at
-// 1.15e-5 for 32 iterations, with this one it takes 18.
+// 1.15e-5 for 32 iterations, with this one it takes 16.
 template <int ENS>
 __global__ void __launch_bounds__(SP_THREADS) split_y_kernel(const XProblem *Pp, int alg, const float *x,
                                                              float *y, unsigned *bar, long spin_limit) {

@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
     ("gen", 30, 700, 2001, 0, {"teamSize": 48}),
     ("smv", 300, 4000, 20000, 7, {}),
     ("dct", 100, 2049, 8192, 0, {}),
+    ("dct", 1000, 32769, 131072, 0, {}),
 ])
 def test_solves_below_the_rounding_of_y(lib, alg, ens, k, m, n, p, extra):
     kw = dict(extra, seed=77, maxiter=60)
@@ -36,7 +37,7 @@ def test_solves_below_the_rounding_of_y(lib, alg, ens, k, m, n, p, extra):
     assert err <= 4 * y * 2.0 ** -24
 
 
-@pytest.mark.parametrize("alg", ["NIHT", "HTP"])
+@pytest.mark.parametrize("alg", ["NIHT", "HTP", "CGIHT"])
 def test_large_transform_meets_its_tolerance(lib, alg):
     """1.7e-7 of ||y||: the general form's measurements left 1.15e-5 here."""
     pl = lib.Plan(alg, "dct", 13107, (1 << 18) + 1, 1 << 20, 0, lib.options(tol=1e-5, seed=77, maxiter=60))
