@@ -1220,7 +1220,7 @@ struct xcs_batch {
   std::vector<XState> last;
   std::vector<int> order;  // order[q] = caller index of queue slot q
   std::vector<int> slot_of;  // slot_of[i] = queue slot of caller index i
-  ReadAhead ahead;           // solution vectors read in order
+  PinnedReadAhead ahead;           // solution vectors read in order
   unsigned long long *phase = nullptr;  // XCS_PHASE_TIMING builds only
   float gen_ms = 0.f, last_ms = 0.f;
   void drop_graph() {
@@ -2779,7 +2779,7 @@ int xcs_batch_create(const char *alg, int count, const int *ens, const int *k, c
 int xcs_batch_solve(xcs_batch *B, float *ms) {
   if (!B) return set_err(XCS_EINVAL, "NULL batch");
   HIP_TRY(hipSetDevice(B->dev));
-  B->ahead.drop();
+  ReadAhead::Writing writing(B->ahead);
   return batch_run(B, ms);
 }
 
@@ -2824,7 +2824,7 @@ int xcs_batch_x(xcs_batch *B, int idx, float *x_out, float *x_true) {
     *src = B->xs + B->xoff[s];
     *n = B->hP[s].n;
   };
-  if (x_out && !B->ahead.get(idx, B->count, 1, piece, out, B->stream))
+  if (x_out && !B->ahead.read(idx, B->count, 1, piece, out, B->stream))
     HIP_TRY(d2h(x_out, B->xs + B->xoff[q], sizeof(float) * P.n, nullptr));
   if (x_true) memcpy(x_true, B->x_true[q].data(), sizeof(float) * P.n);
   return XCS_OK;
@@ -2833,7 +2833,7 @@ int xcs_batch_x(xcs_batch *B, int idx, float *x_out, float *x_true) {
 int xcs_batch_configure(xcs_batch *B, int team_size, int block_size, int big_count) {
   if (!B) return set_err(XCS_EINVAL, "NULL batch");
   HIP_TRY(hipSetDevice(B->dev));
-  B->ahead.drop();
+  ReadAhead::Writing writing(B->ahead);
   return batch_configure(B, team_size, block_size, big_count);
 }
 
@@ -2847,7 +2847,7 @@ int xcs_batch_schedule(xcs_batch *B, int phases, const int *team_sizes, const in
     if (team_sizes[p] < 1) return set_err(XCS_EINVAL, "phase team sizes must be >= 1");
   if (B->alg == ALG_CSMPSP) return set_err(XCS_EINVAL, CSMPSP_OFF);
   HIP_TRY(hipSetDevice(B->dev));
-  B->ahead.drop();
+  ReadAhead::Writing writing(B->ahead);
   HIP_TRY(hipStreamSynchronize(B->stream));
   B->drop_graph();
   B->sched_team.assign(team_sizes, team_sizes + phases);
@@ -2876,7 +2876,7 @@ int xcs_batch_schedule_mode(xcs_batch *B, int adaptive, int split_team) {
   if (split_team < 0 || split_team > BAR_MAX_TEAM)
     return set_err(XCS_EINVAL, "split_team must be in [0, %d]", BAR_MAX_TEAM);
   HIP_TRY(hipSetDevice(B->dev));
-  B->ahead.drop();
+  ReadAhead::Writing writing(B->ahead);
   HIP_TRY(hipStreamSynchronize(B->stream));
   B->drop_graph();
   B->adaptive = adaptive != 0;
@@ -2897,7 +2897,7 @@ int xcs_batch_tune(xcs_batch *B, int probe_iters, const char *cache_path, int ve
     return set_err(XCS_EINVAL, "NULL argument");
   if (probe_iters < 0) return set_err(XCS_EINVAL, "probe_iters must be >= 0");
   HIP_TRY(hipSetDevice(B->dev));
-  B->ahead.drop();
+  ReadAhead::Writing writing(B->ahead);
   return batch_tune(B, probe_iters, cache_path, verbose, team_size, block_size, big_count,
                     probe_ms);
 }
@@ -2914,7 +2914,7 @@ int xcs_batch_info(xcs_batch *B, int *teams, int *team_size, int *block, float *
 int xcs_batch_apply_timed(xcs_batch *B, int reps, float *ms_per, double *bytes) {
   if (!B || reps <= 0 || !ms_per) return set_err(XCS_EINVAL, "bad arguments");
   HIP_TRY(hipSetDevice(B->dev));
-  B->ahead.drop();
+  ReadAhead::Writing writing(B->ahead);
   int per_cu, cus;
   XCS_TRY(batch_occupancy(B->block, &per_cu, &cus));
   const int grid = std::min(B->count, B->nteams);  // works[] has one entry per team

@@ -1,6 +1,7 @@
 // Host side of a call: streams with staging memory that calls share, small
 // transfers in one launch, and the read-back of many solution vectors.
 #pragma once
+#include "xcs_readahead.h"
 
 // ------------------------------------------------------------------ copies --
 // Up to XFER_MAX pieces of floats copied by one launch, either way between
@@ -203,80 +204,23 @@ static void norms_finish(const NormPart *p, int cnt, int n, int k, float norms[3
 }
 
 // -------------------------------------------------------------- read ahead --
-// Reading a handle's solution vectors one after the other: a copy with its own
-// synchronisation costs 11-17 us however short it is, so the second call in a
-// row fetches the next few vectors in one launch and the window doubles while
-// the calls stay in order, to READ_ROWS vectors or READ_BYTES.  A first or a
-// random access fetches its own vector alone, as before.  The window holds what
-// the device memory holds: everything that can write the handle's vectors drops
-// it first.  Measured on MI355X, 512 signals of 16384 with their 4096
-// measurements: 42 us a signal one by one, 14 us in order.
-constexpr int READ_ROWS = 64;
-constexpr size_t READ_BYTES = (size_t)4 << 20;
-struct ReadAhead {
-  std::mutex mu;
-  float *pin = nullptr;
-  size_t cap = 0;
-  int first = 0, cnt = 0, next = -1, win = 0;
-  size_t off[READ_ROWS][2];
-  ~ReadAhead() {
-    if (pin) (void)hipHostFree(pin);
-  }
-  void drop() {
-    std::lock_guard<std::mutex> lock(mu);
-    cnt = win = 0;
-    next = -1;
-  }
-  // Row i of `count`: piece(i, p, &src, &n) gives its p-th piece (one or two of
-  // them), out[p] takes it where not null.  False: the caller copies by itself
-  // (no window for this call, or no staging memory).
+// The window's memory and transfers (xcs_readahead.h) on a stream.
+static float *pinned_alloc(size_t bytes) {
+  void *p = nullptr;
+  if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return (float *)p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+static void pinned_free(float *p) { (void)hipHostFree(p); }
+struct PinnedReadAhead : ReadAhead {
+  PinnedReadAhead() : ReadAhead(pinned_alloc, pinned_free) {}
+  // Row i of `count` rows: see ReadAhead::get.
   template <class F>
-  bool get(int i, int count, int pieces, F piece, float *const out[2], hipStream_t st) {
-    std::lock_guard<std::mutex> lock(mu);
-    if (i < first || i >= first + cnt) {
-      win = i == next ? std::min(READ_ROWS, std::max(4, 2 * win)) : 0;
-      next = i + 1;
-      cnt = 0;
-      if (!win) return false;
-      XferList L;
-      size_t used = 0;
-      const int top = std::min(win, count - i);
-      const float *src[2];
-      long n[2];
-      int w = 0;
-      for (; w < top; w++) {
-        size_t row = 0;
-        for (int p = 0; p < pieces; p++) {
-          piece(i + w, p, &src[p], &n[p]);
-          row += ((size_t)n[p] + 15) / 16 * 16;
-        }
-        if (4 * (used + row) > READ_BYTES) break;
-        if (!pin) {
-          cap = READ_BYTES;
-          if (hipHostMalloc((void **)&pin, cap, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            pin = nullptr;
-            return false;
-          }
-        }
-        for (int p = 0; p < pieces; p++) {
-          off[w][p] = used;
-          L.add(src[p], pin + used, n[p]);
-          used += ((size_t)n[p] + 15) / 16 * 16;
-        }
-      }
-      if (!w) return false;
-      if (xfer(L, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return false;
-      first = i;
-      cnt = w;
-    }
-    next = i + 1;
-    for (int p = 0; p < pieces; p++) {
-      const float *src;
-      long n;
-      piece(i, p, &src, &n);
-      if (out[p]) memcpy(out[p], pin + off[i - first][p], sizeof(float) * (size_t)n);
-    }
-    return true;
+  bool read(int i, int count, int pieces, F piece, float *const out[2], hipStream_t st) {
+    static_assert(2 * READ_ROWS <= XFER_MAX, "one launch a window");
+    XferList L;
+    return get(
+        i, count, pieces, piece, out, [&](const float *src, float *dst, long n) { L.add(src, dst, n); },
+        [&] { return xfer(L, st) == hipSuccess && hipStreamSynchronize(st) == hipSuccess; });
   }
 };

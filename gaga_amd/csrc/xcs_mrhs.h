@@ -1108,7 +1108,7 @@ struct xcs_mrhs {
   int polish_max = 6;  // support-correction steps
   int gemm_big = -1;   // GEMM block tile where M allows: 0 128 x 128, 1 256 x 128, 2 256 x 256, -1 by gemm_tile
   xcs_options opts{};
-  ReadAhead ahead;     // signals read in order
+  PinnedReadAhead ahead;     // signals read in order
   float phase_ms[6] = {0, 0, 0, 0, 0, 0};  // init, low precision, bf16 continuation, refinement, corrections, spare
   ~xcs_mrhs() {
     if (stream) (void)hipStreamSynchronize(stream);
@@ -1519,7 +1519,7 @@ int xcs_mrhs_create(int m, int n, int k, int count, const char *precision,
 int xcs_mrhs_solve(xcs_mrhs *h, float *ms, int *lp_iterations) {
   if (!h) return set_err(XCS_EINVAL, "NULL handle");
   HIP_TRY(hipSetDevice(h->dev));
-  h->ahead.drop();
+  ReadAhead::Writing writing(h->ahead);
   XCS_TRY(mr_solve(h, ms));
   if (lp_iterations)
     for (int q = 0; q < 3; q++) lp_iterations[q] = h->lp_iters[q];
@@ -1560,7 +1560,7 @@ int xcs_mrhs_x(xcs_mrhs *h, int s, float *x_out, float *x_true, float *y) {
     *src = p ? h->D.y + (size_t)i * h->m : h->D.x + (size_t)i * h->n;
     *n = p ? h->m : h->n;
   };
-  if ((x_out || y) && h->ahead.get(s, h->count, 2, piece, out, h->stream)) return XCS_OK;
+  if ((x_out || y) && h->ahead.read(s, h->count, 2, piece, out, h->stream)) return XCS_OK;
   if (x_out)
     HIP_TRY(d2h(x_out, h->D.x + (size_t)s * h->n, 4 * (size_t)h->n, nullptr));
   if (y) HIP_TRY(d2h(y, h->D.y + (size_t)s * h->m, 4 * (size_t)h->m, nullptr));
@@ -1573,7 +1573,7 @@ int xcs_mrhs_gemm_timed(xcs_mrhs *h, int transpose, const char *fmt, int reps, f
   const int f = strcmp(fmt, "fp8") ? FMT_BF16 : FMT_FP8;
   if (f == FMT_FP8 && !h->a8cm) return set_err(XCS_EINVAL, "fp8 copies exist only for fp8 handles");
   HIP_TRY(hipSetDevice(h->dev));
-  h->ahead.drop();
+  ReadAhead::Writing writing(h->ahead);
   MrhsDesc &D = h->D;
   std::vector<float> ones((size_t)h->count, 1.0f);
   HIP_TRY(h2d(transpose ? D.sr : D.sv, ones.data(), 4 * ones.size(), nullptr));

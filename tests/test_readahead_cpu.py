@@ -1,0 +1,22 @@
+"""The read-ahead window of solution vectors on the CPU, under AddressSanitizer and
+UBSan: reads in every order return what the memory holds, also after a window that
+another reader opened while the vectors were being written
+(tests/cpu_checks/readahead_check.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_readahead_under_sanitizers(tmp_path):
+    exe = str(tmp_path / "readahead_check")
+    src = os.path.join(HERE, "cpu_checks", "readahead_check.cpp")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined",
+                           "-fno-sanitize-recover=all", "-o", exe, src])
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "read-ahead checks passed" in out.stdout
