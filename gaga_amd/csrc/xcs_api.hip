@@ -565,6 +565,7 @@ struct xcs_plan {
   int *warm_mask = nullptr;
   float *warm_score = nullptr;
   float *xt_dev = nullptr;  // the planted vector, where the plan was generated
+  std::mutex pin_mu;  // held while a call uses the lane's staging memory
   ~xcs_plan() {
     // nothing of this plan may still run on memory that is about to be freed
     if (stream) (void)hipStreamSynchronize(stream);
@@ -1083,6 +1084,7 @@ static int plan_run(xcs_plan *pl, float *ms, float *x_out = nullptr) {
   static_assert(sizeof(XState) % sizeof(float) == 0 && LANE_X + sizeof(Back) <= LANE_BYTES, "staging memory");
   Back *back = (Back *)(pl->lane.pin + LANE_X);
   const bool x_too = x_out && sizeof(float) * (size_t)P.n <= LANE_X;
+  std::lock_guard<std::mutex> lock(pl->pin_mu);
   XferList L;
   L.add((XState *)P.st, &back->st, sizeof(XState) / sizeof(float));
   L.add(pl->bar + 2, &back->abort_flag, 1);
@@ -2033,6 +2035,7 @@ int xcs_plan_results(xcs_plan *pl, float norms[3], int *iterations, int support[
   const bool x_pin = x_out && sizeof(float) * (size_t)n <= LANE_X;
   const bool planted = pl->xt_dev && (norms || support);
   if (x_pin || planted) {
+    std::lock_guard<std::mutex> lock(pl->pin_mu);
     float *xh = x_pin ? (float *)pl->lane.pin : nullptr;
     NormPart *part = (NormPart *)(pl->lane.pin + LANE_X);
     const int wgs = norm_wgs(n);
