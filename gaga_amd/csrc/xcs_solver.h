@@ -377,7 +377,8 @@ __device__ void find_support_bin(Team &t, Lds &L, const XProblem &P, XG(const fl
 }
 
 // Ascending support list {i : in(i)} into P.supp; returns its length
-// (uniform).  Requires what `in` reads to be visible; ends with supp visible.
+// (uniform; 0 once the team has aborted).  Requires what `in` reads to be visible;
+// ends with supp visible.
 template <class In>
 __device__ int build_support_if(Team &t, const XProblem &P, In &&in) {
   const int n = P.n;
@@ -407,6 +408,9 @@ __device__ int build_support_if(Team &t, const XProblem &P, In &&in) {
   if (t.size > 1) {
     if (threadIdx.x == 0) P.wg_counts[t.rank] = wg_total;
     t.sync();
+    // a wait timed out: the counts may be an earlier, longer instance's, which would
+    // place the list's entries past its end
+    if (t.aborted) return 0;
     int before = 0, all = 0;
     for (int w = threadIdx.x; w < t.size; w += blockDim.x) {
       const int v = P.wg_counts[w];
