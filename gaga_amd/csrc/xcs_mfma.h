@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(G8_NT) gemm_tn8_kernel(GemmArgs g) {
                    :
                    : "v"((gptr_t)(src[i] + (long)s * GT_KB)),
                      "s"(__builtin_amdgcn_readfirstlane(l0 + 8192 * i))
-                   : "memory");  // nothing else here uses m0
+                   : "memory", "m0");
   };
   f32x16_t acc[2][2];
 #pragma unroll
@@ -355,13 +355,14 @@ __global__ void __launch_bounds__(G8_NT) gemm_tn8_kernel(GemmArgs g) {
     __builtin_amdgcn_s_setprio(0);
   };
   // stage s: its loads have landed once at most the next stage's are in flight;
-  // after the barrier every wave has also finished reading stage s - 1, whose
-  // buffer stage s + 2 takes
+  // after the barrier every wave has also finished reading stage s - 1 (lgkmcnt: its
+  // LDS reads have returned, wherever their products are scheduled), whose buffer
+  // stage s + 2 takes
   auto step = [&](uint8_t *cur, uint8_t *nxt2, int s) {
     if (s + 1 < nsteps)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NL) : "memory");
     else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (s + 2 < nsteps) issue(nxt2, s + 2);
