@@ -552,7 +552,8 @@ struct xcs_plan {
   XProblem h{};         // host copy (device pointers)
   XProblem *d = nullptr;
   int team = 1, block = 256, mode = 0;
-  const void *kernel = nullptr;  // solve_resident_kernel or solve_split_kernel instead of solve_coop_kernel
+  int form = FORM_GENERAL;       // SolveForm the plan is laid out for
+  const void *kernel = nullptr;  // and its kernel, where that is not solve_coop_kernel
   long spin_limit = BAR_SPIN_LIMIT;  // team-barrier wait bound (sleeps)
   double *red = nullptr;
   unsigned *bar = nullptr;
@@ -695,6 +696,7 @@ static int plan_resident(xcs_plan *pl, int alg, const xcs_options *o) {
   }
   if (team > per * cus || team > BAR_MAX_TEAM) return XCS_OK;
   if (!res_fits(alg, P.ens, P.n, P.lda, P.num_bins, P.timing, team)) return XCS_OK;
+  pl->form = FORM_RESIDENT;
   pl->kernel = kernel;
   pl->team = team;
   pl->block = block;
@@ -746,6 +748,7 @@ static int plan_split(xcs_plan *pl, int alg, const xcs_options *o) {
   }
   if (team > per * cus || team > BAR_MAX_TEAM) return XCS_OK;
   if (!split_fits(alg, P.ens, P.m, P.n, P.log2n, P.num_bins, P.timing, team, block)) return XCS_OK;
+  pl->form = FORM_SPLIT;
   pl->kernel = kernel;
   pl->team = team;
   pl->block = block;
@@ -806,7 +809,7 @@ static int plan_alloc(xcs_plan *pl, int alg, int ens, int k, int m, int n, int p
   }
   pl->team = std::min({team, maxb, BAR_MAX_TEAM});
   XCS_TRY(plan_resident(pl, alg, o));
-  if (!pl->kernel) XCS_TRY(plan_split(pl, alg, o));
+  if (pl->form == FORM_GENERAL) XCS_TRY(plan_split(pl, alg, o));
   // CSMPSP is switched off on the device: two of its runs (a 4-workgroup team
   // and later a single workgroup) faulted the GPU and the cause is not yet
   // found; it stays off until it is.
@@ -878,7 +881,7 @@ static int plan_make_y(xcs_plan *pl, const int *d_supp, int cnt, const float *d_
     HIP_TRY(hipMemcpyAsync((int *)P.supp, d_supp, sizeof(int) * cnt, hipMemcpyDeviceToDevice,
                            pl->stream));
   XCS_TRY(plan_upload_desc(pl));
-  if (pl->kernel && P.ens == ENS_GEN) {
+  if (pl->form == FORM_RESIDENT) {
     if (pl->block <= 512)
       hipLaunchKernelGGL(resident_y_kernel<512>, dim3(pl->team), dim3(pl->block), 0, pl->stream,
                          (const XProblem *)pl->d, d_x, cnt, d_y);
@@ -886,7 +889,7 @@ static int plan_make_y(xcs_plan *pl, const int *d_supp, int cnt, const float *d_
       hipLaunchKernelGGL(resident_y_kernel<1024>, dim3(pl->team), dim3(pl->block), 0, pl->stream,
                          (const XProblem *)pl->d, d_x, cnt, d_y);
     HIP_TRY(hipGetLastError());
-  } else if (pl->kernel) {
+  } else if (pl->form == FORM_SPLIT) {
     HIP_TRY(hipMemsetAsync(pl->bar, 0, sizeof(unsigned) * BAR_WORDS, pl->stream));
     long limit = BAR_SPIN_LIMIT;
     int alg = P.alg;
@@ -1039,7 +1042,7 @@ static int plan_generate(xcs_plan *pl, int alg, int ens, int k, int m, int n, in
 }
 
 static int launch_solve(xcs_plan *pl, int budget) {
-  if (pl->kernel) {
+  if (solve_form(pl->form, pl->h.warm != nullptr) != FORM_GENERAL) {
     void *args[] = {(void *)&pl->d, (void *)&budget, (void *)&pl->bar, (void *)&pl->spin_limit};
     HIP_TRY(hipLaunchCooperativeKernel(pl->kernel, dim3(pl->team), dim3(pl->block), args, 0, pl->stream));
     return XCS_OK;

@@ -3,6 +3,7 @@
 // compiler, which is how the CPU tests exercise it).
 //
 //  * the chunk geometry of the gen support gather (A_S x_S);
+//  * the form a plan's solve runs in;
 //  * the names of the ten algorithms, indexed by the Alg codes;
 //  * the autotuner's cache key of a batch.
 #pragma once
@@ -44,6 +45,13 @@ XCS_HD inline int gather_blocks(int cnt) {
   const int b = (cnt + GATHER_BLOCK - 1) / GATHER_BLOCK;
   return b < 1 ? 1 : b;
 }
+
+// The form of a single solve: the general one (solve_coop_kernel), or the ones with
+// the vectors in LDS.  A plan is laid out for one of them; a solve from a warm start
+// (a given support) runs in the general form, the only one that reads it, on the
+// plan's team (at most one workgroup per CU, which the general form always fits).
+enum SolveForm { FORM_GENERAL = 0, FORM_RESIDENT = 1, FORM_SPLIT = 2 };
+inline int solve_form(int planned, bool warm) { return warm ? FORM_GENERAL : planned; }
 
 constexpr int NUM_ALGS = 10;
 // Algorithm names as the reference's option strings spell them
