@@ -1690,22 +1690,12 @@ static int batch_capture(xcs_batch *B) {
   return XCS_OK;
 }
 
-// Teams of c workgroups for up to `want` instances: whole groups of eight (one
-// per XCD, see batch_team), with a few spare teams where the chip has room for
-// them rather than a few instances that wait.
-static int batch_teams(const xcs_batch *B, int want, int c) {
-  const int most = B->resident / c;
-  int nteams = std::min(want, most);
-  if (c > 1 && nteams >= 8) nteams = (nteams + 7) / 8 * 8 <= most ? (nteams + 7) / 8 * 8 : nteams - nteams % 8;
-  return nteams;
-}
-
 // A later phase of the tail schedule: the `cnt` instances at queue positions
 // B->list[0, cnt) on teams of c workgroups (whole teams per XCD where they
 // fit), at most `budget` more iterations each.  Cooperative launch for c > 1.
 static int batch_enqueue_phase(xcs_batch *B, int cnt, int c, int budget) {
   c = std::max(1, std::min(c, std::min(B->resident, BAR_MAX_TEAM)));
-  const int nteams = batch_teams(B, cnt, c);
+  const int nteams = batch_teams(B->resident, cnt, c);
   const int grid = nteams * c, n_big = c > 1 ? cnt : 0;
   hipLaunchKernelGGL(batch_reset_kernel, dim3(64), dim3(256), 0, B->stream, B->xs, (size_t)0,
                      (int *)B->sts, (size_t)0, B->queue, B->bar, (size_t)BAR_WORDS * nteams);
@@ -1819,38 +1809,14 @@ static double batch_bytes1(const xcs_batch *B, int q) {
   return P.ens == ENS_GEN ? 4.0 * P.lda * (double)P.n : P.ens == ENS_SMV ? 8.0 * P.nz : 24.0 * P.n;
 }
 
-// One solve on the configured geometry (teams of c for the n_big largest, no
-// tail schedule), in larger teams where the chip has room for them.  A workgroup
-// streams about 100 GB/s, so a large instance on a few workgroups takes long after
-// the others are done.  Teams of twice the size are taken, again and again,
-// while every large instance still has its team at once, a workgroup keeps GROW_BYTES
-// a product (below that the team's barriers take the time) and the longest wait
-// shrinks: the bytes a workgroup streams for the largest instance and, where the
-// other instances can't all run beside the teams, for the largest of those after it.
-// Measured on MI355X, ms per solve before and after: instances of both ensembles, n =
-// 1024 to 8192, the largest quarter in teams of 4, CGIHT: 256 of them 21.0 -> 16.6, 128
-// 14.7 -> 10.5, 64 9.4 -> 4.2, 16 5.6 -> 3.6; 20 of 2048 x 8192 in teams of 4 16.2 -> 7.4.
-constexpr double GROW_BYTES = 2e6;
-static int batch_run_teams(xcs_batch *B) {
-  const int big = B->n_big, small = B->count - big;
+// The geometry of a solve on teams without a tail schedule.
+static BatchPick batch_pick(const xcs_batch *B) {
   double most = 0.0, most1 = 0.0;
-  for (int q = 0; q < big; q++) most = std::max(most, batch_bytes1(B, q));
-  for (int q = big; q < B->count; q++) most1 = std::max(most1, batch_bytes1(B, q));
-  int c = B->c, grid = B->grid;
-  double wait = 0.0;
-  for (int d = B->c; d <= std::min(B->resident, BAR_MAX_TEAM) && (d == B->c || most / d >= GROW_BYTES); d *= 2) {
-    const int teams = batch_teams(B, big + (small + d - 1) / d, d);
-    const double w = most / d + ((long)teams * d >= (long)big * d + small ? 0.0 : most1);
-    if (d > B->c && teams < big) break;
-    if (d > B->c && w >= wait) continue;
-    wait = w;
-    if (d > B->c) {
-      c = d;
-      grid = teams * d;
-    }
-  }
-  return batch_enqueue(B, B->budget, c, grid);
+  for (int q = 0; q < B->n_big; q++) most = std::max(most, batch_bytes1(B, q));
+  for (int q = B->n_big; q < B->count; q++) most1 = std::max(most1, batch_bytes1(B, q));
+  return batch_pick(B->count, B->n_big, B->c, B->resident, BAR_MAX_TEAM, most, most1, true);
 }
+static bool batch_picks(const xcs_batch *B) { return B->c > 1 && B->sched_budget.empty() && B->n_big > 0; }
 
 static int batch_run(xcs_batch *B, float *ms) {
   if (B->adaptive && B->c == 1 && B->sched_budget.size() >= 2) return batch_run_adaptive(B, ms);
@@ -1861,8 +1827,9 @@ static int batch_run(xcs_batch *B, float *ms) {
   HIP_TRY(hipEventRecord(e0, B->stream));
   if (B->graph) {
     HIP_TRY(hipGraphLaunch(B->graph, B->stream));
-  } else if (B->c > 1 && B->sched_budget.empty() && B->n_big > 0) {
-    XCS_TRY(batch_run_teams(B));
+  } else if (batch_picks(B)) {
+    const BatchPick p = batch_pick(B);
+    XCS_TRY(batch_enqueue(B, B->budget, p.c, p.teams * p.c));
   } else {
     XCS_TRY(batch_enqueue(B, B->sched_budget.empty() ? B->budget : B->sched_budget[0]));
   }

@@ -3,7 +3,7 @@
 // compiler, which is how the CPU tests exercise it).
 //
 //  * the chunk geometry of the gen support gather (A_S x_S);
-//  * the form a plan's solve runs in;
+//  * the form a plan's solve runs in, and the teams a batch's does;
 //  * the names of the ten algorithms, indexed by the Alg codes;
 //  * the autotuner's cache key of a batch.
 #pragma once
@@ -52,6 +52,48 @@ XCS_HD inline int gather_blocks(int cnt) {
 // plan's team (at most one workgroup per CU, which the general form always fits).
 enum SolveForm { FORM_GENERAL = 0, FORM_RESIDENT = 1, FORM_SPLIT = 2 };
 inline int solve_form(int planned, bool warm) { return warm ? FORM_GENERAL : planned; }
+
+// Teams of c workgroups for up to `want` instances, of `resident` workgroups in all:
+// whole groups of eight (one per XCD), with a few spare teams where the chip has room
+// for them rather than a few instances that wait.
+inline int batch_teams(int resident, int want, int c) {
+  const int most = resident / c;
+  const int teams = std::min(want, most);
+  if (c == 1 || teams < 8) return teams;
+  return (teams + 7) / 8 * 8 <= most ? (teams + 7) / 8 * 8 : teams - teams % 8;
+}
+
+// The geometry of one batch solve without a tail schedule: teams of c for the `big`
+// largest of `count` instances, single workgroups for the others.  With `grow`, in
+// larger teams where the chip has room for them.  A workgroup streams about 100 GB/s,
+// so a large instance on a few workgroups takes long after the others are done.
+// Teams of twice the size are taken, again and again, while every large instance
+// still has its team at once, a workgroup keeps GROW_BYTES a product (below that the
+// team's barriers take the time) and the longest wait shrinks: the bytes a workgroup
+// streams for the largest instance (`most`) and, where the other instances can't all
+// run beside the teams, for the largest of those after it (`most1`).
+// Measured on MI355X, ms per solve before and after: instances of both ensembles, n =
+// 1024 to 8192, the largest quarter in teams of 4, CGIHT: 256 of them 21.0 -> 16.6, 128
+// 14.7 -> 10.5, 64 9.4 -> 4.2, 16 5.6 -> 3.6; 20 of 2048 x 8192 in teams of 4 16.2 -> 7.4.
+constexpr double GROW_BYTES = 2e6;
+struct BatchPick {
+  int c, teams;
+};
+inline BatchPick batch_pick(int count, int big, int c, int resident, int max_team, double most, double most1,
+                            bool grow) {
+  const int small = count - big;
+  BatchPick best{c, 0};
+  double wait = 0.0;
+  for (int d = c; d == c || (grow && d <= std::min(resident, max_team) && most / d >= GROW_BYTES); d *= 2) {
+    const int teams = batch_teams(resident, big + (small + d - 1) / d, d);
+    const double w = most / d + ((long)teams * d >= (long)big * d + small ? 0.0 : most1);
+    if (d > c && teams < big) break;
+    if (d > c && w >= wait) continue;
+    wait = w;
+    best = BatchPick{d, teams};
+  }
+  return best;
+}
 
 constexpr int NUM_ALGS = 10;
 // Algorithm names as the reference's option strings spell them
