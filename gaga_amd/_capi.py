@@ -24,7 +24,7 @@ EXPORTS = (
     "xcs_mlp_set_data", "xcs_mlp_train", "xcs_plan_solve_warm", "xcs_mlp_features", "xcs_stream_copy", "xcs_mrhs_destroy",
     "xcs_last_error", "xcs_version", "xcs_results_line", "xcs_results_append",
     "xcs_cs_gen_noalloc", "xcs_batch_schedule", "xcs_batch_phase_counts", "xcs_stream_read",
-    "xcs_batch_schedule_mode",
+    "xcs_batch_schedule_mode", "xcs_batch_exact", "xcs_batch_ran",
 )
 
 
@@ -127,6 +127,8 @@ def load():
         L.xcs_batch_results.argtypes = [_P, _P, _P, _P, _P]
         L.xcs_batch_x.argtypes = [_P, _I, _P, _P]
         L.xcs_batch_info.argtypes = [_P, _P, _P, _P, _P]
+        L.xcs_batch_exact.argtypes = [_P, _I]
+        L.xcs_batch_ran.argtypes = [_P, _P, _P]
         L.xcs_batch_destroy.argtypes = [_P]
         L.xcs_batch_destroy.restype = None
         L.xcs_batch_phase_ticks.argtypes = [_P, _P]
@@ -483,10 +485,18 @@ class Batch:
         _ck(load().xcs_batch_phase_counts(self._h, _p(out), phases))
         return out
 
-    def configure(self, team_size, block_size, big_count=-1):
+    def configure(self, team_size, block_size, big_count=-1, exact=False):
         """team_size workgroups per instance for the big_count largest instances
-        (-1: all), one workgroup for the rest."""
+        (-1: all), one workgroup for the rest.  Where the chip has room a solve takes
+        larger teams, unless exact is set (ran() tells)."""
         _ck(load().xcs_batch_configure(self._h, int(team_size), int(block_size), int(big_count)))
+        _ck(load().xcs_batch_exact(self._h, 1 if exact else 0))
+
+    def ran(self):
+        """(teams, team_size) of the last solve."""
+        t, c = ctypes.c_int(), ctypes.c_int()
+        _ck(load().xcs_batch_ran(self._h, ctypes.byref(t), ctypes.byref(c)))
+        return t.value, c.value
 
     def tune(self, probe_iters=32, cache=None, verbose=False):
         """Pick the team geometry by timing candidates on this batch; returns

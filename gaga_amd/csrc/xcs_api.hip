@@ -12,6 +12,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <array>
 #include <vector>
 
 #include "../../include/gaga_amd.h"
@@ -1187,6 +1188,8 @@ struct xcs_batch {
   hipStream_t stream = nullptr;
   int alg = 0, count = 0, c = 1, block = 256, nteams = 0, grid = 0, budget = 0;
   int n_big = 0;  // instances [0, n_big) (queue order) go to teams of c workgroups
+  bool exact = false;  // teams as configured, also where the chip has room for larger ones
+  int ran_c = 0, ran_teams = 0;  // the last solve's first launch
   int resident = 0;  // workgroups resident at this block size (workspace sized for them)
   int *list = nullptr;  // queue slots of the instances a later phase of the tail schedule takes
   // tail schedule: phase 0 solves every instance on the configured geometry for at
@@ -1643,6 +1646,8 @@ static int batch_generate(xcs_batch *B, int alg, int count, const int *ens, cons
 // Reset, then solve: the two launches of one batched solve, on B->stream.
 // budget: iterations per instance in this launch.
 static int batch_enqueue(xcs_batch *B, int budget, int c, int grid) {
+  B->ran_c = c;
+  B->ran_teams = grid / c;
   const int rgrid = (int)std::min<size_t>(4096, (B->xs_len + 255) / 256 + 1);
   hipLaunchKernelGGL(batch_reset_kernel, dim3(rgrid), dim3(256), 0, B->stream, B->xs, B->xs_len,
                      (int *)B->sts, sizeof(XState) / sizeof(int) * (size_t)B->count, B->queue,
@@ -1755,6 +1760,8 @@ static int batch_run_adaptive(xcs_batch *B, float *ms) {
     lv.c[l] = l ? std::max(1, std::min(B->sched_team[l], std::min(B->resident, BAR_MAX_TEAM))) : 1;
     lv.budget[l] = l + 1 == levels ? B->budget : B->sched_budget[l];
   }
+  B->ran_c = 1;
+  B->ran_teams = B->resident;
   lv.split_c = B->split_team >= 2 ? std::min(B->split_team, std::min(B->resident, BAR_MAX_TEAM)) : 0;
   // a partly formed team per level must never hold every workgroup
   const int chk = sched_levels_check(lv, B->resident);
@@ -1814,7 +1821,7 @@ static BatchPick batch_pick(const xcs_batch *B) {
   double most = 0.0, most1 = 0.0;
   for (int q = 0; q < B->n_big; q++) most = std::max(most, batch_bytes1(B, q));
   for (int q = B->n_big; q < B->count; q++) most1 = std::max(most1, batch_bytes1(B, q));
-  return batch_pick(B->count, B->n_big, B->c, B->resident, BAR_MAX_TEAM, most, most1, true);
+  return batch_pick(B->count, B->n_big, B->c, B->resident, BAR_MAX_TEAM, most, most1, !B->exact);
 }
 static bool batch_picks(const xcs_batch *B) { return B->c > 1 && B->sched_budget.empty() && B->n_big > 0; }
 
@@ -1901,6 +1908,9 @@ static int batch_tune(xcs_batch *B, int probe_iters, const char *cache_path, int
   const int splits[] = {-1, B->count / 16, B->count / 8, B->count / 4};
   float best = 1e30f;
   int best_c = B->c, best_b = B->block, best_big = -1;
+  // what the candidates so far ran as: where the chip has room for larger teams,
+  // several of them come to the same launch, which is timed once
+  std::vector<std::array<int, 4>> timed;
   for (int bi = 0; bi < 3; bi++)
     for (int ti = 0; ti < 4; ti++)
       for (int si = 0; si < 4; si++) {
@@ -1911,14 +1921,18 @@ static int batch_tune(xcs_batch *B, int probe_iters, const char *cache_path, int
         XCS_TRY(batch_occupancy(blk, &per_cu, &cus));
         if (c > 1 && per_cu * cus / c < 8) continue;
         XCS_TRY(batch_configure(B, c, blk, big));
+        const BatchPick as = batch_picks(B) ? batch_pick(B) : BatchPick{B->c, B->nteams};
+        const std::array<int, 4> key = {as.c, as.teams, blk, B->n_big};
+        if (std::find(timed.begin(), timed.end(), key) != timed.end()) continue;
+        timed.push_back(key);
         B->budget = budget;
         float ms = 0.f;
         const int rc = batch_run(B, &ms);
         B->budget = saved_budget;
         if (rc != XCS_OK) return rc;
         if (verbose) {
-          fprintf(stderr, "tune: team %d block %4d team instances %5d: %9.2f ms\n", c, blk,
-                  B->n_big, ms);
+          fprintf(stderr, "tune: team %d (ran %d) block %4d team instances %5d: %9.2f ms\n", c, B->ran_c,
+                  blk, B->n_big, ms);
           fflush(stderr);
         }
         if (ms < best) {
@@ -2881,6 +2895,20 @@ int xcs_batch_info(xcs_batch *B, int *teams, int *team_size, int *block, float *
   if (team_size) *team_size = B->c;
   if (block) *block = B->block;
   if (gen_ms) *gen_ms = B->gen_ms;
+  return XCS_OK;
+}
+
+int xcs_batch_ran(xcs_batch *B, int *teams, int *team_size) {
+  if (!B) return set_err(XCS_EINVAL, "NULL batch");
+  if (!B->ran_c) return set_err(XCS_EINVAL, "the batch has not been solved");
+  if (teams) *teams = B->ran_teams;
+  if (team_size) *team_size = B->ran_c;
+  return XCS_OK;
+}
+
+int xcs_batch_exact(xcs_batch *B, int exact) {
+  if (!B) return set_err(XCS_EINVAL, "NULL batch");
+  B->exact = exact != 0;
   return XCS_OK;
 }
 

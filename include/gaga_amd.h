@@ -207,9 +207,15 @@ int xcs_batch_solve(xcs_batch *batch, float *ms);
 /* Change the team geometry: team_size workgroups of block_size threads per instance for the
  * big_count largest instances (big_count < 0: all of them); the rest run one per workgroup
  * once those are taken.  Without a tail schedule a solve takes teams of twice, four times, ...
- * team_size where the chip has room for all of them at once.  Recovery does not depend on
- * the geometry (reduction order does). */
+ * team_size where the chip has room for all of them at once (unless xcs_batch_exact says
+ * otherwise).  Recovery does not depend on the geometry (reduction order does). */
 int xcs_batch_configure(xcs_batch *batch, int team_size, int block_size, int big_count);
+/* exact != 0: solves run teams of exactly the configured size; 0 (the default): larger ones
+ * where the chip has room. */
+int xcs_batch_exact(xcs_batch *batch, int exact);
+/* The teams of the last solve (its first launch, where a tail schedule made several);
+ * xcs_batch_info reports the configured geometry. */
+int xcs_batch_ran(xcs_batch *batch, int *teams, int *team_size);
 /* Tail schedule (no counterpart in the reference, whose sweep driver runs one problem per
  * call): phase 0 solves every instance on the configured geometry for at most budgets[0]
  * iterations; phase p = 1 .. phases-1 gives the instances still running teams of
@@ -237,7 +243,8 @@ int xcs_batch_schedule_mode(xcs_batch *batch, int adaptive, int split_team);
 int xcs_batch_phase_counts(xcs_batch *batch, int *counts, int phases);
 /* Autotuner: time every candidate geometry (team 1/2/4/8 x block 256/512/1024 x teams for all,
  * or for the largest 1/16, 1/8, 1/4 of the instances) on this batch with each instance capped
- * at probe_iters iterations (0: whole solves), keep the fastest.  cache_path (may be NULL) is
+ * at probe_iters iterations (0: whole solves), keep the fastest; candidates that come to the
+ * same launch (larger teams where the chip has room) are timed once.  cache_path (may be NULL) is
  * a text file of "<signature> <team> <block> <big_count> <ms>" lines: a hit skips the probes,
  * a miss appends the result.  verbose != 0 prints each candidate's time to stderr. */
 int xcs_batch_tune(xcs_batch *batch, int probe_iters, const char *cache_path, int verbose,
