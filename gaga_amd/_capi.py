@@ -600,8 +600,8 @@ class ManyRHS:
                                       int(ref_outer), int(ref_inner)))
 
     def gemm_tile(self, tile):
-        """GEMM block tile: 0 128 x 128, 1 256 x 128, 2 256 x 256 (True means 1);
-        until it is called each product's tile follows from its sizes."""
+        """GEMM block tile: 0 128 x 128, 1 256 x 128, 2 256 x 256 (True means 1), -1 (the
+        default) each product's by its sizes."""
         _ck(load().xcs_mrhs_gemm_tile(self._h, int(tile)))
 
     def samples(self, per, seed=1):

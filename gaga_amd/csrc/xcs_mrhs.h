@@ -1142,23 +1142,25 @@ struct xcs_mrhs {
 // by the kernel that reads the product, so they cost no pass of their own; they
 // matter for narrow products (few active signals) and small matrices, which
 // leave most of the chip idle unsplit.  Measured on MI355X: BF16 A^T R of 16384 x
-// 4096 with up to 128 columns 61 us unsplit, 24 with its four slices.
+// 4096 with up to 128 columns 61 us unsplit, 24 with its four slices.  A forced tile
+// keeps the slices, and with them the order of every sum: the tile does not change
+// a result.  The column count (the active signals) does, in the products' rounding.
 static void mr_gemm_shape(int forced, int M, int N, long kbytes, int *tile, int *ks) {
   const long stages = kbytes / GT_KB;
   auto fits = [&](int k) { return stages % k == 0 && stages / k >= 2; };
   const long t128 = (long)(M / 128) * ((N + 127) / 128);
-  if (M % 256 == 0 && forced != 0) {
-    for (int k = 1; k <= 4; k *= 2)
+  *tile = 0;
+  if (M % 256 == 0)
+    for (int k = 1; k <= 4 && !*tile; k *= 2)
       if (fits(k) && gemm_tile(M, N, k)) {
         *tile = 1;
         *ks = k;
-        if (forced < 0 || forced == 1) return;
-        break;
       }
+  if (!*tile) {
+    *ks = 1;
+    while (*ks < MR_KMAX && t128 * *ks < 256 && fits(2 * *ks)) *ks *= 2;
   }
-  *tile = forced > 0 && M % 256 == 0 ? forced : 0;
-  *ks = 1;
-  while (*ks < MR_KMAX && t128 * *ks < 256 && fits(2 * *ks)) *ks *= 2;
+  if (forced >= 0) *tile = M % 256 == 0 ? forced : 0;
 }
 
 enum { MR_AX = 0, MR_G = 1, MR_W = 2 };
@@ -1205,12 +1207,11 @@ static int mr_gemm(xcs_mrhs *h, int fmt, int which, int cols, const int *ncols, 
 static size_t mr_product_floats(int M, int cols, int K) {
   size_t most = 0;
   for (int N = 1; N <= cols; N++)
-    for (int esz = 1; esz <= 2; esz++)
-      for (int forced = -1; forced <= 2; forced++) {
-        int tile, ks;
-        mr_gemm_shape(forced, M, N, (long)K * esz, &tile, &ks);
-        most = std::max(most, (size_t)ks * N * M);
-      }
+    for (int esz = 1; esz <= 2; esz++) {
+      int tile, ks;
+      mr_gemm_shape(-1, M, N, (long)K * esz, &tile, &ks);
+      most = std::max(most, (size_t)ks * N * M);
+    }
   return most;
 }
 
@@ -1654,7 +1655,7 @@ int xcs_mrhs_configure(xcs_mrhs *h, float c_bf16, float c_fp8, int exact_max, in
 
 int xcs_mrhs_gemm_tile(xcs_mrhs *h, int tile) {
   if (!h) return set_err(XCS_EINVAL, "NULL handle");
-  if (tile < 0 || tile > 2) return set_err(XCS_EINVAL, "tile must be 0, 1 or 2");
+  if (tile < -1 || tile > 2) return set_err(XCS_EINVAL, "tile must be -1 (by sizes), 0, 1 or 2");
   h->gemm_big = tile;
   return XCS_OK;
 }

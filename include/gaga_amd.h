@@ -302,9 +302,10 @@ int xcs_mrhs_fp32_solve(xcs_mrhs *handle, int first, int cnt, int mode, float *m
 int xcs_mrhs_configure(xcs_mrhs *handle, float c_bf16, float c_fp8, int corrections,
                        int ref_outer, int ref_inner);
 /* GEMM block tile of the products where the row count allows (no counterpart in the
- * reference): 0 128 x 128 with 4 waves, 1 256 x 128 with 8 waves, 2 256 x 256 with 8 waves;
- * until it is called each product's tile follows from its sizes.  Results do not depend
- * on it. */
+ * reference): 0 128 x 128 with 4 waves, 1 256 x 128 with 8 waves, 2 256 x 256 with 8 waves,
+ * -1 (the default) each product's by its sizes.  Results do not depend on it.  They do depend, in
+ * the rounding of the products only, on the number of signals that are still active: it decides
+ * in how many slices a product sums. */
 int xcs_mrhs_gemm_tile(xcs_mrhs *handle, int tile);
 /* Device ms of the last solve's phases: start, low-precision phase, BF16 continuation,
  * refinement, support corrections (with their refinements), 0. */
