@@ -761,7 +761,7 @@ __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, doubl
                                                                     int groups, int sel) {
   constexpr int SLOTS = MR_RT / 8, ROWS = MR_RT / 16;
   static_assert(MR_RLIST % SLOTS == 0, "whole rounds");
-  __shared__ uint2 list[MR_RLIST];  // (byte offset of the column in a block, value)
+  __shared__ uint2 list[MR_RLIST];  // (column, value)
   __shared__ double red[ROWS][MR_RB];
   const int s = mr_signal(D, sel, blockIdx.x >> 3);
   if (s < 0) return;
@@ -772,7 +772,10 @@ __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, doubl
   const int *sup = D.supp + s * n;
   bool staged = false;
   for (int b = (blockIdx.x & 7) + 8 * blockIdx.y; b < blocks; b += 8 * groups) {
-    const char *base = reinterpret_cast<const char *>(D.A32b + (long)b * n * MR_RB);
+    const char *base = reinterpret_cast<const char *>(D.A32b + (long)b * n * MR_RB) + 16 * sub;
+    // the column's part of this row block (64-bit: a block is longer than 4 GB beyond
+    // 2^25 columns)
+    auto column = [&](unsigned j) { return *(const float4 *)(base + (size_t)j * (4 * MR_RB)); };
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c0 = 0; c0 < cnt; c0 += MR_RLIST) {
       const int c1 = min(MR_RLIST, (cnt - c0 + SLOTS - 1) / SLOTS * SLOTS);
@@ -782,7 +785,7 @@ __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, doubl
           uint2 e = make_uint2(0u, 0u);
           if (c0 + c < cnt) {
             const int j = sup[c0 + c];
-            e = make_uint2((unsigned)j * (4u * MR_RB), __float_as_uint(x[j]));
+            e = make_uint2((unsigned)j, __float_as_uint(x[j]));
           }
           list[c] = e;
         }
@@ -803,13 +806,13 @@ __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, doubl
 #pragma unroll
         for (int u = 0; u < MR_RU; u++) e[u] = list[c + u * SLOTS];
 #pragma unroll
-        for (int u = 0; u < MR_RU; u++) v[u] = *(const float4 *)(base + (e[u].x + 16u * sub));
+        for (int u = 0; u < MR_RU; u++) v[u] = column(e[u].x);
 #pragma unroll
         for (int u = 0; u < MR_RU; u++) add(v[u], e[u].y);
       }
       for (; c < c1; c += SLOTS) {
         const uint2 e = list[c];
-        add(*(const float4 *)(base + (e.x + 16u * sub)), e.y);
+        add(column(e.x), e.y);
       }
     }
 #pragma unroll

@@ -1,0 +1,23 @@
+"""The many-RHS exact residual where its row-blocked copy of A is longer than 32-bit
+offsets reach."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def test_columns_beyond_32_bit_offsets(lib):
+    # 128-byte pieces: offsets beyond 2^32 from column 2^25 on; half of the signals have theirs there
+    n, count = 1 << 26, 8
+    R = lib.ManyRHS(128, n, 1, count, "bf16",
+                    lib.options(tol=1e-5, seed=3, vecDistribution="gaussian", maxiter=50))
+    R.solve()
+    r = R.results()
+    true = [R.x(s)[1] for s in range(count)]
+    assert any(np.flatnonzero(t)[0] >= 1 << 25 for t in true)
+    for s in range(count):
+        x = R.x(s)[0]
+        assert np.array_equal(np.flatnonzero(x), np.flatnonzero(true[s]))
+        # one column of unit length: |x - x_true| <= |r| / |a| with |a| > 1 / 2
+        assert np.abs(x - true[s]).max() <= 2e-5 and r["resid_rel"][s] <= 1e-6
+    R.close()
