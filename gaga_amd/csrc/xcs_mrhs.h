@@ -59,7 +59,8 @@ struct MrhsDesc {
   double *ref;  // per signal: gamma, |r|^2, |y|^2, spare
   int *supp, *supp_cnt;
   float *cp, *cd;  // refinement: CG direction and correction, by list position
-  const float *A32b;  // A in FP32, in blocks of MR_RB rows
+  const float *A32b;  // A in FP32, in blocks of MR_RB rows (null: column-major only)
+  const float *A32;   // A in FP32, column-major
 };
 
 __device__ __forceinline__ float4 mr_ld4(const float *p, long o) {
@@ -752,11 +753,14 @@ __global__ void __launch_bounds__(MR_VT) mr_ref_supp_kernel(MrhsDesc D, int sel)
 // workgroups have to keep step for that: more loads a lane run them further apart
 // (256 threads with 4 / 2 / 1 loads: 324 / 246 / 286 us at 37 / 71 / 78% hits; 128 with
 // 8 / 4 / 2: 315 / 296 / 219; 64 with 4: 219).
+// BLOCKED = false reads the column-major matrix in the same order, for handles that had no
+// memory for the other (the same bits).
 constexpr int MR_RB = 32;
 constexpr int MR_RT = 128;
 constexpr int MR_RU = 2;
 constexpr int MR_RLIST = 1024;  // support entries held in LDS at a time
 constexpr int MR_MAXM = 8192;
+template <bool BLOCKED>
 __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, double *part,
                                                                     int groups, int sel) {
   constexpr int SLOTS = MR_RT / 8, ROWS = MR_RT / 16;
@@ -772,10 +776,13 @@ __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, doubl
   const int *sup = D.supp + s * n;
   bool staged = false;
   for (int b = (blockIdx.x & 7) + 8 * blockIdx.y; b < blocks; b += 8 * groups) {
-    const char *base = reinterpret_cast<const char *>(D.A32b + (long)b * n * MR_RB) + 16 * sub;
+    const char *base = reinterpret_cast<const char *>(BLOCKED ? D.A32b + (long)b * n * MR_RB
+                                                              : D.A32 + (long)b * MR_RB) + 16 * sub;
     // the column's part of this row block (64-bit: a block is longer than 4 GB beyond
     // 2^25 columns)
-    auto column = [&](unsigned j) { return *(const float4 *)(base + (size_t)j * (4 * MR_RB)); };
+    auto column = [&](unsigned j) {
+      return *(const float4 *)(base + (BLOCKED ? (size_t)j * (4 * MR_RB) : (size_t)j * (4 * (size_t)m)));
+    };
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c0 = 0; c0 < cnt; c0 += MR_RLIST) {
       const int c1 = min(MR_RLIST, (cnt - c0 + SLOTS - 1) / SLOTS * SLOTS);
@@ -1247,10 +1254,6 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   hipLaunchKernelGGL(gen_matrix_kernel, dim3((int)std::min<size_t>(65536, (mn + 255) / 256)),
                      dim3(256), 0, h->stream, h->A32, m, n, m, o->seed, o->instance);
   HIP_TRY(hipGetLastError());
-  XCS_TRY(h->alloc(&h->A32b, mn));
-  hipLaunchKernelGGL(mr_blocks_kernel, dim3((int)std::min<size_t>(65536, (mn / 4 + MR_THREADS - 1) / MR_THREADS)),
-                     dim3(MR_THREADS), 0, h->stream, (const float4 *)h->A32, m, n, (float4 *)h->A32b);
-  HIP_TRY(hipGetLastError());
   XCS_TRY(h->alloc(&h->cs, (size_t)n));
   XCS_TRY(h->alloc(&h->a16cm, 2 * mn));
   XCS_TRY(h->alloc(&h->a16rm, 2 * mn));
@@ -1279,7 +1282,7 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
   D.restart = o->restart;
   D.maxiter = o->maxiter > 0 ? o->maxiter : 5000;
   D.tol = o->tol_reference_default ? (float)(10 ^ (-4)) : o->tol;
-  D.A32b = h->A32b;
+  D.A32 = h->A32;
   D.colscale = h->cs;
   float *y;
   XCS_TRY(h->alloc(&y, S * m));
@@ -1342,6 +1345,16 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
     HIP_TRY(d2h(h->val_true.data(), d_vals, 4 * S * k, nullptr));
     HIP_TRY(d2h(h->sup_true.data(), d_sup, 4 * S * k, nullptr));
   }
+  // the row-blocked copy for the exact residual, where there is memory left for it
+  if (h->alloc(&h->A32b, mn) == XCS_OK) {
+    hipLaunchKernelGGL(mr_blocks_kernel, dim3((int)std::min<size_t>(65536, (mn / 4 + MR_THREADS - 1) / MR_THREADS)),
+                       dim3(MR_THREADS), 0, h->stream, (const float4 *)h->A32, m, n, (float4 *)h->A32b);
+    HIP_TRY(hipGetLastError());
+    D.A32b = h->A32b;
+  } else {
+    (void)hipGetLastError();
+    h->A32b = nullptr;
+  }
   hipLaunchKernelGGL(mr_make_y_kernel, dim3(count), dim3(MR_THREADS), 0, h->stream, h->A32, m,
                      d_vals, d_sup, k, y);
   HIP_TRY(hipGetLastError());
@@ -1364,8 +1377,12 @@ static int mr_exact_resid(xcs_mrhs *h, int sel) {
   int groups = 1;
   while (groups < per && 8L * groups * cols < 4096) groups *= 2;
   groups = std::min(groups, per);
-  hipLaunchKernelGGL(mr_exact_resid_kernel, dim3(8 * cols, groups), dim3(MR_RT), 0, h->stream, h->D,
-                     h->part, groups, sel);
+  if (h->D.A32b)
+    hipLaunchKernelGGL(mr_exact_resid_kernel<true>, dim3(8 * cols, groups), dim3(MR_RT), 0, h->stream, h->D,
+                       h->part, groups, sel);
+  else
+    hipLaunchKernelGGL(mr_exact_resid_kernel<false>, dim3(8 * cols, groups), dim3(MR_RT), 0, h->stream, h->D,
+                       h->part, groups, sel);
   HIP_TRY(hipGetLastError());
   return XCS_OK;
 }
