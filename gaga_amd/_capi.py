@@ -24,7 +24,7 @@ EXPORTS = (
     "xcs_mlp_set_data", "xcs_mlp_train", "xcs_plan_solve_warm", "xcs_mlp_features", "xcs_stream_copy", "xcs_mrhs_destroy",
     "xcs_last_error", "xcs_version", "xcs_results_line", "xcs_results_append",
     "xcs_cs_gen_noalloc", "xcs_batch_schedule", "xcs_batch_phase_counts", "xcs_stream_read",
-    "xcs_batch_schedule_mode", "xcs_batch_exact", "xcs_batch_ran",
+    "xcs_batch_schedule_mode", "xcs_batch_exact", "xcs_batch_ran", "xcs_plan_form",
 )
 
 
@@ -87,6 +87,7 @@ def load():
         L.xcs_plan_destroy.restype = None
         L.xcs_plan_bytes.argtypes = [_P, _P]
         L.xcs_plan_geometry.argtypes = [_P, _P, _P]
+        L.xcs_plan_form.argtypes = [_P, _P, _P, _P, _P]
         L.xcs_plan_apply_timed.argtypes = [_P, _I, _I, _P, _P]
         L.xcs_batch_bytes.argtypes = [_P, _P]
         L.xcs_batch_apply_timed.argtypes = [_P, _I, _P, _P]
@@ -353,6 +354,13 @@ class Plan:
         t, b = ctypes.c_int(0), ctypes.c_int(0)
         _ck(load().xcs_plan_geometry(self._h, ctypes.byref(t), ctypes.byref(b)))
         return t.value, b.value
+
+    def form(self):
+        """(form, support bits in LDS, workgroups with their rows' entries in LDS, with
+        their columns'): form is "general", "resident" or "split"."""
+        v = [ctypes.c_int(0) for _ in range(4)]
+        _ck(load().xcs_plan_form(self._h, *[ctypes.byref(q) for q in v]))
+        return ("general", "resident", "split")[v[0].value], bool(v[1].value), v[2].value, v[3].value
 
     def solve_warm(self, net=None, cg_steps=3):
         """CGIHT from the network's predicted support (net None: the k largest

@@ -2104,6 +2104,34 @@ int xcs_plan_bytes(xcs_plan *pl, double *bytes) {
   return XCS_OK;
 }
 
+int xcs_plan_form(xcs_plan *pl, int *form, int *support_bits, int *rows_staged, int *columns_staged) {
+  if (!pl) return set_err(XCS_EINVAL, "NULL plan");
+  HIP_TRY(hipSetDevice(pl->dev));
+  const XProblem &P = pl->h;
+  int bits = 0, rows = 0, cols = 0;
+  if (pl->form == FORM_SPLIT && P.ens == ENS_SMV && (support_bits || rows_staged || columns_staged)) {
+    const SplitGeom G = split_geom(P.ens, P.alg, P.m, P.n, P.log2n, P.num_bins, pl->team);
+    bits = G.filter;
+    if (rows_staged || columns_staged) {
+      std::vector<int> rp((size_t)P.m + 1), cp((size_t)P.n + 1);
+      HIP_TRY(d2h(rp.data(), P.row_ptr, sizeof(int) * rp.size(), nullptr));
+      HIP_TRY(d2h(cp.data(), P.col_ptr, sizeof(int) * cp.size(), nullptr));
+      for (int w = 0; w < pl->team; w++) {
+        const int j0 = (int)std::min<long>(P.n, (long)w * G.nl), i0 = (int)std::min<long>(P.m, (long)w * G.rl);
+        const int nlv = std::min(G.nl, P.n - j0), rlv = std::min(G.rl, P.m - i0);
+        const SplitStage T = split_stage(G, P.n, rlv, nlv, rp[i0 + rlv] - rp[i0], cp[j0 + nlv] - cp[j0]);
+        rows += T.rows;
+        cols += T.cols;
+      }
+    }
+  }
+  if (form) *form = pl->form;
+  if (support_bits) *support_bits = bits;
+  if (rows_staged) *rows_staged = rows;
+  if (columns_staged) *columns_staged = cols;
+  return XCS_OK;
+}
+
 int xcs_plan_geometry(xcs_plan *pl, int *team_size, int *block_size) {
   if (!pl || !team_size || !block_size) return set_err(XCS_EINVAL, "NULL argument");
   *team_size = pl->team;

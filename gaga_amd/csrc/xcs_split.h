@@ -81,6 +81,20 @@ __host__ __device__ inline SplitGeom split_geom(int ens, int alg, int m, int n, 
   G.filter = ens == ENS_SMV && G.lds + res_up16((size_t)n / 8 + 8) <= (size_t)SP_LDS;
   return G;
 }
+// smv with the support bits in LDS: what LDS has left takes the own rows' columns (rn
+// entries of rlv rows), then the own columns' rows and values (cn entries of nlv).
+struct SplitStage {
+  bool rows, cols;
+};
+__host__ __device__ inline SplitStage split_stage(const SplitGeom &G, int n, int rlv, int nlv, int rn, int cn) {
+  SplitStage T{false, false};
+  if (!G.filter) return T;
+  size_t left = (size_t)SP_LDS - G.lds - res_up16((size_t)n / 8 + 8);
+  T.rows = left >= res_up16(4 * ((size_t)rlv + 1 + rn + 8));
+  if (T.rows) left -= res_up16(4 * ((size_t)rlv + 1)) + res_up16(4 * (size_t)rn);
+  T.cols = left >= res_up16(4 * ((size_t)nlv + 1 + 2 * (size_t)cn + 12));
+  return T;
+}
 inline bool split_fits(int alg, int ens, int m, int n, int log2n, int num_bins, int timing,
                        int team, int block) {
   if ((alg != ALG_NIHT && alg != ALG_HTP && alg != ALG_CGIHT) || timing || team < 2 ||
@@ -1033,10 +1047,8 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
   R.rt = &rt;
   auto column = [&](int i) { return sp_column<ENS>(R, t, n, i); };
   if (ENS == ENS_SMV && G.filter) {
-    // the matrix entries do not change during a solve: what LDS has left takes the
-    // own rows' columns, then the own columns' rows and values
-    unsigned char *q = lds + G.lds + res_up16((size_t)n / 8 + 8), *end = lds + SP_LDS;
-    auto room = [&](int words) { return (size_t)(end - q) >= res_up16(4 * (size_t)words); };
+    // the matrix entries do not change during a solve
+    unsigned char *q = lds + G.lds + res_up16((size_t)n / 8 + 8);
     auto take = [&](int words) {
       unsigned char *r = q;
       q += res_up16(4 * (size_t)words);
@@ -1044,15 +1056,16 @@ __global__ void __launch_bounds__(SP_THREADS) solve_split_kernel(const XProblem 
     };
     R.rbase = P.row_ptr[R.i0];
     const int rn = P.row_ptr[R.i0 + R.rlv] - R.rbase;
-    if (room(R.rlv + 1 + rn + 8)) {
+    const int cbase = P.col_ptr[R.j0], cn = P.col_ptr[R.j0 + R.nlv] - cbase;
+    const SplitStage T = split_stage(G, n, R.rlv, R.nlv, rn, cn);
+    if (T.rows) {
       int *rp = (int *)take(R.rlv + 1), *cols = (int *)take(rn);
       for (int i = threadIdx.x; i <= R.rlv; i += nt) rp[i] = P.row_ptr[R.i0 + i] - R.rbase;
       for (int e = threadIdx.x; e < rn; e += nt) cols[e] = P.cols[R.rbase + e];
       R.lrp = rp;
       R.lcols = cols;
     }
-    const int cbase = P.col_ptr[R.j0], cn = P.col_ptr[R.j0 + R.nlv] - cbase;
-    if (room(R.nlv + 1 + 2 * cn + 12)) {
+    if (T.cols) {
       int *cp = (int *)take(R.nlv + 1), *rows = (int *)take(cn);
       float *vals = (float *)take(cn);
       for (int i = threadIdx.x; i <= R.nlv; i += nt) cp[i] = P.col_ptr[R.j0 + i] - cbase;

@@ -186,6 +186,11 @@ int xcs_plan_bytes(xcs_plan *plan, double *bytes);
 /* The team geometry the plan runs with once defaults are applied (no counterpart in the
  * reference): team_size workgroups of block_size threads per cooperative launch. */
 int xcs_plan_geometry(xcs_plan *plan, int *team_size, int *block_size);
+/* The form its solves run in: 0 the general one, 1 resident (gen: the vectors in every
+ * workgroup's LDS), 2 split (smv, dct: slices of them).  smv in the split form: whether the
+ * support bits are in LDS too, and in how many workgroups the own rows' and the own columns'
+ * matrix entries are (0 otherwise).  Any pointer may be NULL. */
+int xcs_plan_form(xcs_plan *plan, int *form, int *support_bits, int *rows_staged, int *columns_staged);
 void xcs_plan_destroy(xcs_plan *plan);
 
 /* ---- batched persistent form: many independent instances in one launch ---- */

@@ -25,6 +25,7 @@ def test_plans(lib, mode, alg, ens, k, m, n, p, extra):
     if ens == "smv":
         kw["matrixEnsemble"] = "binary"
     pl = lib.Plan(alg, ens, k, m, n, p, lib.options(barrierSpinLimit=1, **kw))
+    assert pl.form()[0] == ("general" if alg == "FIHT" else "split")
     for _ in range(2):
         with pytest.raises(lib.GagaError, match="team barrier timed out"):
             pl.solve()
