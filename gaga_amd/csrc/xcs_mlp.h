@@ -270,28 +270,27 @@ __global__ void __launch_bounds__(1024) mlp_final_kernel(const float *part, int 
 
 // FP32 tiled GEMM, C[i][j] = sum_k A(i, k) B(j, k) with strided operands,
 // 64 x 64 tile per 256-thread block, 4 x 4 per thread, K in steps of 16
-// through LDS; blockIdx.z = K split (slice z of C at z * c_split).
+// through LDS.
 __global__ void __launch_bounds__(256) f32_gemm_kernel(int M, int N, int K, const float *A,
                                                        long sai, long sak, const float *Bm,
                                                        long sbj, long sbk, float *C, long sci,
-                                                       long scj, int ksplit, long c_split) {
+                                                       long scj) {
   __shared__ float As[16][64 + 4], Bs[16][64 + 4];
   const int i0 = blockIdx.x * 64, j0 = blockIdx.y * 64;
-  const int kc = (K + ksplit - 1) / ksplit, ka = blockIdx.z * kc, kb = min(K, ka + kc);
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
   float acc[4][4] = {};
   // consecutive threads walk the operand's contiguous index (K or the row)
   const bool a_kc = sak == 1, b_kc = sbk == 1;
-  for (int k0 = ka; k0 < kb; k0 += 16) {
+  for (int k0 = 0; k0 < K; k0 += 16) {
     for (int e = threadIdx.x; e < 16 * 64; e += 256) {
       const int kk = a_kc ? (e & 15) : (e >> 6), r = a_kc ? (e >> 4) : (e & 63);
       const int k = k0 + kk, i = i0 + r;
-      As[kk][r] = (k < kb && i < M) ? A[(long)i * sai + (long)k * sak] : 0.f;
+      As[kk][r] = (k < K && i < M) ? A[(long)i * sai + (long)k * sak] : 0.f;
     }
     for (int e = threadIdx.x; e < 16 * 64; e += 256) {
       const int kk = b_kc ? (e & 15) : (e >> 6), r = b_kc ? (e >> 4) : (e & 63);
       const int k = k0 + kk, j = j0 + r;
-      Bs[kk][r] = (k < kb && j < N) ? Bm[(long)j * sbj + (long)k * sbk] : 0.f;
+      Bs[kk][r] = (k < K && j < N) ? Bm[(long)j * sbj + (long)k * sbk] : 0.f;
     }
     __syncthreads();
 #pragma unroll
@@ -309,13 +308,12 @@ __global__ void __launch_bounds__(256) f32_gemm_kernel(int M, int N, int K, cons
     }
     __syncthreads();
   }
-  float *Cz = C + (long)blockIdx.z * c_split;
 #pragma unroll
   for (int q = 0; q < 4; q++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int i = i0 + ty * 4 + q, j = j0 + tx * 4 + r;
-      if (i < M && j < N) Cz[(long)i * sci + (long)j * scj] = acc[q][r];
+      if (i < M && j < N) C[(long)i * sci + (long)j * scj] = acc[q][r];
     }
 }
 
@@ -921,7 +919,7 @@ int xcs_mrhs_samples(xcs_mrhs *h, int per, unsigned int seed, float *X_out, floa
     // G[s*n + j] = sum_i A[j*m + i] y_s[i]
     hipLaunchKernelGGL(f32_gemm_kernel, dim3((unsigned)((n + 63) / 64), (unsigned)((S + 63) / 64), 1),
                        dim3(256), 0, h->stream, (int)n, (int)S, (int)m, (const float *)h->A32, m, 1L,
-                       h->D.y, m, 1L, G, 1L, n, 1, 0L);
+                       h->D.y, m, 1L, G, 1L, n);
     hipLaunchKernelGGL(mlp_features_kernel, dim3((unsigned)S), dim3(1024), 0, h->stream, G, (int)n,
                        (int)m, h->k, Xf);
     hipLaunchKernelGGL(mlp_samples_kernel, dim3((unsigned)S), dim3(1024), 0, h->stream, G, Xf,

@@ -8,8 +8,10 @@
 //   A^T r    -> A_cm^T * R    (A column-major; K = m)
 //   A p_S    -> A_rm * P
 // Every per-signal step between two products (residual, thresholds, step
-// sizes, the k-bin support update, the stopping rules) is the single-instance
-// engine's code run by one workgroup per signal.
+// sizes, the k-bin support update, the stopping rules) is run by one workgroup per
+// signal: the single-instance engine's rules, in kernels of their own that read and
+// write each vector once (the selection's walk and the stopping rules are shared:
+// sp_walk, res_stop_update, res_continue).
 //
 // Precision: the products read A in BF16 (RNE) or OCP FP8 e4m3 with one scale
 // per column (s_j = max_i |A_ij| / 448) and the signal operand in the same
@@ -759,7 +761,7 @@ constexpr int MR_RB = 32;
 constexpr int MR_RT = 128;
 constexpr int MR_RU = 2;
 constexpr int MR_RLIST = 1024;  // support entries held in LDS at a time
-constexpr int MR_MAXM = 8192;
+constexpr int MR_MAXM = 8192;  // rows accepted (the interface's limit; the kernels have none)
 template <bool BLOCKED>
 __global__ void __launch_bounds__(MR_RT) mr_exact_resid_kernel(MrhsDesc D, double *part,
                                                                     int groups, int sel) {

@@ -17,9 +17,9 @@
 // device-scope stores and loads that go past the L2s, so it needs no fence.
 // HTP's CG steps live on the support: A^T reads the support's columns only and
 // a step takes two exchanges.
-// Measured on MI355X: CGIHT 2048 x 8192 (15 iterations) 1.70 -> 0.55 ms, 35 us an
-// iteration, of which A^T r takes about 10; NIHT 256 x 1024 0.9 -> 0.25 ms; HTP
-// 1001 x 5003 1.65 -> 0.34 ms (plan_resident has the team sizes).
+// Measured on MI355X: CGIHT 2048 x 8192 (15 iterations) 1.70 -> 0.55 ms, 37 us an
+// iteration, of which A^T r takes 7.4 and the exchanges 12; NIHT 256 x 1024 0.9 -> 0.25
+// ms; HTP 1001 x 5003 1.65 -> 0.34 ms (plan_resident has the team sizes).
 //
 // The arithmetic is that of the general solver except for the order of sums.
 #pragma once

@@ -64,10 +64,10 @@ typedef struct xcs_options {
                                 dynamic detection, 3 a sort at every step (gaga_gen.cu:168) */
   float alpha;               /* 'alpha' (alpha_start) of the timing variants, in [0, 1);
                                 xcs_options_default sets 0.25 */
-  long barrier_spin_limit;   /* bound of every multi-workgroup team-barrier wait, in sleeps
-                                (0: the default, 2^26); a wait that exceeds it abandons the
-                                solve with XCS_EHIP ("team barrier timed out") instead of
-                                hanging */
+  long barrier_spin_limit;   /* bound of every wait of a multi-workgroup team, in polls of
+                                about a microsecond (0: the default, 2^26); a wait that
+                                exceeds it abandons the solve with XCS_EHIP ("team barrier
+                                timed out") instead of hanging */
 } xcs_options;
 
 /* Fill *opts with the reference defaults for (alg, ens, n). */
@@ -181,7 +181,8 @@ int xcs_plan_trace(xcs_plan *plan, int *k_bin, float *resid_norm, int len);
  * *ms_per = device ms per application, *bytes = its algorithmic bytes. */
 int xcs_plan_apply_timed(xcs_plan *plan, int transpose, int reps, float *ms_per, double *bytes);
 /* Algorithmic bytes moved by the operator applications of the last solve
- * (gen A_S x_S: 4m|S|+8|S|+4m; gen A^T r: 4mn+4m+4n; smv: 8nz+4m+4n; dct: 4n+8m). */
+ * (gen A_S x_S: 4m|S|+8|S|+4m; gen A^T r: 4mn+4m+4n, or 4m|S|+4m+4|S| where a CG step forms it
+ * on the support only; smv: 8nz+4m+4n; dct: 4n+8m). */
 int xcs_plan_bytes(xcs_plan *plan, double *bytes);
 /* The team geometry the plan runs with once defaults are applied (no counterpart in the
  * reference): team_size workgroups of block_size threads per cooperative launch. */
