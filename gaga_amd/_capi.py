@@ -25,6 +25,7 @@ EXPORTS = (
     "xcs_last_error", "xcs_version", "xcs_results_line", "xcs_results_append",
     "xcs_cs_gen_noalloc", "xcs_batch_schedule", "xcs_batch_phase_counts", "xcs_stream_read",
     "xcs_batch_schedule_mode", "xcs_batch_exact", "xcs_batch_ran", "xcs_plan_form",
+    "xcs_mrhs_row_blocks",
 )
 
 
@@ -105,6 +106,7 @@ def load():
         L.xcs_mrhs_gemm_timed.argtypes = [_P, _I, _C, _I, _P, _P]
         L.xcs_mrhs_phase_ms.argtypes = [_P, _P]
         L.xcs_mrhs_samples.argtypes = [_P, _I, ctypes.c_uint, _P, _P]
+        L.xcs_mrhs_row_blocks.argtypes = [_P, _I]
         L.xcs_mrhs_gemm_tile.argtypes = [_P, _I]
         L.xcs_mlp_create.argtypes = [ctypes.c_uint, _P]
         L.xcs_mlp_destroy.argtypes = [_P]
@@ -611,6 +613,11 @@ class ManyRHS:
         """GEMM block tile: 0 128 x 128, 1 256 x 128, 2 256 x 256 (True means 1), -1 (the
         default) each product's by its sizes."""
         _ck(load().xcs_mrhs_gemm_tile(self._h, int(tile)))
+
+    def row_blocks(self, keep):
+        """keep=False gives back the row-blocked copy of A (4 m n bytes), True makes it
+        again; results do not depend on it."""
+        _ck(load().xcs_mrhs_row_blocks(self._h, 1 if keep else 0))
 
     def samples(self, per, seed=1):
         """Training samples of every signal: (X (count*per x 8), labels)."""

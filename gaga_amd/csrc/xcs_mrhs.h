@@ -1231,6 +1231,19 @@ static size_t mr_product_floats(int M, int cols, int K) {
   return most;
 }
 
+// The row-blocked copy of A, made if it is not there.
+static int mr_row_blocks(xcs_mrhs *h) {
+  if (h->A32b) return XCS_OK;
+  const size_t mn = (size_t)h->m * h->n;
+  float *blocks;
+  XCS_TRY(h->alloc(&blocks, mn, false));
+  hipLaunchKernelGGL(mr_blocks_kernel, dim3((int)std::min<size_t>(65536, (mn / 4 + MR_THREADS - 1) / MR_THREADS)),
+                     dim3(MR_THREADS), 0, h->stream, (const float4 *)h->A32, h->m, h->n, (float4 *)blocks);
+  HIP_TRY(hipGetLastError());
+  h->D.A32b = h->A32b = blocks;
+  return XCS_OK;
+}
+
 static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *precision,
                      const xcs_options *o) {
   if (!precision || (strcmp(precision, "bf16") && strcmp(precision, "fp8")))
@@ -1352,15 +1365,7 @@ static int mr_create(xcs_mrhs *h, int m, int n, int k, int count, const char *pr
     HIP_TRY(d2h(h->sup_true.data(), d_sup, 4 * S * k, nullptr));
   }
   // the row-blocked copy for the exact residual, where there is memory left for it
-  if (h->alloc(&h->A32b, mn, false) == XCS_OK) {
-    hipLaunchKernelGGL(mr_blocks_kernel, dim3((int)std::min<size_t>(65536, (mn / 4 + MR_THREADS - 1) / MR_THREADS)),
-                       dim3(MR_THREADS), 0, h->stream, (const float4 *)h->A32, m, n, (float4 *)h->A32b);
-    HIP_TRY(hipGetLastError());
-    D.A32b = h->A32b;
-  } else {
-    (void)hipGetLastError();
-    h->A32b = nullptr;
-  }
+  if (mr_row_blocks(h) != XCS_OK) (void)hipGetLastError();
   hipLaunchKernelGGL(mr_make_y_kernel, dim3(count), dim3(MR_THREADS), 0, h->stream, h->A32, m,
                      d_vals, d_sup, k, y);
   HIP_TRY(hipGetLastError());
@@ -1683,6 +1688,19 @@ int xcs_mrhs_gemm_tile(xcs_mrhs *h, int tile) {
   if (!h) return set_err(XCS_EINVAL, "NULL handle");
   if (tile < -1 || tile > 2) return set_err(XCS_EINVAL, "tile must be -1 (by sizes), 0, 1 or 2");
   h->gemm_big = tile;
+  return XCS_OK;
+}
+
+int xcs_mrhs_row_blocks(xcs_mrhs *h, int keep) {
+  if (!h) return set_err(XCS_EINVAL, "NULL handle");
+  HIP_TRY(hipSetDevice(h->dev));
+  if (keep) return mr_row_blocks(h);
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  if (h->A32b) {
+    h->allocs.erase(std::find(h->allocs.begin(), h->allocs.end(), (void *)h->A32b));
+    (void)hipFree(h->A32b);
+  }
+  h->D.A32b = h->A32b = nullptr;
   return XCS_OK;
 }
 

@@ -313,6 +313,11 @@ int xcs_mrhs_configure(xcs_mrhs *handle, float c_bf16, float c_fp8, int correcti
  * the rounding of the products only, on the number of signals that are still active: it decides
  * in how many slices a product sums. */
 int xcs_mrhs_gemm_tile(xcs_mrhs *handle, int tile);
+/* keep = 0 gives back the copy of A that the exact residual reads by blocks of rows (4 m n
+ * bytes; it then reads A as it is, for the same bits in about twice the time); otherwise the copy
+ * is made if it is not there (XCS_ENOMEM where it does not fit).  A handle is created with it
+ * where there is memory left. */
+int xcs_mrhs_row_blocks(xcs_mrhs *handle, int keep);
 /* Device ms of the last solve's phases: start, low-precision phase, BF16 continuation,
  * refinement, support corrections (with their refinements), 0. */
 int xcs_mrhs_phase_ms(xcs_mrhs *handle, float *ms6);
