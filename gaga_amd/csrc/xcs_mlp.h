@@ -639,7 +639,7 @@ static float *mlp_pin(xcs_mlp *net, long B) {
 
 // Forward over B coordinates in net->X; logits in net->logit.  With labels
 // in net->lab: backward into net->g (and per-coordinate losses).  Eight launches
-// for a training pass (nineteen before); measured on MI355X at B = 8192: l1 8.5,
+// for a training pass (nineteen before); measured on MI355X at B = 8192: l1 5.6,
 // the GEMMs 14 each, out 22, dW2 50 (its FP32 matrix-rate floor is 27), in 10, the
 // sums 9 us; an Adam step of 8192 504 -> 126 us, of 100 171 -> 77 us.
 static int mlp_pass(xcs_mlp *net, int B, bool train, float pos_w) {
